@@ -229,6 +229,25 @@ int rp_gs_pass_fused(int prec, const void *const *V, int k, void *w, uint64_t n,
  * overlap on one GPU (from several host threads or streams) race. */
 int rp_gs_pass_fused_noalloc(int prec, const void *const *V, int k, void *w, uint64_t n,
                              double *h, double *norm, double fuse_min, int *normalized);
+/* Arnoldi steps j0 .. m-1 (m <= 64) with one wait for all of them (no
+ * counterpart in the reference, which waits for every dot product,
+ * inc/algo.h:144-173): for each j, V[j+1] = H V[j], one Gram-Schmidt pass of
+ * it against V[0..j] as rp_gs_pass_fused with fuse_min = min_norm, and
+ * V[j+1] divided by its norm.  V holds m + 1 device pointers, all different,
+ * V[0..j0] orthonormal on entry.  A step whose norm is below min_norm (> 0)
+ * is the last: its V[j+1] is left as the pass made it, and nothing of the
+ * steps behind it runs.  *done = steps made; out receives RP_STEP_DOUBLES
+ * doubles per step: h (2 (j+1) of them), at 2 RP_MAX_SWEEP_VECS the norm, and
+ * after it 1 when the pass itself normalized (*normalized of
+ * rp_gs_pass_fused). */
+#define RP_STEP_DOUBLES (2 * RP_MAX_SWEEP_VECS + 2)
+int rp_arnoldi_steps(rp_terms_t h, void *const *V, int j0, int m, double min_norm, double *out,
+                     int *done);
+/* The m Lanczos steps (m <= 64) of Krylov::ground_state (inc/algo.h:180-257)
+ * with one wait: for j = 0 .. m-1, V[j+1] = H V[j], alpha[j] = Re <V[j]|V[j+1]>
+ * and, but for the last, V[j+1] -= alpha[j] V[j] + beta[j-1] V[j-1], beta[j] =
+ * ||V[j+1]||, V[j+1] /= beta[j].  V[0] is normalized; beta holds m - 1. */
+int rp_lanczos_steps(rp_terms_t h, void *const *V, int m, double *alpha, double *beta);
 /* y += sum_i c[i] V[i] for k vectors (any k; one sweep per 16 of them), c
    given as 2k doubles (re, im) */
 int rp_lincomb(int prec, void *y, const void *const *V, int k, const double *c, uint64_t n);

@@ -102,6 +102,8 @@ def hip():
                                  _c.POINTER(_c.c_int)],
             "rp_gs_pass_fused_noalloc": [_c.c_int, _vp, _c.c_int, _vp, _u64, _vp,
                                          _c.POINTER(_dbl), _dbl, _c.POINTER(_c.c_int)],
+            "rp_arnoldi_steps": [_vp, _vp, _c.c_int, _c.c_int, _dbl, _vp, _c.POINTER(_c.c_int)],
+            "rp_lanczos_steps": [_vp, _vp, _c.c_int, _vp, _vp],
             "rp_lincomb": [_c.c_int, _vp, _vp, _c.c_int, _vp, _u64],
             "rp_prof_enable": [_c.c_int], "rp_prof_reset": [],
             "rp_prof_query": [_c.c_int, _c.POINTER(_u64), _c.POINTER(_dbl)],

@@ -72,8 +72,10 @@ namespace rp {
 template <typename R, typename A>
 __global__ void __launch_bounds__(kSmallThreads)
 k_apply_small(const typename CxA<R>::T *__restrict__ in, typename CxA<R>::T *__restrict__ out,
-              uint32_t dim, const FlatTerm<A> *__restrict__ terms, int nterms, int accumulate)
+              uint32_t dim, const FlatTerm<A> *__restrict__ terms, int nterms, int accumulate,
+              const int *__restrict__ stop)
 {
+    if (stop && *stop) return;
     uint32_t m = blockIdx.x * kSmallThreads + threadIdx.x;
     if (m >= dim) return;
     A ar = 0, ai = 0;
@@ -106,8 +108,10 @@ k_apply_small(const typename CxA<R>::T *__restrict__ in, typename CxA<R>::T *__r
 template <typename R, typename A>
 __global__ void __launch_bounds__(kSmallThreads)
 k_apply_split(const typename CxA<R>::T *__restrict__ in, typename CxA<A>::T *__restrict__ part,
-              uint32_t dim, const FlatTerm<A> *__restrict__ terms, int nterms, int per)
+              uint32_t dim, const FlatTerm<A> *__restrict__ terms, int nterms, int per,
+              const int *__restrict__ stop)
 {
+    if (stop && *stop) return;
     uint32_t m = blockIdx.x * kSmallThreads + threadIdx.x;
     if (m >= dim) return;
     const int t0 = blockIdx.y * per;
@@ -132,8 +136,9 @@ k_apply_split(const typename CxA<R>::T *__restrict__ in, typename CxA<A>::T *__r
 template <typename R, typename A>
 __global__ void __launch_bounds__(kSmallThreads)
 k_split_reduce(const typename CxA<A>::T *__restrict__ part, typename CxA<R>::T *__restrict__ out,
-               uint32_t dim, int slices, int accumulate)
+               uint32_t dim, int slices, int accumulate, const int *__restrict__ stop)
 {
+    if (stop && *stop) return;
     for (uint32_t m = blockIdx.x * kSmallThreads + threadIdx.x; m < dim;
          m += gridDim.x * kSmallThreads) {
         A ar = 0, ai = 0;
@@ -541,8 +546,10 @@ template <typename R, typename A, int TB, int NT, int D, bool GA>
 __global__ void __launch_bounds__(NT, (apply_waves_per_eu<R, TB, NT, D>()))
 k_apply_tiled(const typename CxA<R>::T *__restrict__ in, typename CxA<R>::T *__restrict__ out,
               const GroupRuns *__restrict__ groups, int ngroups, const SubRec<A> *__restrict__ subs,
-              const TermRec<A> *__restrict__ terms, int accumulate, TileMap tm)
+              const TermRec<A> *__restrict__ terms, int accumulate, TileMap tm,
+              const int *__restrict__ stop)
 {
+    if (stop && *stop) return;
     using T = typename CxA<R>::T;
     constexpr int TILE = 1 << TB;
     static_assert(NT == 1024 || NT == 512 || NT == 256 || NT == 128,
@@ -822,8 +829,10 @@ template <int TB, int NT>
 __global__ void __launch_bounds__(NT, (apply_waves_per_eu<float, TB, NT, 2>()))
 k_apply_stream(const float2 *__restrict__ in, float2 *__restrict__ out,
                const GroupC *__restrict__ groups, int ngroups, const SubC *__restrict__ subs,
-               const TermC *__restrict__ terms, int accumulate, TileMap tm)
+               const TermC *__restrict__ terms, int accumulate, TileMap tm,
+               const int *__restrict__ stop)
 {
+    if (stop && *stop) return;
     __shared__ float2 tile0[1 << TB];
     __shared__ float2 tile1[1 << TB];
     stream_tile<TB, NT>(in, out, groups, ngroups, subs, terms, accumulate, tile_index(tm) << TB,
@@ -1111,7 +1120,7 @@ static void free_handle(rp_terms *h)
 }
 
 template <typename R, typename A, int TB, int NT, int D = 2>
-static int launch_tiled(rp_terms *h, void *res, const void *vec, int accumulate)
+static int launch_tiled(rp_terms *h, void *res, const void *vec, int accumulate, const int *stop)
 {
     using T = typename CxA<R>::T;
     const uint64_t grid = (1ull << h->len) >> TB;
@@ -1119,26 +1128,27 @@ static int launch_tiled(rp_terms *h, void *res, const void *vec, int accumulate)
         if (h->group_acc && h->d_csubs) {
             RP_LAUNCH(RP_KERNEL_APPLY, (k_apply_stream<TB, NT>), dim3((unsigned)grid), dim3(NT), 0,
                       (const T *)vec, (T *)res, (const GroupC *)h->d_cgroups, (int)h->ngroups,
-                      (const SubC *)h->d_csubs, (const TermC *)h->d_cterms, accumulate, h->tmap);
+                      (const SubC *)h->d_csubs, (const TermC *)h->d_cterms, accumulate, h->tmap,
+                      stop);
             return RP_OK;
         }
         if (h->group_acc) {
             RP_LAUNCH(RP_KERNEL_APPLY, (k_apply_tiled<R, A, TB, NT, D, true>), dim3((unsigned)grid),
                       dim3(NT), 0, (const T *)vec, (T *)res, (const GroupRuns *)h->d_groups,
                       (int)h->ngroups, (const SubRec<A> *)h->d_subs,
-                      (const TermRec<A> *)h->d_terms, accumulate, h->tmap);
+                      (const TermRec<A> *)h->d_terms, accumulate, h->tmap, stop);
             return RP_OK;
         }
     }
     RP_LAUNCH(RP_KERNEL_APPLY, (k_apply_tiled<R, A, TB, NT, D, false>), dim3((unsigned)grid),
               dim3(NT), 0, (const T *)vec, (T *)res, (const GroupRuns *)h->d_groups,
               (int)h->ngroups, (const SubRec<A> *)h->d_subs, (const TermRec<A> *)h->d_terms,
-              accumulate, h->tmap);
+              accumulate, h->tmap, stop);
     return RP_OK;
 }
 
 template <typename R, typename A>
-static int apply_impl(rp_terms *h, void *res, const void *vec, int accumulate)
+static int apply_impl(rp_terms *h, void *res, const void *vec, int accumulate, const int *stop)
 {
     using T = typename CxA<R>::T;
     const uint64_t dim = 1ull << h->len;
@@ -1154,34 +1164,35 @@ static int apply_impl(rp_terms *h, void *res, const void *vec, int accumulate)
             const int per = (int)((h->nterms + slices - 1) / slices);
             RP_LAUNCH(RP_KERNEL_APPLY, (k_apply_split<R, A>), dim3(grid, slices),
                       dim3(kSmallThreads), 0, (const T *)vec, (P *)h->d_split, (uint32_t)dim,
-                      (const FlatTerm<A> *)h->d_flat, (int)h->nterms, per);
+                      (const FlatTerm<A> *)h->d_flat, (int)h->nterms, per, stop);
             RP_LAUNCH(RP_KERNEL_APPLY, (k_split_reduce<R, A>), dim3(grid), dim3(kSmallThreads), 0,
-                      (const P *)h->d_split, (T *)res, (uint32_t)dim, slices, accumulate);
+                      (const P *)h->d_split, (T *)res, (uint32_t)dim, slices, accumulate,
+                      stop);
             return RP_OK;
         }
         RP_LAUNCH(RP_KERNEL_APPLY, (k_apply_small<R, A>), dim3(grid), dim3(kSmallThreads), 0,
                   (const T *)vec, (T *)res, (uint32_t)dim, (const FlatTerm<A> *)h->d_flat,
-                  (int)h->nterms, accumulate);
+                  (int)h->nterms, accumulate, stop);
         return RP_OK;
     }
     switch (tiling_key(h->tile_bits, h->threads, h->depth)) {
-    case tiling_key(8, 128, 2): return launch_tiled<R, A, 8, 128>(h, res, vec, accumulate);
-    case tiling_key(10, 128, 2): return launch_tiled<R, A, 10, 128>(h, res, vec, accumulate);
-    case tiling_key(12, 512, 2): return launch_tiled<R, A, 12, 512>(h, res, vec, accumulate);
+    case tiling_key(8, 128, 2): return launch_tiled<R, A, 8, 128>(h, res, vec, accumulate, stop);
+    case tiling_key(10, 128, 2): return launch_tiled<R, A, 10, 128>(h, res, vec, accumulate, stop);
+    case tiling_key(12, 512, 2): return launch_tiled<R, A, 12, 512>(h, res, vec, accumulate, stop);
     case tiling_key(11, 256, 4):
-        if constexpr (sizeof(R) == 8) return launch_tiled<R, A, 11, 256, 4>(h, res, vec, accumulate);
+        if constexpr (sizeof(R) == 8) return launch_tiled<R, A, 11, 256, 4>(h, res, vec, accumulate, stop);
         break;
     case tiling_key(12, 512, 3):
-        if constexpr (sizeof(R) == 4) return launch_tiled<R, A, 12, 512, 3>(h, res, vec, accumulate);
+        if constexpr (sizeof(R) == 4) return launch_tiled<R, A, 12, 512, 3>(h, res, vec, accumulate, stop);
         break;
     case tiling_key(12, 512, 4):
-        if constexpr (sizeof(R) == 4) return launch_tiled<R, A, 12, 512, 4>(h, res, vec, accumulate);
+        if constexpr (sizeof(R) == 4) return launch_tiled<R, A, 12, 512, 4>(h, res, vec, accumulate, stop);
         break;
     case tiling_key(12, 1024, 2):
-        if constexpr (sizeof(R) == 4) return launch_tiled<R, A, 12, 1024>(h, res, vec, accumulate);
+        if constexpr (sizeof(R) == 4) return launch_tiled<R, A, 12, 1024>(h, res, vec, accumulate, stop);
         break;
     case tiling_key(13, 1024, 2):
-        if constexpr (sizeof(R) == 4) return launch_tiled<R, A, 13, 1024>(h, res, vec, accumulate);
+        if constexpr (sizeof(R) == 4) return launch_tiled<R, A, 13, 1024>(h, res, vec, accumulate, stop);
         break;
     default: break;
     }
@@ -1239,12 +1250,20 @@ static void free_tables(rp_terms *h)
         if (*p) { (void)hipFree(*p); *p = nullptr; }
 }
 
-static int apply_dispatch(rp_terms *h, void *res, const void *vec, int accumulate)
+static int apply_dispatch(rp_terms *h, void *res, const void *vec, int accumulate,
+                          const int *stop = nullptr)
 {
-    if (h->prec == RP_C128) return apply_impl<double, double>(h, res, vec, accumulate);
-    if (h->acc64) return apply_impl<float, double>(h, res, vec, accumulate);
-    return apply_impl<float, float>(h, res, vec, accumulate);
+    if (h->prec == RP_C128) return apply_impl<double, double>(h, res, vec, accumulate, stop);
+    if (h->acc64) return apply_impl<float, double>(h, res, vec, accumulate, stop);
+    return apply_impl<float, float>(h, res, vec, accumulate, stop);
 }
+
+namespace rp {
+int apply_queued(rp_terms_t h, void *res, const void *vec, const int *stop)
+{
+    return apply_dispatch(h, res, vec, 0, stop);
+}
+}  // namespace rp
 
 // rebuild the device tables for another tiling (from the stored term list)
 static int retile(rp_terms *h, int tb, int nt, int d)

@@ -74,6 +74,10 @@ int vec_scratch_setup(int device);
 int apply_dots_launch(rp_terms_t h, void *res, const void *vec, const void *const *V, int k,
                       double *part, int width, uint64_t max_rows, uint64_t *rows);
 
+// res = H vec queued on the library stream (rp_apply.hip); every kernel of it
+// returns at once when *stop (device memory, may be null) is set
+int apply_queued(rp_terms_t h, void *res, const void *vec, const int *stop);
+
 // launch bracketing for the optional per-class timing
 void prof_begin(int cls, hipEvent_t *start, hipEvent_t *stop);
 void prof_end(int cls, hipEvent_t start, hipEvent_t stop);
@@ -82,6 +86,10 @@ int prof_collect();   // must be called after a stream synchronization
 // blocks of the persistent-style reduction kernels
 constexpr int kRedBlocks = 1024;
 constexpr int kRedThreads = 256;
+// the pinned host buffer: scalars of one call in [0, kHostSteps), then a slot
+// of results for each of the up to 64 queued steps of a Krylov recurrence
+constexpr int kHostSteps = 4096;
+constexpr int kHostSlot = 136;
 
 inline size_t elem_bytes(int prec) { return prec == RP_C64 ? 8 : 16; }
 inline bool valid_prec(int prec) { return prec == RP_C64 || prec == RP_C128; }

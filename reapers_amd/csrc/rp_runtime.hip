@@ -113,7 +113,7 @@ int rp_init(int device)
     // block, plus room for the reduced results
     c.work_bytes = (size_t)kRedBlocks * (2 * 64 + 1) * sizeof(double) + 64 * 1024;
     RP_CHECK_HIP(dev_malloc(&c.work, c.work_bytes));
-    c.pinned_doubles = 4096;
+    c.pinned_doubles = kHostSteps + RP_MAX_SWEEP_VECS * kHostSlot;
     RP_CHECK_HIP(hipHostMalloc((void **)&c.pinned, c.pinned_doubles * sizeof(double),
                                hipHostMallocDefault));
     int st = vec_scratch_setup(device);

@@ -10,6 +10,7 @@
 // a second small kernel, so every reduction is deterministic for a given n.
 #include "rp_internal.h"
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <vector>
@@ -31,12 +32,26 @@ static inline int grid_for(uint64_t units, int threads, int cap)
 constexpr int kEwThreads = 256;
 constexpr int kEwMaxBlocks = 65536;
 constexpr int kMaxVecs = RP_MAX_SWEEP_VECS;   // vectors per fused sweep (API limit)
-constexpr int kDotChunk = 8;      // vectors whose dots one launch accumulates
-constexpr int kUpdChunk = 16;     // vectors one update / lincomb launch reads
+constexpr int kDotChunk = 8;      // most vectors whose dots one workgroup accumulates
+constexpr int kUpdChunk = 16;     // vectors an update / lincomb thread loads at once
 constexpr int kWaves = kRedThreads / 64;
 
-struct VecPtrs16 { const void *p[kUpdChunk]; };
-struct Coefs16 { double c[2 * kUpdChunk]; };
+// basis pointers and coefficients as kernel arguments (read by scalar loads)
+struct VecPtrs { const void *p[kMaxVecs]; };
+struct Coefs { double c[2 * kMaxVecs]; };
+
+// Workspace of the reductions (doubles): the partials, up to kDotBlocks for
+// each of 2 kMaxVecs + 1 columns (kRedBlocks are reserved), then the results of the pass in flight:
+//   [0, 2k) coefficients h; kResNorm (host only) the norm after the pass when
+//   it was not fused; kResIn ||w||^2 before it; kResBeta the fused norm (0: not
+//   fused); kResStop (an int) set by an Arnoldi step that needs the host;
+//   kResCount arrival counters of the dot workgroups, zero between launches.
+// The pinned host copy that the kernels write has the layout up to kResStop.
+constexpr int kResNorm = 2 * kMaxVecs, kResIn = kResNorm + 1, kResBeta = kResNorm + 2,
+              kResStop = kResNorm + 4, kResCount = kResNorm + 8;
+constexpr int kResDoubles = kResCount + kMaxVecs / 2;
+static_assert(kResBeta < kHostSlot && (size_t)kResDoubles * sizeof(double) < 32 * 1024,
+              "result slots");
 
 // ---------------------------------------------------------------------------
 // elementwise kernels
@@ -193,90 +208,235 @@ k_reduce_cols(const double *__restrict__ partial, int nparts, int width, double 
     if (threadIdx.x == 0) out[j] = sh[kWaves];
 }
 
-// <V[q]|w> for the KC vectors of one chunk, FP64 partials per block written
-// to partial[block*width + 2*(q0+q) + {0,1}]; with wnorm, also ||w||^2 to
-// partial[block*width + 2*kMaxVecs].  All KC loads of an element are issued
-// before any use.
-template <typename R, int KC>
-__global__ void __launch_bounds__(kRedThreads)
-k_dots(VecPtrs16 V, const typename Cx<R>::T *__restrict__ w, uint64_t n,
-       double *__restrict__ partial, int width, int q0, int wnorm)
+// Sums of NV (a power of two up to 64) per-lane values over the wavefront by
+// recursive halving: each exchange halves the values a lane carries, so NV
+// sums take about 2 NV + 6 - 2 log2 NV shuffles instead of 6 NV.  On return
+// v[0] of every lane l holds the sum of value l >> (6 - log2 NV).
+template <int NV>
+__device__ __forceinline__ void wave_multi_sum(double (&v)[NV])
+{
+    int off = 32;
+#pragma unroll
+    for (int h = NV / 2; h > 0; h >>= 1, off >>= 1) {
+        const bool hi = (threadIdx.x & off) != 0;
+#pragma unroll
+        for (int i = 0; i < h; i++) {
+            const double keep = hi ? v[i + h] : v[i], send = hi ? v[i] : v[i + h];
+            v[i] = keep + __shfl_xor(send, off, 64);
+        }
+    }
+    for (; off > 0; off >>= 1) v[0] += __shfl_xor(v[0], off, 64);
+}
+
+// Partials that another workgroup of the same launch reads: written through
+// to memory and read past the caches (device-scope accesses), with a wait
+// for the writes before the arrival is counted.  A device-scope fence would
+// order them too, but it writes the whole L2 back: with one in each of 2048
+// workgroups a dot sweep over 12 vectors of 2^23 complex<float> took 267 us
+// instead of 172.
+__device__ __forceinline__ void put_shared(double *p, double v)
+{
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ double get_shared(const double *p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// count this workgroup's arrival, its writes by put_shared complete (called
+// by the wavefront that made them); true in the last of n workgroups
+__device__ __forceinline__ bool arrive_last(unsigned *count, unsigned n)
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_s_waitcnt(0);
+    unsigned before = 0;
+    if ((threadIdx.x & 63) == 0)
+        before = __hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return __builtin_amdgcn_readfirstlane(before) == n - 1;
+}
+
+constexpr int pow2_at_least(int v) { return v <= 1 ? 1 : 2 * pow2_at_least((v + 1) / 2); }
+
+// Dots of one Gram-Schmidt pass: workgroup (x, y) forms the FP64 partials of
+// <V[q]|w> over its share of the elements for the KC vectors q0 = y KC ..
+// (the last row of workgroups repeats the last vector past k), and row y = 0
+// also ||w||^2.  The last workgroup of a row y to arrive adds the row's
+// partials in an order of their own, so the result does not depend on which
+// one that was, and writes res (and host, pinned memory, when given).  real:
+// the imaginary parts are written as zero (Lanczos).
+//
+// HBM bound for vectors beyond the caches; for the short vectors of small
+// chains bound by latency: the reduction by the last workgroup saves the
+// separate reduction launches (4.5 us each with their gap, two to three a
+// pass), the recursive halving the shuffles of the workgroup's reduction.
+// At most kDotBlocks workgroups a row, so that every thread of the last one
+// has all its partials in flight at once (past the caches each read takes
+// about 1 us); from 2^16 elements they have 1024 threads.
+constexpr int kDotBlocks = 256;
+template <typename R, int KC, int NT>
+__global__ void __launch_bounds__(NT)
+k_gs_dots(VecPtrs V, int k, const typename Cx<R>::T *__restrict__ w, uint64_t n,
+          double *__restrict__ part, double *__restrict__ res, int real,
+          double *__restrict__ host, const int *__restrict__ stop)
 {
     using T = typename Cx<R>::T;
-    __shared__ double sh[(kWaves + 1) * (2 * KC + 1)];
-    double acc[2 * KC + 1];
+    constexpr int NV = pow2_at_least(KC ? 2 * KC : 1), W = NT / 64;
+    constexpr int SH = 6 - (NV == 1 ? 0 : NV == 2 ? 1 : NV == 4 ? 2 : NV == 8 ? 3 : 4);
+    __shared__ double sh[W][NV + 1];
+    __shared__ int last;
+    if (stop && *stop) return;
+    const int y = blockIdx.y, q0 = y * KC, nb = gridDim.x;
+    double acc[NV], wn = 0.0;
 #pragma unroll
-    for (int q = 0; q < 2 * KC + 1; q++) acc[q] = 0.0;
+    for (int q = 0; q < NV; q++) acc[q] = 0.0;
+    const T *vp[KC ? KC : 1];
+#pragma unroll
+    for (int q = 0; q < KC; q++) vp[q] = (const T *)V.p[min(q0 + q, k - 1)];
     GRID_STRIDE(i, n) {
-        const T y = w[i];
-        T x[KC];
+        const T e = w[i];
+        T x[KC ? KC : 1];
 #pragma unroll
-        for (int q = 0; q < KC; q++) x[q] = ((const T *)V.p[q])[i];
-        const double yr = y.x, yi = y.y;
+        for (int q = 0; q < KC; q++) x[q] = vp[q][i];
+        const double yr = e.x, yi = e.y;
 #pragma unroll
         for (int q = 0; q < KC; q++) {
             const double xr = x[q].x, xi = x[q].y;
             acc[2 * q] += xr * yr + xi * yi;
             acc[2 * q + 1] += xr * yi - xi * yr;
         }
-        acc[2 * KC] += yr * yr + yi * yi;
+        wn += yr * yr + yi * yi;
     }
-    block_reduce<2 * KC + 1>(acc, sh);
-    if (threadIdx.x < 2 * KC)
-        partial[(size_t)blockIdx.x * width + 2 * q0 + threadIdx.x] =
-            sh[kWaves * (2 * KC + 1) + threadIdx.x];
-    if (wnorm && threadIdx.x == 2 * KC)
-        partial[(size_t)blockIdx.x * width + 2 * kMaxVecs] = sh[kWaves * (2 * KC + 1) + 2 * KC];
-}
-
-// w -= sum_q h[q0+q] V[q] for the KC vectors of one chunk (FP64 arithmetic,
-// one rounding); the last chunk also writes ||w||^2 partials.
-// Fused normalization (last chunk, fuse_min > 0): with all k coefficients h
-// and ||w||^2 before the pass in res, beta^2 = ||w||^2 - sum |h_q|^2 is the
-// norm of the result when the basis is orthonormal; if beta^2 >= ||w||^2 / 2
-// (no cancellation to speak of) and beta >= fuse_min, the result is written
-// scaled by 1/beta and beta is stored to res[2 kMaxVecs + 2] (else 0).
-template <typename R, int KC>
-__global__ void __launch_bounds__(kRedThreads)
-k_gs_update(VecPtrs16 V, const double *__restrict__ h, typename Cx<R>::T *__restrict__ w,
-            uint64_t n, double *__restrict__ partial, const double *__restrict__ res, int k,
-            double fuse_min)
-{
-    using T = typename Cx<R>::T;
-    __shared__ double hs[2 * KC];
-    __shared__ double sh[(kWaves + 1) * 1];
-    __shared__ double fscale;
-    if (threadIdx.x < 2 * KC) hs[threadIdx.x] = h[threadIdx.x];
-    if (threadIdx.x == 0) {
-        double scale = 1.0, beta = 0.0;
-        if (fuse_min > 0) {
-            double s2 = 0;
-            for (int q = 0; q < k; q++) s2 += res[2 * q] * res[2 * q] + res[2 * q + 1] * res[2 * q + 1];
-            const double wn2 = res[2 * kMaxVecs + 1];
-            const double b2 = wn2 - s2;
-            if (b2 > 0 && b2 >= 0.5 * wn2 && sqrt(b2) >= fuse_min) {
-                beta = sqrt(b2);
-                scale = 1.0 / beta;
-            }
-            if (blockIdx.x == 0) ((double *)res)[2 * kMaxVecs + 2] = beta;
-        }
-        fscale = scale;
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    if constexpr (KC > 0) {
+        wave_multi_sum<NV>(acc);
+        if ((lane & ((1 << SH) - 1)) == 0) sh[wid][lane >> SH] = acc[0];
+    }
+    if (y == 0) {
+        wn = wave_sum(wn);
+        if (lane == 0) sh[wid][NV] = wn;
     }
     __syncthreads();
-    const double f = fscale;
-    double nacc[1] = {0.0};
-    GRID_STRIDE(i, n) {
-        const T y = w[i];
-        T x[KC];
+    // columns of this row: 2 per vector, and ||w||^2 (column kResNorm)
+    const int nv = KC ? 2 * min(KC, k - q0) : 0, ncol = nv + (y == 0 ? 1 : 0);
+    auto column = [&](int c) { return part + (size_t)(c < nv ? 2 * q0 + c : kResNorm) * kDotBlocks; };
+    auto store = [&](int c, double v) {
+        const int at = c < nv ? 2 * q0 + c : kResIn;
+        if (real && c < nv && (c & 1)) v = 0.0;
+        res[at] = v;
+        if (host) host[at] = v;
+    };
+    if (threadIdx.x < 64) {
+        if (lane < ncol) {
+            const int c = lane < nv ? lane : NV;
+            double v = 0;
 #pragma unroll
-        for (int q = 0; q < KC; q++) x[q] = ((const T *)V.p[q])[i];
-        double yr = y.x, yi = y.y;
+            for (int q = 0; q < W; q++) v += sh[q][c];
+            if (nb == 1) store(lane, v);
+            else put_shared(column(lane) + blockIdx.x, v);
+        }
+        if (nb > 1) {
+            const bool l = arrive_last((unsigned *)(res + kResCount) + y, (unsigned)nb);
+            if (lane == 0) last = l;
+        }
+    }
+    if (nb == 1) return;
+    __syncthreads();
+    if (!last) return;
+    // G threads per column (32 column slots for at most 17 columns)
+    constexpr int G = NT / 32, PER = kDotBlocks / G;
+    const int c = threadIdx.x / G, g = threadIdx.x % G;
+    if (c < ncol) {
+        const double *col = column(c);
+        double p[PER], v = 0;
 #pragma unroll
-        for (int q = 0; q < KC; q++) {
-            const double xr = x[q].x, xi = x[q].y, hr = hs[2 * q], hi = hs[2 * q + 1];
+        for (int i = 0; i < PER; i++) p[i] = g + i * G < nb ? get_shared(col + g + i * G) : 0.0;
+#pragma unroll
+        for (int i = 0; i < PER; i++) v += p[i];
+#pragma unroll
+        for (int off = G / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+        if (g == 0) store(c, v);
+    }
+    if (threadIdx.x == 0) ((unsigned *)(res + kResCount))[y] = 0;
+}
+
+// sum over q of h_q x_q for the KC vectors from p on, added to (yr, yi) or
+// (SIGN < 0) subtracted from it; h uniform, read by scalar loads
+template <typename R, int KC, int SIGN>
+__device__ __forceinline__ void add_vectors(const VecPtrs &V, int p, const double *__restrict__ h,
+                                            uint64_t i, double &yr, double &yi)
+{
+    using T = typename Cx<R>::T;
+    T x[KC];
+#pragma unroll
+    for (int q = 0; q < KC; q++) x[q] = ((const T *)V.p[p + q])[i];
+#pragma unroll
+    for (int q = 0; q < KC; q++) {
+        const double xr = x[q].x, xi = x[q].y, hr = h[2 * (p + q)], hi = h[2 * (p + q) + 1];
+        if (SIGN < 0) {
             yr -= hr * xr - hi * xi;
             yi -= hr * xi + hi * xr;
+        } else {
+            yr += hr * xr - hi * xi;
+            yi += hr * xi + hi * xr;
         }
+    }
+}
+
+// w -= sum_q h_q V[q] over all k vectors (FP64 arithmetic, one rounding; KR =
+// k mod 16, 16 for 0: the vectors after the full chunks of 16, LONG where
+// there are any), h = res[0..2k).
+// Fused normalization (fuse_min > 0): beta^2 = ||w||^2 - sum |h_q|^2 is the
+// norm of the result when the basis is orthonormal; if beta^2 >= ||w||^2 / 2
+// (no cancellation to speak of) and beta >= fuse_min, the result is written
+// scaled by 1/beta and beta stored (else 0); otherwise the workgroups leave
+// partials of the result's norm.  Block 0 copies h and beta to host.
+//
+// Bound by HBM; the elements are walked from the end, where the dot sweep
+// just finished, so that what is left of the basis in the 256 MB Infinity
+// Cache is read from there.
+template <typename R, int KR, bool LONG>
+__global__ void __launch_bounds__(kRedThreads)
+k_gs_update(VecPtrs V, int k, typename Cx<R>::T *__restrict__ w, uint64_t n,
+            double *__restrict__ part, const double *__restrict__ hc, double *res, double fuse_min,
+            double *__restrict__ host, const int *__restrict__ stop)
+{
+    using T = typename Cx<R>::T;
+    __shared__ double sh[(kWaves + 1) * 1];
+    __shared__ double fbeta;
+    if (stop && *stop) return;
+    if (threadIdx.x < 64) {
+        const int q = threadIdx.x;
+        const double hr = q < k ? hc[2 * q] : 0.0, hi = q < k ? hc[2 * q + 1] : 0.0;
+        if (blockIdx.x == 0 && q < k) {
+            host[2 * q] = hr;
+            host[2 * q + 1] = hi;
+        }
+        double beta = 0.0;
+        if (fuse_min > 0) {
+            const double s2 = wave_sum(hr * hr + hi * hi), wn2 = hc[kResIn], b2 = wn2 - s2;
+            if (b2 > 0 && b2 >= 0.5 * wn2 && sqrt(b2) >= fuse_min) beta = sqrt(b2);
+        }
+        if (q == 0) {
+            fbeta = beta;
+            if (blockIdx.x == 0) {
+                res[kResBeta] = beta;
+                host[kResBeta] = beta;
+            }
+        }
+    }
+    __syncthreads();
+    const double beta = fbeta, f = beta > 0 ? 1.0 / beta : 1.0;
+    double nacc[1] = {0.0};
+    const uint64_t rows = (n + kRedThreads - 1) / kRedThreads;
+    for (uint64_t r = blockIdx.x; r < rows; r += gridDim.x) {
+        const uint64_t i = (rows - 1 - r) * kRedThreads + threadIdx.x;
+        if (i >= n) continue;
+        const T e = w[i];
+        double yr = e.x, yi = e.y;
+        int p = 0;
+        if constexpr (LONG)
+            for (; p + kUpdChunk < k; p += kUpdChunk)
+                add_vectors<R, kUpdChunk, -1>(V, p, hc, i, yr, yi);
+        add_vectors<R, KR, -1>(V, p, hc, i, yr, yi);
         T o;
         o.x = (R)(yr * f);
         o.y = (R)(yi * f);
@@ -284,95 +444,88 @@ k_gs_update(VecPtrs16 V, const double *__restrict__ h, typename Cx<R>::T *__rest
         const double orr = o.x, oi = o.y;
         nacc[0] += orr * orr + oi * oi;
     }
-    if (partial) {
+    if (beta == 0) {
         block_reduce<1>(nacc, sh);
-        if (threadIdx.x == 0) partial[blockIdx.x] = sh[kWaves];
+        if (threadIdx.x == 0) part[blockIdx.x] = sh[kWaves];
     }
 }
 
-// y += sum_q c[q] V[q] for the KC vectors of one chunk (FP64 arithmetic)
-template <typename R, int KC>
+// The end of a pass that was not fused (nothing to do after one that was):
+// every workgroup adds the nb norm partials in the same order; block 0 gives
+// the norm to res (and as the second coefficient of a Lanczos step behind)
+// and to host.  With scale, w is divided by the norm unless it is below
+// min_norm or not a number: then stop is set for the Arnoldi steps queued
+// behind, and w left as the pass made it.
+template <typename R>
 __global__ void __launch_bounds__(kRedThreads)
-k_lincomb(VecPtrs16 V, Coefs16 c, typename Cx<R>::T *__restrict__ y, uint64_t n)
+k_gs_finish(typename Cx<R>::T *__restrict__ w, uint64_t n, const double *__restrict__ part, int nb,
+            double *res, int scale, double min_norm, double *__restrict__ host, int *stop)
+{
+    __shared__ double sh[(kWaves + 1) * 1];
+    if ((stop && *(volatile int *)stop) || res[kResBeta] > 0) return;
+    double v[1] = {0.0};
+    for (int p = threadIdx.x; p < nb; p += kRedThreads) v[0] += part[p];
+    block_reduce<1>(v, sh);
+    const double norm = sqrt(sh[kWaves]);
+    const bool ok = norm >= min_norm;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        res[2] = norm;
+        res[3] = 0.0;
+        host[kResNorm] = norm;
+        if (scale && !ok && stop) *stop = 1;
+    }
+    if (!scale || !ok) return;
+    const R f = (R)(1.0 / norm);
+    GRID_STRIDE(i, n) {
+        auto e = w[i];
+        e.x *= f;
+        e.y *= f;
+        w[i] = e;
+    }
+}
+
+// y += sum_q c[q] V[q] over k vectors (FP64 arithmetic, one rounding; KR as
+// in k_gs_update)
+template <typename R, int KR, bool LONG>
+__global__ void __launch_bounds__(kRedThreads)
+k_lincomb(VecPtrs V, Coefs c, int k, typename Cx<R>::T *__restrict__ y, uint64_t n)
 {
     using T = typename Cx<R>::T;
     GRID_STRIDE(i, n) {
         T o = y[i];
-        T x[KC];
-#pragma unroll
-        for (int q = 0; q < KC; q++) x[q] = ((const T *)V.p[q])[i];
         double yr = o.x, yi = o.y;
-#pragma unroll
-        for (int q = 0; q < KC; q++) {
-            const double xr = x[q].x, xi = x[q].y, cr = c.c[2 * q], ci = c.c[2 * q + 1];
-            yr += cr * xr - ci * xi;
-            yi += cr * xi + ci * xr;
-        }
+        int p = 0;
+        if constexpr (LONG)
+            for (; p + kUpdChunk < k; p += kUpdChunk)
+                add_vectors<R, kUpdChunk, 1>(V, p, c.c, i, yr, yi);
+        add_vectors<R, KR, 1>(V, p, c.c, i, yr, yi);
         o.x = (R)yr;
         o.y = (R)yi;
         y[i] = o;
     }
 }
 
-// norm^2 / sum |x|^2 partials
-template <typename R>
-__global__ void __launch_bounds__(kRedThreads)
-k_nrm2_partial(const typename Cx<R>::T *__restrict__ a, uint64_t n, double *__restrict__ partial)
-{
-    __shared__ double sh[(kWaves + 1) * 1];
-    double acc[1] = {0.0};
-    GRID_STRIDE(i, n) {
-        auto x = a[i];
-        double xr = x.x, xi = x.y;
-        acc[0] += xr * xr + xi * xi;
-    }
-    block_reduce<1>(acc, sh);
-    if (threadIdx.x == 0) partial[blockIdx.x] = sh[kWaves];
-}
-
-template <typename R>
-__global__ void __launch_bounds__(kRedThreads)
-k_dot_partial(const typename Cx<R>::T *__restrict__ a, const typename Cx<R>::T *__restrict__ b,
-              uint64_t n, double *__restrict__ partial)
-{
-    __shared__ double sh[(kWaves + 1) * 2];
-    double acc[2] = {0.0, 0.0};
-    GRID_STRIDE(i, n) {
-        auto x = a[i];
-        auto y = b[i];
-        double xr = x.x, xi = x.y, yr = y.x, yi = y.y;
-        acc[0] += xr * yr + xi * yi;
-        acc[1] += xr * yi - xi * yr;
-    }
-    block_reduce<2>(acc, sh);
-    if (threadIdx.x < 2) partial[2 * blockIdx.x + threadIdx.x] = sh[kWaves * 2 + threadIdx.x];
-}
-
 // ---------------------------------------------------------------------------
 // host helpers
 // ---------------------------------------------------------------------------
+constexpr size_t kPartDoubles = (size_t)kRedBlocks * (2 * kMaxVecs + 1);
 static inline double *ws_partial() { return (double *)ctx().work; }
-// [0, B*(2*kMaxVecs+1)): dot partials (2 kMaxVecs columns of coefficients
-// and one of ||w||^2 per block); [B*2*kMaxVecs, B*(2*kMaxVecs+1)): norm
-// partials of the update, written after the dot partials are reduced; then
-// the reduced results (B = kRedBlocks)
-static inline double *ws_result()
-{
-    return (double *)ctx().work + (size_t)kRedBlocks * (2 * kMaxVecs + 1);
-}
+static inline double *ws_result() { return ws_partial() + kPartDoubles; }
 
 // The Gram-Schmidt pass's workspace in a file-scope device array, for
 // rp_gs_pass_fused_noalloc: the partials and results of the library
 // workspace layout above, 1.06 MB.  Each device holds its own copy; the
 // host reaches it only through the address hipGetSymbolAddress returns for
 // the current device (taken once per device at rp_init).
-constexpr size_t kGsScratchDoubles = (size_t)kRedBlocks * (2 * kMaxVecs + 1) + 2 * kMaxVecs + 8;
-static __device__ __align__(256) double scratch[kGsScratchDoubles];
+static __device__ __align__(256) double scratch[kPartDoubles + kResDoubles];
 static std::vector<double *> g_scratch_ptr;     // per device, null until set up
 
 int vec_scratch_setup(int device)
 {
     if (device < 0) return set_error(RP_ERR_INVALID_ARGUMENT, "bad device %d", device);
+    // the arrival counters and the stop flag start at zero
+    RP_CHECK_HIP(hipMemsetAsync(ws_result(), 0, kResDoubles * sizeof(double), ctx().stream));
+    RP_CHECK_HIP(hipStreamSynchronize(ctx().stream));
     if ((size_t)device >= g_scratch_ptr.size()) g_scratch_ptr.resize(device + 1, nullptr);
     if (g_scratch_ptr[device]) return RP_OK;
     void *p = nullptr;
@@ -390,46 +543,21 @@ static double *vec_scratch(int device)
     return g_scratch_ptr[device];
 }
 
+// workgroups of a sweep: one element per thread up to 2^16 elements, then
+// four, so that a row of dot partials stays short; at most kRedBlocks
 static inline int red_blocks(uint64_t n)
 {
-    return grid_for(n, kRedThreads, kRedBlocks);
+    const uint64_t one = (n + kRedThreads - 1) / kRedThreads;
+    if (one <= 256) return (int)(one < 1 ? 1 : one);
+    const uint64_t four = (n + 4 * kRedThreads - 1) / (4 * kRedThreads);
+    return (int)(four < 256 ? 256 : four > (uint64_t)kRedBlocks ? kRedBlocks : four);
 }
 
-// copy `cnt` doubles from a device result area (default: the workspace's)
-// to the host (synchronizes)
-static int fetch_results(double *dst, int cnt, const double *src = nullptr)
+// wait for the queued kernels: their results are then in pinned host memory
+static int wait_results()
 {
-    Context &c = ctx();
-    RP_CHECK_HIP(hipMemcpyAsync(c.pinned, src ? src : ws_result(), sizeof(double) * cnt,
-                                hipMemcpyDeviceToHost, c.stream));
-    RP_CHECK_HIP(hipStreamSynchronize(c.stream));
+    RP_CHECK_HIP(hipStreamSynchronize(ctx().stream));
     prof_collect();
-    memcpy(dst, c.pinned, sizeof(double) * cnt);
-    return RP_OK;
-}
-
-template <typename R>
-static int dot_impl(const void *a, const void *b, uint64_t n, double *out2)
-{
-    using T = typename Cx<R>::T;
-    int nb = red_blocks(n);
-    RP_LAUNCH(RP_KERNEL_OTHER, k_dot_partial<R>, dim3(nb), dim3(kRedThreads), 0,
-              (const T *)a, (const T *)b, n, ws_partial());
-    RP_LAUNCH(RP_KERNEL_OTHER, k_reduce_cols, dim3(2), dim3(kRedThreads), 0,
-              (const double *)ws_partial(), nb, 2, ws_result());
-    return fetch_results(out2, 2);
-}
-
-template <typename R>
-static int nrm2_launch(const void *a, uint64_t n, double *dst_dev, double *part = nullptr)
-{
-    using T = typename Cx<R>::T;
-    int nb = red_blocks(n);
-    if (!part) part = ws_partial();
-    RP_LAUNCH(RP_KERNEL_OTHER, k_nrm2_partial<R>, dim3(nb), dim3(kRedThreads), 0,
-              (const T *)a, n, part);
-    RP_LAUNCH(RP_KERNEL_OTHER, k_reduce_cols, dim3(1), dim3(kRedThreads), 0,
-              (const double *)part, nb, 1, dst_dev);
     return RP_OK;
 }
 
@@ -446,78 +574,169 @@ static int nrm2_launch(const void *a, uint64_t n, double *dst_dev, double *part 
     case 15: LAUNCH(15); break; default: LAUNCH(16); break;                       \
     }
 
-// One Gram-Schmidt pass; res layout: [0, 2k) h, [2 kMaxVecs] ||w_out||^2,
-// [2 kMaxVecs + 1] ||w_in||^2, [2 kMaxVecs + 2] fused beta (0: not fused)
-// pre / pre_rows: the dot partials of w already formed by the apply's
-// epilogue (rows of width doubles, ||w||^2 in column 2 kMaxVecs); the pass
-// then starts from their reduction
+// queue the dots of w against V[0..k) and ||w||^2 (k = 0: only that).  Each
+// workgroup takes up to 8 vectors (w is read once for all of them), 4 where
+// the vectors are so short that more workgroups matter more.
+template <typename R>
+static int dots_launch(int cls, const VecPtrs &P, int k, const void *w, uint64_t n, double *work,
+                       int real, double *host, const int *stop)
+{
+    using T = typename Cx<R>::T;
+    const int most = n <= (1u << 15) ? kDotChunk / 2 : kDotChunk;
+    const int rows = k > 0 ? (k + most - 1) / most : 1;
+    const int kc = (k + rows - 1) / rows;
+    const int nt = n <= (1u << 16) ? 256 : 1024;
+    const dim3 grid((unsigned)std::min<uint64_t>((n + nt - 1) / nt, kDotBlocks), rows);
+    double *res = work + kPartDoubles;
+#define RP_DOTS(KC)                                                               \
+    if (nt == 256)                                                                \
+        RP_LAUNCH(cls, (k_gs_dots<R, KC, 256>), grid, dim3(256), 0, P, k, (const T *)w, n, work,   \
+                  res, real, host, stop);                                         \
+    else                                                                          \
+        RP_LAUNCH(cls, (k_gs_dots<R, KC, 1024>), grid, dim3(1024), 0, P, k, (const T *)w, n, work, \
+                  res, real, host, stop);                                         \
+    break
+    switch (kc) {
+    case 0: RP_DOTS(0);
+    case 1: RP_DOTS(1);
+    case 2: RP_DOTS(2);
+    case 3: RP_DOTS(3);
+    case 4: RP_DOTS(4);
+    case 5: RP_DOTS(5);
+    case 6: RP_DOTS(6);
+    case 7: RP_DOTS(7);
+    default: RP_DOTS(8);
+    }
+#undef RP_DOTS
+    return RP_OK;
+}
+
+// queue the update of w by V[0..k) and the end of the pass
+template <typename R>
+static int update_launch(const VecPtrs &P, int k, void *w, uint64_t n, double *work, double *host,
+                         double fuse_min, int scale, double min_norm, int *stop)
+{
+    using T = typename Cx<R>::T;
+    const int nb = red_blocks(n), kr = (k - 1) % kUpdChunk + 1;
+    double *res = work + kPartDoubles;
+#define RP_UPD(KR)                                                                \
+    RP_LAUNCH(RP_KERNEL_GS, (k_gs_update<R, KR, false>), dim3(nb), dim3(kRedThreads), 0, P, k,     \
+              (T *)w, n, work, (const double *)res, res, fuse_min, host, (const int *)stop)
+#define RP_UPD_LONG(KR)                                                           \
+    RP_LAUNCH(RP_KERNEL_GS, (k_gs_update<R, KR, true>), dim3(nb), dim3(kRedThreads), 0, P, k,      \
+              (T *)w, n, work, (const double *)res, res, fuse_min, host, (const int *)stop)
+    if (k <= kUpdChunk) {
+        RP_KC_SWITCH(kr, RP_UPD)
+    } else {
+        RP_KC_SWITCH(kr, RP_UPD_LONG)
+    }
+#undef RP_UPD
+#undef RP_UPD_LONG
+    RP_LAUNCH(RP_KERNEL_GS, k_gs_finish<R>, dim3(scale ? nb : 1), dim3(kRedThreads), 0, (T *)w, n,
+              (const double *)work, nb, res, scale, min_norm, host, stop);
+    return RP_OK;
+}
+
+// One Gram-Schmidt pass.  pre / pre_rows: the dot partials of w already
+// formed by the apply's epilogue (rows of 2 kMaxVecs + 1 doubles, ||w||^2 in
+// the last column); the pass then starts from their reduction
 template <typename R>
 static int gs_pass_impl(const void *const *V, int k, void *w, uint64_t n, double *h,
                         double *norm, double fuse_min, int *normalized, double *work = nullptr,
                         const double *pre = nullptr, uint64_t pre_rows = 0)
 {
-    using T = typename Cx<R>::T;
-    const int nb = red_blocks(n);
-    const int width = 2 * kMaxVecs + 1;
-    // the workspace: the library's, or the caller-chosen one of the same layout
-    double *const part = work ? work : ws_partial();
-    double *res = part + (size_t)kRedBlocks * (2 * kMaxVecs + 1);
-    double *npart = part + (size_t)kRedBlocks * (2 * kMaxVecs);   // norm partials
-    const bool fuse = fuse_min > 0 && k > 0;
+    double *host = ctx().pinned;
+    if (!work) work = ws_partial();
+    double *res = work + kPartDoubles;
+    VecPtrs P{};
+    for (int q = 0; q < k; q++) P.p[q] = V[q];
+    int st;
     if (pre) {
+        const int width = 2 * kMaxVecs + 1;
         if (k > 0)
             RP_LAUNCH(RP_KERNEL_GS, k_reduce_cols, dim3(2 * k), dim3(kRedThreads), 0, pre,
                       (int)pre_rows, width, res);
-        RP_LAUNCH(RP_KERNEL_GS, k_reduce_cols, dim3(1), dim3(kRedThreads), 0,
-                  pre + 2 * kMaxVecs, (int)pre_rows, width,
-                  res + 2 * kMaxVecs + (k > 0 ? 1 : 0));
-    } else if (k > 0) {
-        for (int q0 = 0; q0 < k; q0 += kDotChunk) {
-            const int kc = k - q0 < kDotChunk ? k - q0 : kDotChunk;
-            VecPtrs16 P{};
-            for (int q = 0; q < kc; q++) P.p[q] = V[q0 + q];
-            const int wn = fuse && q0 == 0;
-#define RP_DOTS(KC)                                                               \
-    RP_LAUNCH(RP_KERNEL_GS, (k_dots<R, KC>), dim3(nb), dim3(kRedThreads), 0, P, (const T *)w, n, \
-              part, width, q0, wn)
-            RP_KC_SWITCH(kc, RP_DOTS)
-#undef RP_DOTS
-        }
-        RP_LAUNCH(RP_KERNEL_GS, k_reduce_cols, dim3(2 * k), dim3(kRedThreads), 0,
-                  (const double *)part, nb, width, res);
-        if (fuse)
-            RP_LAUNCH(RP_KERNEL_GS, k_reduce_cols, dim3(1), dim3(kRedThreads), 0,
-                      (const double *)part + 2 * kMaxVecs, nb, width,
-                      res + 2 * kMaxVecs + 1);
+        RP_LAUNCH(RP_KERNEL_GS, k_reduce_cols, dim3(1), dim3(kRedThreads), 0, pre + 2 * kMaxVecs,
+                  (int)pre_rows, width, k > 0 ? res + kResIn : host + kResIn);
+    } else if ((st = dots_launch<R>(RP_KERNEL_GS, P, k, w, n, work, 0,
+                                    k > 0 ? nullptr : host, nullptr))) {
+        return st;
     }
-    if (k == 0) {
-        if (!pre) {
-            int st = nrm2_launch<R>(w, n, res + 2 * kMaxVecs, part);
-            if (st) return st;
-        }
-    } else {
-        for (int q0 = 0; q0 < k; q0 += kUpdChunk) {
-            const int kc = k - q0 < kUpdChunk ? k - q0 : kUpdChunk;
-            const bool last = q0 + kc == k;
-            VecPtrs16 P{};
-            for (int q = 0; q < kc; q++) P.p[q] = V[q0 + q];
-#define RP_UPD(KC)                                                                \
-    RP_LAUNCH(RP_KERNEL_GS, (k_gs_update<R, KC>), dim3(nb), dim3(kRedThreads), 0, P,          \
-              (const double *)(res + 2 * q0), (T *)w, n, last ? npart : (double *)nullptr,   \
-              (const double *)res, k, (last && fuse) ? fuse_min : 0.0)
-            RP_KC_SWITCH(kc, RP_UPD)
-#undef RP_UPD
-        }
-        RP_LAUNCH(RP_KERNEL_GS, k_reduce_cols, dim3(1), dim3(kRedThreads), 0,
-                  (const double *)npart, nb, 1, res + 2 * kMaxVecs);
-    }
-    double tmp[2 * kMaxVecs + 3];
-    int st = fetch_results(tmp, 2 * kMaxVecs + 3, res);
-    if (st) return st;
-    for (int q = 0; q < 2 * k; q++) h[q] = tmp[q];
-    const double beta = fuse ? tmp[2 * kMaxVecs + 2] : 0.0;
+    if (k > 0 &&
+        (st = update_launch<R>(P, k, w, n, work, host, fuse_min, 0, 0.0, (int *)nullptr)))
+        return st;
+    if ((st = wait_results())) return st;
+    for (int q = 0; q < 2 * k; q++) h[q] = host[q];
+    const double beta = k > 0 ? host[kResBeta] : 0.0;
     if (normalized) *normalized = beta > 0 ? 1 : 0;
-    *norm = beta > 0 ? beta : sqrt(tmp[2 * kMaxVecs]);
+    *norm = k == 0 ? sqrt(host[kResIn]) : beta > 0 ? beta : host[kResNorm];
+    return RP_OK;
+}
+
+template <typename R>
+static int dot_impl(const void *a, const void *b, uint64_t n, double *out2)
+{
+    double *host = ctx().pinned;
+    VecPtrs P{};
+    P.p[0] = a;
+    int st = dots_launch<R>(RP_KERNEL_OTHER, P, 1, b, n, ws_partial(), 0, host, nullptr);
+    if (st || (st = wait_results())) return st;
+    out2[0] = host[0];
+    out2[1] = host[1];
+    return RP_OK;
+}
+
+template <typename R>
+static int nrm2_impl(const void *a, uint64_t n, double *nrm)
+{
+    double *host = ctx().pinned;
+    int st = dots_launch<R>(RP_KERNEL_OTHER, VecPtrs{}, 0, a, n, ws_partial(), 0, host, nullptr);
+    if (st || (st = wait_results())) return st;
+    *nrm = sqrt(host[kResIn]);
+    return RP_OK;
+}
+
+// Steps j0 .. m-1 of an Arnoldi (or Lanczos) recurrence queued without a wait
+// between them: every step applies, forms its coefficients, updates and
+// normalizes on the device and leaves its results in a pinned slot of its
+// own; one wait ends them all.  A step whose norm is below min_norm raises
+// the stop flag, which every kernel queued behind it reads first.
+template <typename R>
+static int steps_impl(rp_terms_t hd, void *const *V, int j0, int m, uint64_t n, double min_norm,
+                      int lanczos)
+{
+    Context &c = ctx();
+    double *work = ws_partial(), *res = ws_result();
+    int *stop = lanczos ? nullptr : (int *)(res + kResStop);
+    int st = RP_OK;
+    VecPtrs P{};
+    if (!lanczos)
+        for (int j = 0; j < j0; j++) P.p[j] = V[j];
+    for (int j = j0; j < m; j++) {
+        double *host = c.pinned + kHostSteps + (size_t)(j - j0) * kHostSlot;
+        // not reached before the stop: neither normalized nor a norm
+        host[kResBeta] = 0;
+        host[kResNorm] = 0;
+    }
+    for (int j = j0; j < m; j++) {
+        double *host = c.pinned + kHostSteps + (size_t)(j - j0) * kHostSlot;
+        if ((st = apply_queued(hd, V[j + 1], V[j], stop))) break;
+        if (lanczos) {
+            P.p[0] = V[j];
+            P.p[1] = j > j0 ? V[j - 1] : nullptr;
+            if ((st = dots_launch<R>(RP_KERNEL_GS, P, 1, V[j + 1], n, work, 1, host, stop))) break;
+            if (j == m - 1) break;
+            st = update_launch<R>(P, j > j0 ? 2 : 1, V[j + 1], n, work, host, 0.0, 1, 0.0, stop);
+        } else {
+            P.p[j] = V[j];
+            if ((st = dots_launch<R>(RP_KERNEL_GS, P, j + 1, V[j + 1], n, work, 0, nullptr,
+                                     stop))) break;
+            st = update_launch<R>(P, j + 1, V[j + 1], n, work, host, min_norm, 1, min_norm, stop);
+        }
+        if (st) break;
+    }
+    const int wst = wait_results();
+    if (st || wst) return st ? st : wst;
     return RP_OK;
 }
 
@@ -526,19 +745,28 @@ static int lincomb_impl(void *y, const void *const *V, int k, const double *c, u
 {
     using T = typename Cx<R>::T;
     const int nb = red_blocks(n);
-    for (int q0 = 0; q0 < k; q0 += kUpdChunk) {
-        const int kc = k - q0 < kUpdChunk ? k - q0 : kUpdChunk;
-        VecPtrs16 P{};
-        Coefs16 C{};
+    for (int q0 = 0; q0 < k; q0 += kMaxVecs) {
+        const int kc = k - q0 < kMaxVecs ? k - q0 : kMaxVecs, kr = (kc - 1) % kUpdChunk + 1;
+        VecPtrs P{};
+        Coefs C{};
         for (int q = 0; q < kc; q++) {
             P.p[q] = V[q0 + q];
             C.c[2 * q] = c[2 * (q0 + q)];
             C.c[2 * q + 1] = c[2 * (q0 + q) + 1];
         }
-#define RP_LC(KC)                                                                 \
-    RP_LAUNCH(RP_KERNEL_OTHER, (k_lincomb<R, KC>), dim3(nb), dim3(kRedThreads), 0, P, C, (T *)y, n)
-        RP_KC_SWITCH(kc, RP_LC)
+#define RP_LC(KR)                                                                 \
+    RP_LAUNCH(RP_KERNEL_OTHER, (k_lincomb<R, KR, false>), dim3(nb), dim3(kRedThreads), 0, P, C, kc,\
+              (T *)y, n)
+#define RP_LC_LONG(KR)                                                            \
+    RP_LAUNCH(RP_KERNEL_OTHER, (k_lincomb<R, KR, true>), dim3(nb), dim3(kRedThreads), 0, P, C, kc, \
+              (T *)y, n)
+        if (kc <= kUpdChunk) {
+            RP_KC_SWITCH(kr, RP_LC)
+        } else {
+            RP_KC_SWITCH(kr, RP_LC_LONG)
+        }
 #undef RP_LC
+#undef RP_LC_LONG
     }
     return RP_OK;
 }
@@ -546,9 +774,6 @@ static int lincomb_impl(void *y, const void *const *V, int k, const double *c, u
 }  // namespace rp
 
 using namespace rp;
-
-#define RP_PREC_DISPATCH(prec, FN, ...)                                           \
-    ((prec) == RP_C64 ? FN<float>(__VA_ARGS__) : FN<double>(__VA_ARGS__))
 
 extern "C" {
 
@@ -681,14 +906,7 @@ int rp_vec_norm(int prec, const void *v, uint64_t n, double *nrm)
     RP_REQUIRE(nrm, "null output");
     if (n == 0) { *nrm = 0; return RP_OK; }
     RP_REQUIRE(v, "null vector");
-    st = prec == RP_C64 ? nrm2_launch<float>(v, n, ws_result())
-                        : nrm2_launch<double>(v, n, ws_result());
-    if (st) return st;
-    double s;
-    st = fetch_results(&s, 1);
-    if (st) return st;
-    *nrm = sqrt(s);
-    return RP_OK;
+    return prec == RP_C64 ? nrm2_impl<float>(v, n, nrm) : nrm2_impl<double>(v, n, nrm);
 }
 
 int rp_init_random(int prec, void *v, uint64_t n, uint64_t seed)
@@ -827,6 +1045,71 @@ int rp_apply_gs(rp_terms_t hd, void *res, const void *vec, const void *const *V,
                                      (const double *)c.epi_work, rows)
                : gs_pass_impl<double>(V, k, res, n, h, norm, fuse_min, normalized, nullptr,
                                       (const double *)c.epi_work, rows);
+}
+
+static int steps_check(rp_terms_t hd, void *const *V, int j0, int m, const double *out,
+                       rp_terms_info_t *info)
+{
+    int st = check_init();
+    if (st) return st;
+    RP_REQUIRE(hd, "null term handle");
+    RP_REQUIRE(V && out, "null argument");
+    RP_REQUIRE(j0 >= 0 && j0 < m && m <= kMaxVecs, "need 0 <= j0 < m <= 64");
+    for (int j = 0; j <= m; j++) {
+        RP_REQUIRE(V[j], "null basis vector");
+        RP_REQUIRE(j == 0 || V[j] != V[j - 1], "consecutive vectors must be different buffers");
+    }
+    return rp_terms_info(hd, info);
+}
+
+int rp_arnoldi_steps(rp_terms_t hd, void *const *V, int j0, int m, double min_norm, double *out,
+                     int *done)
+{
+    rp_terms_info_t info;
+    int st = steps_check(hd, V, j0, m, out, &info);
+    if (st) return st;
+    RP_REQUIRE(done, "null argument");
+    RP_REQUIRE(min_norm > 0, "min_norm must be positive");
+    for (int j = 0; j <= m; j++)
+        for (int i = 0; i < j; i++) RP_REQUIRE(V[i] != V[j], "vectors must be different buffers");
+    const uint64_t n = 1ull << info.len;
+    st = info.prec == RP_C64 ? steps_impl<float>(hd, V, j0, m, n, min_norm, 0)
+                             : steps_impl<double>(hd, V, j0, m, n, min_norm, 0);
+    const double *slots = ctx().pinned + kHostSteps;
+    *done = 0;
+    bool raised = st != RP_OK;
+    for (int j = j0; j < m && !raised; j++) {
+        const double *s = slots + (size_t)(j - j0) * kHostSlot, beta = s[kResBeta];
+        double *o = out + (size_t)(j - j0) * RP_STEP_DOUBLES;
+        for (int q = 0; q < 2 * (j + 1); q++) o[q] = s[q];
+        o[2 * kMaxVecs] = beta > 0 ? beta : s[kResNorm];
+        o[2 * kMaxVecs + 1] = beta > 0 ? 1.0 : 0.0;
+        (*done)++;
+        raised = !(beta > 0 || s[kResNorm] >= min_norm);
+    }
+    // the stop flag is taken down for the next call
+    if (raised)
+        RP_CHECK_HIP(hipMemsetAsync(ws_result() + kResStop, 0, sizeof(double), ctx().stream));
+    return st;
+}
+
+int rp_lanczos_steps(rp_terms_t hd, void *const *V, int m, double *alpha, double *beta)
+{
+    rp_terms_info_t info;
+    int st = steps_check(hd, V, 0, m, alpha, &info);
+    if (st) return st;
+    RP_REQUIRE(m == 1 || beta, "null argument");
+    for (int j = 2; j <= m; j++) RP_REQUIRE(V[j] != V[j - 2], "vectors must be different buffers");
+    const uint64_t n = 1ull << info.len;
+    st = info.prec == RP_C64 ? steps_impl<float>(hd, V, 0, m, n, 0.0, 1)
+                             : steps_impl<double>(hd, V, 0, m, n, 0.0, 1);
+    if (st) return st;
+    for (int j = 0; j < m; j++) {
+        const double *s = ctx().pinned + kHostSteps + (size_t)j * kHostSlot;
+        alpha[j] = s[0];
+        if (j < m - 1) beta[j] = s[kResNorm];
+    }
+    return RP_OK;
 }
 
 int rp_lincomb(int prec, void *y, const void *const *V, int k, const double *c, uint64_t n)

@@ -78,7 +78,52 @@ class Krylov {
                         int &m, double &beta, Reorth mode, KrylovStats &st) {
         const size_t dim = s.dim();
         const auto len = s.spin_chain_length();
-        for (int j = j0; j < m; j++) {
+        // With the selective criterion nearly every step ends after one
+        // pass.  A backend that can queues all steps on that assumption and
+        // waits once; the step that needs another pass is the last of them,
+        // gets it here, and the rest go one by one.
+        int j = j0;
+        if constexpr (requires(std::vector<const typename Impl::template VecType<FpType> *> &V,
+                               std::vector<typename Impl::ArnoldiStep> &q) {
+                          Impl::arnoldi_steps(len, A, V, 0, 0.0, q);
+                      }) {
+            const double eta = 1 / std::sqrt(2.0), norm0 = eta / 2;
+            std::vector<const typename Impl::template VecType<FpType> *> V(m + 1);
+            for (int i = 0; i <= m; i++) {
+                (void)s.buf(i);
+                V[i] = &s.vec(i);
+            }
+            std::vector<typename Impl::ArnoldiStep> q;
+            if (mode == Reorth::Selective && j0 < m && !Impl::fused_first_pass() &&
+                Impl::arnoldi_steps(len, A, V, j0, eta * norm0, q)) {
+                for (auto &step : q) {
+                    bool normalized = step.normalized, ok = true;
+                    st.matvecs++;
+                    if (normalized || step.norm >= eta * norm0) {
+                        st.gs_passes++;
+                        beta = step.norm;
+                        for (int i = 0; i <= j; i++) H(i, j) = step.h[i];
+                    } else {
+                        // its first pass is done; V_{j+1} is not normalized
+                        ok = orthogonalize(s, H, j, beta, mode, st, normalized,
+                                           [&](auto &, std::vector<cd> &r, double, bool &nz) {
+                                               r = step.h;
+                                               nz = false;
+                                               return step.norm;
+                                           });
+                        if (ok && !normalized)
+                            Impl::scale_vec(dim, s.buf(j + 1), (FpType)(1.0 / beta));
+                    }
+                    if (!ok) {
+                        m = j + 1;
+                        return false;
+                    }
+                    if (j != m - 1) H(j + 1, j) = beta;
+                    j++;
+                }
+            }
+        }
+        for (; j < m; j++) {
             bool normalized, ok;
             using VecList = std::vector<const typename Impl::template VecType<FpType> *>;
             bool fused = false;
@@ -290,7 +335,19 @@ public:
         int numiter = 0;
         double energy = 0;
         while (true) {
-            for (int i = 0; i < krydim; i++) {
+            bool queued = false;
+            if constexpr (requires(std::vector<const typename Impl::template VecType<FpType> *> &V) {
+                              Impl::lanczos_steps(len, ham, V, alpha, beta);
+                          }) {
+                // all steps queued on the device, one wait
+                std::vector<const typename Impl::template VecType<FpType> *> V(krydim + 1);
+                for (int i = 0; i <= krydim; i++) {
+                    (void)s.buf(i);
+                    V[i] = &s.vec(i);
+                }
+                queued = Impl::lanczos_steps(len, ham, V, alpha, beta);
+            }
+            for (int i = 0; i < krydim && !queued; i++) {
                 Impl::apply_ops_overwrite(len, s.buf(i + 1), ham, s.buf(i));
                 alpha[i] = Impl::vec_prod64(dim, s.buf(i), s.buf(i + 1)).real();
                 if (i == krydim - 1) break;

@@ -456,6 +456,55 @@ public:
         return nrm;
     }
 
+    // One queued step of an Arnoldi recurrence (rp_arnoldi_steps)
+    struct ArnoldiStep {
+        std::vector<std::complex<double>> h;
+        double norm;
+        bool normalized;
+    };
+
+    // Arnoldi steps j0 .. V.size()-2 on the basis V, up to and including the
+    // first whose norm after one Gram-Schmidt pass is below min_norm; false
+    // (and nothing done) where the operator is applied as a dense matrix
+    template<RealScalar FpType>
+    static bool arnoldi_steps(typename SpinOp<FpType>::IndexType len,
+                              const DevSumOps<FpType> &ops,
+                              const std::vector<const DeviceVec<FpType> *> &V, int j0,
+                              double min_norm, std::vector<ArnoldiStep> &steps) {
+        if (use_dense(len, ops)) return false;
+        std::vector<void *> p(V.size());
+        for (size_t i = 0; i < V.size(); i++) p[i] = (void *)V[i]->ptr;
+        const int m = (int)V.size() - 1;
+        std::vector<double> out((size_t)RP_STEP_DOUBLES * (m - j0));
+        int done = 0;
+        RP_CALL(rp_arnoldi_steps(ops.device_terms(len), p.data(), j0, m, min_norm, out.data(),
+                                 &done));
+        steps.resize(done);
+        for (int s = 0; s < done; s++) {
+            const double *o = out.data() + (size_t)RP_STEP_DOUBLES * s;
+            steps[s].h.resize(j0 + s + 1);
+            for (int i = 0; i <= j0 + s; i++) steps[s].h[i] = {o[2 * i], o[2 * i + 1]};
+            steps[s].norm = o[2 * RP_MAX_SWEEP_VECS];
+            steps[s].normalized = o[2 * RP_MAX_SWEEP_VECS + 1] != 0;
+        }
+        return true;
+    }
+
+    // the Lanczos steps of Krylov::ground_state on the vectors V (rp_lanczos_steps);
+    // false (and nothing done) where they are not available
+    template<RealScalar FpType>
+    static bool lanczos_steps(typename SpinOp<FpType>::IndexType len,
+                              const DevSumOps<FpType> &ops,
+                              const std::vector<const DeviceVec<FpType> *> &V,
+                              std::vector<double> &alpha, std::vector<double> &beta) {
+        const int m = (int)V.size() - 1;
+        if (use_dense(len, ops) || m > RP_MAX_SWEEP_VECS) return false;
+        std::vector<void *> p(V.size());
+        for (size_t i = 0; i < V.size(); i++) p[i] = (void *)V[i]->ptr;
+        RP_CALL(rp_lanczos_steps(ops.device_terms(len), p.data(), m, alpha.data(), beta.data()));
+        return true;
+    }
+
     // res = mat * vec for a dim x dim device matrix (mat_mul,
     // inc/gpuimpl.h:1009-1022); res and vec must differ
     template<RealScalar FpType, typename Mat>

@@ -1,0 +1,177 @@
+"""Queued Krylov steps (rp_arnoldi_steps, rp_lanczos_steps) and the
+Gram-Schmidt sweeps at the edges of their launch shapes, against numpy in 64
+bits.
+
+Tolerances: a dot product or norm of n terms accumulated in FP64 is off by at
+most n eps64 relative to the product of the norms, far below the one rounding
+of each stored component, eps(state) / 2; sums over k vectors and the
+normalization add a few of those."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from conftest import random_pauli_sum
+from gpu_util import DeviceBuffer, Terms, prec_of
+
+pytestmark = pytest.mark.gpu
+
+_vp = ctypes.c_void_p
+EPS = {np.complex64: 6e-8, np.complex128: 1.2e-16}
+STEP = 2 * 64 + 2
+
+
+def _hermitian(rng, length, nterms):
+    """Random Pauli strings with phases that make every term Hermitian."""
+    bits, _ = random_pauli_sum(rng, length, nterms)
+    co = []
+    for b in bits:
+        y = sum(1 for s in range(length) if (int(b) >> (2 * s)) & 3 == 3)
+        co.append(rng.standard_normal() * 1j ** (y % 4))
+    return bits, np.array(co)
+
+
+def _dense(length, bits, coeff):
+    n = 1 << length
+    m = np.zeros((n, n), np.complex128)
+    i = np.arange(n)
+    for b, c in zip(bits, coeff):
+        x = sum(((int(b) >> (2 * s)) & 1) << s for s in range(length))
+        z = sum(((int(b) >> (2 * s + 1)) & 1) << s for s in range(length))
+        sign = np.array([(-1) ** bin(v & z).count("1") for v in range(n)])
+        m[i ^ x, i] += c * sign
+    return m
+
+
+def _arnoldi(H, v, m):
+    V, h = [v], np.zeros((m + 1, m), np.complex128)
+    for j in range(m):
+        w = H @ V[j]
+        c = np.array([np.vdot(u, w) for u in V])
+        w = w - sum(a * u for a, u in zip(c, V))
+        h[:j + 1, j] = c
+        h[j + 1, j] = np.linalg.norm(w)
+        V.append(w / h[j + 1, j])
+    return V, h
+
+
+def _ptrs(bufs):
+    return (_vp * len(bufs))(*[b.ptr.value for b in bufs])
+
+
+@pytest.mark.parametrize("dtype", [np.complex64, np.complex128])
+@pytest.mark.parametrize("length,m,j0", [(2, 2, 0), (5, 9, 0), (9, 19, 0), (9, 6, 2), (10, 34, 0)])
+def test_arnoldi_steps(gpu, dtype, length, m, j0):
+    rng = np.random.default_rng(100 * length + m)
+    bits, co = _hermitian(rng, length, 6 * length)
+    if dtype == np.complex64:
+        co = co.real.astype(np.float32).astype(float) + 1j * co.imag.astype(np.float32).astype(float)
+    n = 1 << length
+    H, hnorm = _dense(length, bits, co), np.abs(co).sum()     # ||H|| <= sum |c|
+    v = rng.standard_normal(n) + 1j * rng.standard_normal(n)
+    V, h = _arnoldi(H, v / np.linalg.norm(v), m)
+    t = Terms(length, bits, co, prec_of(dtype))
+    bufs = [DeviceBuffer.from_array((V[j] if j <= j0 else np.zeros(n)).astype(dtype))
+            for j in range(m + 1)]
+    out, done = np.zeros((m - j0, STEP)), ctypes.c_int()
+    gpu.check(gpu.hip().rp_arnoldi_steps(t.h, _ptrs(bufs), j0, m, 1e-3,
+                                         out.ctypes.data_as(_vp), ctypes.byref(done)))
+    assert done.value == m - j0
+    # one rounding per stored component, carried through the recurrence: each
+    # step multiplies the error of the last by about ||H|| / H(j+1, j)
+    grow = np.cumprod([max(1.0, hnorm / abs(h[j + 1, j])) for j in range(m)])
+    for j in range(j0, m):
+        o = out[j - j0]
+        tol = 8 * EPS[dtype] * grow[j]
+        got = o[0:2 * j + 2:2] + 1j * o[1:2 * j + 2:2]
+        assert np.abs(got - h[:j + 1, j]).max() <= tol * hnorm
+        assert abs(o[128] - h[j + 1, j]) <= tol * hnorm
+        assert o[129] in (0.0, 1.0)
+        got = bufs[j + 1].to_array(dtype, n)
+        assert np.linalg.norm(got - V[j + 1]) <= tol
+        assert abs(np.linalg.norm(got.astype(np.complex128)) - 1) <= 4 * EPS[dtype]
+
+
+@pytest.mark.parametrize("dtype", [np.complex64, np.complex128])
+def test_arnoldi_steps_stop(gpu, dtype):
+    """An invariant subspace: Z0 + 2 X1 acts on |00> in a space of dimension
+    2, so step 1 leaves nothing; the steps behind it do not run, and the next
+    call starts clean."""
+    length, m = 2, 6
+    bits, co = np.array([2, 1 << 2], np.uint64), np.array([1.0, 2.0 + 0j])
+    t = Terms(length, bits, co, prec_of(dtype))
+    for _ in range(2):
+        v = np.zeros(4, dtype)
+        v[0] = 1
+        mark = np.full(4, 7, dtype)
+        bufs = [DeviceBuffer.from_array(v if j == 0 else mark) for j in range(m + 1)]
+        out, done = np.zeros((m, STEP)), ctypes.c_int()
+        gpu.check(gpu.hip().rp_arnoldi_steps(t.h, _ptrs(bufs), 0, m, 0.25,
+                                             out.ctypes.data_as(_vp), ctypes.byref(done)))
+        assert done.value == 2
+        assert np.allclose(out[0, :2], [1, 0]) and out[0, 128] == 2.0
+        assert abs(out[1, 128]) < 1e-6
+        for j in range(3, m + 1):
+            assert np.array_equal(bufs[j].to_array(dtype, 4), mark)
+
+
+@pytest.mark.parametrize("length,m", [(3, 1), (3, 2), (8, 12), (10, 30)])
+def test_lanczos_steps(gpu, length, m):
+    rng = np.random.default_rng(length)
+    bits, co = _hermitian(rng, length, 4 * length)
+    n = 1 << length
+    H, hnorm = _dense(length, bits, co), np.abs(co).sum()     # ||H|| <= sum |c|
+    v = rng.standard_normal(n) + 1j * rng.standard_normal(n)
+    V, al, be = [v / np.linalg.norm(v)], [], []
+    for i in range(m):
+        w = H @ V[i]
+        al.append(np.vdot(V[i], w).real)
+        if i == m - 1:
+            break
+        w = w - al[i] * V[i] - (be[i - 1] * V[i - 1] if i else 0)
+        be.append(np.linalg.norm(w))
+        V.append(w / be[i])
+    t = Terms(length, bits, co, gpu.RP_C128)
+    bufs = [DeviceBuffer.from_array(V[0] if j == 0 else np.zeros(n, np.complex128))
+            for j in range(m + 1)]
+    a, b = np.zeros(m), np.zeros(max(1, m - 1))
+    gpu.check(gpu.hip().rp_lanczos_steps(t.h, _ptrs(bufs), m, a.ctypes.data_as(_vp),
+                                         b.ctypes.data_as(_vp)))
+    grow = np.cumprod([max(1.0, hnorm / x) for x in be] or [1.0])[-1]
+    tol = 16 * 1.2e-16 * grow * hnorm
+    assert np.abs(a - al).max() <= tol
+    assert np.abs(b[:m - 1] - be).max() <= tol if m > 1 else True
+
+
+@pytest.mark.parametrize("dtype", [np.complex64, np.complex128])
+@pytest.mark.parametrize("n,k", [(1, 1), (63, 3), (256, 4), (257, 5), (32768, 17), (32769, 9),
+                                 (65536, 8), (65537, 16), (262143, 33), (300001, 2), (4096, 64)])
+def test_gs_pass_edges(gpu, dtype, n, k):
+    """One pass at the sizes where the launch shape changes (workgroup size
+    at 2^16 elements, vectors per workgroup at 2^15, chunks of 16 in the
+    update), twice in a row on the same workspace."""
+    rng = np.random.default_rng(n + k)
+    V = (rng.standard_normal((k, n)) + 1j * rng.standard_normal((k, n))) / np.sqrt(2 * n * k)
+    V = V.astype(dtype)
+    w = (rng.standard_normal(n) + 1j * rng.standard_normal(n)).astype(dtype)
+    V64, w64 = V.astype(np.complex128), w.astype(np.complex128)
+    ref = V64.conj() @ w64
+    r = w64 - ref @ V64
+    vb = [DeviceBuffer.from_array(V[q]) for q in range(k)]
+    for _ in range(2):
+        wb = DeviceBuffer.from_array(w)
+        h, nrm = np.zeros(2 * k), ctypes.c_double()
+        gpu.check(gpu.hip().rp_gs_pass(prec_of(dtype), _ptrs(vb), k, wb.ptr, n,
+                                       h.ctypes.data_as(_vp), ctypes.byref(nrm)))
+        size = np.linalg.norm(V64, axis=1).max() * np.linalg.norm(w64)
+        assert np.abs(h.view(np.complex128) - ref).max() <= 4e-16 * np.sqrt(n + 16) * size
+        got = wb.to_array(dtype, n).astype(np.complex128)
+        assert np.linalg.norm(got - r) <= 4 * EPS[dtype] * np.linalg.norm(w64)
+        assert abs(nrm.value - np.linalg.norm(got)) <= 1e-13 * max(nrm.value, 1e-300)
+    re, im = ctypes.c_double(), ctypes.c_double()
+    wb = DeviceBuffer.from_array(w)
+    gpu.check(gpu.hip().rp_vec_prod(prec_of(dtype), vb[0].ptr, wb.ptr, n, ctypes.byref(re),
+                                    ctypes.byref(im)))
+    assert abs(complex(re.value, im.value) - ref[0]) <= 4e-16 * np.sqrt(n + 16) * size
+    gpu.check(gpu.hip().rp_vec_norm(prec_of(dtype), wb.ptr, n, ctypes.byref(nrm)))
+    assert abs(nrm.value - np.linalg.norm(w64)) <= 1e-13 * nrm.value
