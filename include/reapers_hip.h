@@ -142,7 +142,7 @@ typedef struct {
     int      prec;          /* RP_C64 / RP_C128 */
     int      len;           /* spin chain length */
     int      tile_bits;     /* b: log2 of the amplitude tile one workgroup owns
-                               (0: one thread per amplitude, no tiles) */
+                               (0: no tiles) */
     uint64_t nterms;        /* terms after dropping zero coefficients */
     uint64_t nflips;        /* distinct flip masks x (G_0) */
     uint64_t ngroups;       /* distinct x >> b: input tile passes (G_b) */
@@ -158,8 +158,8 @@ typedef struct {
                                orders the groups by XCD class (0: contiguous tiles,
                                groups by flip mask) */
 } rp_terms_info_t;
-/* the apply kernel family a term handle launches: one thread per amplitude
-   (tile_bits 0); tiles with per-sub records; tiles with the compact sub
+/* the apply kernel family a term handle launches: one wavefront per 64 or 256
+   amplitudes and slice of the flip masks (tile_bits 0); tiles with per-sub records; tiles with the compact sub
    stream (complex<float>, group accumulation, two LDS tiles) */
 #define RP_APPLY_SMALL  0
 #define RP_APPLY_TILED  1
@@ -169,11 +169,11 @@ int rp_terms_info(rp_terms_t h, rp_terms_info_t *info);
  * in the reference): tile bits / threads / pipeline depth must be one of the
  * instantiated combinations -- (8,128,2), (10,128,2), (12,512,2) for both
  * precisions; (12,512,3), (12,512,4), (12,1024,2), (13,1024,2) for RP_C64; (11,256,4) for
- * RP_C128 -- or tile bits 0 with 256 threads: the one-thread-per-amplitude
- * kernel, its depth the number of term slices (1, 8, 32, 128) that
- * separate workgroups sum before a second pass adds them in slice order.
- * The autotuner (RP_TERMS_AUTOTUNE) chooses among the same set, the sliced
- * kernel only up to len 16. */
+ * RP_C128 -- or, up to len 16, tile bits 0 with 256 threads: the kernel
+ * without tiles, its depth the number of slices (1, 8, 32, 128) of the flip
+ * masks that separate wavefronts sum.  The autotuner (RP_TERMS_AUTOTUNE)
+ * chooses among the same set, the kernel without tiles up to len 18 and for
+ * at most 40 flip masks. */
 int rp_terms_set_tiling(rp_terms_t h, int tile_bits, int threads, int depth);
 
 /* GPUImpl::apply_ops + krnl_apply_ops (src/krnl.cu:220-257, 80-94):

@@ -49,18 +49,21 @@ constexpr int kSmallThreads = 256;
 struct rp_terms {
     int prec = RP_C64;
     int len = 0;
-    int tile_bits = 0;       // 0: small kernel (one thread per amplitude)
+    int tile_bits = 0;       // 0: no tiles (k_apply_wave)
     int threads = 0;         // workgroup size of the tiled kernel
-    int depth = 2;           // LDS tiles in the tiled kernel's pipeline; for the
-                             // small kernel the number of term slices (1: none)
+    int depth = 2;           // LDS tiles in the tiled kernel's pipeline; without
+                             // tiles the number of term slices (1: none)
     int acc64 = 1;           // accumulate in FP64
     int group_acc = 0;       // FP32 within a group, FP64 across groups (complex<float>)
     uint64_t nterms = 0, nflips = 0, ngroups = 0, nsubs = 0;
     rp::TileMap tmap{};               // output-tile order of the tiled kernels
-    void *d_groups = nullptr, *d_subs = nullptr, *d_terms = nullptr, *d_flat = nullptr;
+    void *d_groups = nullptr, *d_subs = nullptr, *d_terms = nullptr;
+    void *d_wflips = nullptr, *d_wsubs = nullptr, *d_wterms = nullptr, *d_wcut = nullptr;
+                                      // k_apply_wave
     void *d_cgroups = nullptr, *d_csubs = nullptr, *d_cterms = nullptr;   // compact stream
-    void *d_split = nullptr;          // per-slice partial sums of the split small kernel
-    size_t split_bytes = 0;
+    void *d_split = nullptr;          // per-slice partial sums of k_apply_wave and
+                                      // the arrival counters behind them
+    int rows = 1;                     // its amplitudes per lane
     double apply_passes = 0;          // measured apply cost in state passes (autotune)
     std::vector<uint64_t> raw_bits;   // the uploaded term list, for re-tiling
     std::vector<double> raw_coeff;
@@ -68,96 +71,290 @@ struct rp_terms {
 
 namespace rp {
 
-// one thread per amplitude; terms in (x-sorted) flat order
-template <typename R, typename A>
-__global__ void __launch_bounds__(kSmallThreads)
-k_apply_small(const typename CxA<R>::T *__restrict__ in, typename CxA<R>::T *__restrict__ out,
-              uint32_t dim, const FlatTerm<A> *__restrict__ terms, int nterms, int accumulate,
-              const int *__restrict__ stop)
+// XCD-aware numbering: consecutive workgroup ids go to different XCDs, so
+// give each XCD a contiguous range of tiles
+__device__ __forceinline__ uint32_t xcd_tile_index()
 {
-    if (stop && *stop) return;
-    uint32_t m = blockIdx.x * kSmallThreads + threadIdx.x;
-    if (m >= dim) return;
-    A ar = 0, ai = 0;
-    for (int t = 0; t < nterms; t++) {
-        const FlatTerm<A> f = terms[t];
-        const auto v = in[m ^ f.x];
-        const A vr = v.x, vi = v.y;
-        const bool neg = parity32(m & f.z);
-        const A cr = neg ? -f.cr : f.cr;
-        const A ci = neg ? -f.ci : f.ci;
-        ar += cr * vr - ci * vi;
-        ai += cr * vi + ci * vr;
-    }
-    if (accumulate) {
-        const auto o = out[m];
-        ar += (A)o.x;
-        ai += (A)o.y;
-    }
-    typename CxA<R>::T o;
-    o.x = (R)ar;
-    o.y = (R)ai;
-    out[m] = o;
+    const uint32_t nb = gridDim.x, b = blockIdx.x;
+    return (nb & 7u) == 0 ? (b & 7u) * (nb >> 3) + (b >> 3) : b;
 }
 
-// The small kernel with the terms split into gridDim.y slices: slice s sums
-// its contiguous range of the x-sorted terms for one amplitude per thread and
-// writes the partial sum; k_split_reduce adds the slices in slice order.  For
-// chains of up to 16 sites, where 2^len / 256 workgroups alone cannot fill
-// the GPU.
-template <typename R, typename A>
-__global__ void __launch_bounds__(kSmallThreads)
-k_apply_split(const typename CxA<R>::T *__restrict__ in, typename CxA<A>::T *__restrict__ part,
-              uint32_t dim, const FlatTerm<A> *__restrict__ terms, int nterms, int per,
-              const int *__restrict__ stop)
+// ---------------------------------------------------------------------------
+// The apply without tiles: a wavefront owns 64 ROWS consecutive amplitudes
+// (lane l the amplitudes r 64 + l of them) and gathers the input amplitudes of
+// one flip mask after the other straight from memory; the XOR keeps each
+// gather inside an aligned block of 64, so it is coalesced.  The terms that
+// share a flip mask are first summed to the coefficient they have at each
+// amplitude, d(m) = sum c (-1)^popcount(m & z), so that the amplitude is read
+// and multiplied once for all of them: 2 to 3 VALU instructions per term, the
+// lane part of its sign a 64-bit mask made at upload (a scalar operand of a
+// select), the part of the wavefront's own index bits scalar.  Terms with no
+// phase bit among the row bits are summed once for all rows.
+//
+// For chains of up to kWaveMaxLen sites, whose tiles are too few to fill the
+// 256 CUs, the flip masks are cut into `depth` slices of about equal work,
+// one per wavefront, so that all CUs have several wavefronts; the four of a
+// workgroup add their sums in LDS, workgroups through memory, the last one to
+// arrive in slice order.  Bound by latency there: dense SYK N=24 FP64 (10626
+// terms, 4096 amplitudes) took 33 us in one chain of loads per term and slice
+// and 14 us in a second launch that added the slices.
+// ---------------------------------------------------------------------------
+// One flip mask.  One or two terms of one kind (real, or kWaveImag imaginary
+// coefficients) stand in the record itself (kWaveTwo: two); kWaveRow: one of
+// them has phase bits among the row bits.  Otherwise (kWaveMulti) the terms
+// from `term` on: real ones without and with such bits, then imaginary ones
+// likewise, their counts z0, z1 and the halves of l0.
+template <typename A> struct alignas(16) SubW { uint64_t l0, l1; A c0, c1; uint32_t z0, z1, kind, term; };
+enum : uint32_t { kWaveImag = 1, kWaveRow = 2, kWaveTwo = 4, kWaveMulti = 8 };
+template <typename A> struct TermW { uint64_t lanes; A c; uint32_t z, pad; };
+
+constexpr int kWaveMaxLen = 18, kWaveMaxFlips = 40;
+constexpr int kWavePad = 16;       // flip masks read past the end of the list
+
+// c with the sign of (-1)^popcount(v), v uniform
+__device__ __forceinline__ float uniform_sign(float c, uint32_t v)
 {
-    if (stop && *stop) return;
-    uint32_t m = blockIdx.x * kSmallThreads + threadIdx.x;
-    if (m >= dim) return;
-    const int t0 = blockIdx.y * per;
-    const int t1 = min(nterms, t0 + per);
-    A ar = 0, ai = 0;
-    for (int t = t0; t < t1; t++) {
-        const FlatTerm<A> f = terms[t];
-        const auto v = in[m ^ f.x];
-        const A vr = v.x, vi = v.y;
-        const bool neg = parity32(m & f.z);
-        const A cr = neg ? -f.cr : f.cr;
-        const A ci = neg ? -f.ci : f.ci;
-        ar += cr * vr - ci * vi;
-        ai += cr * vi + ci * vr;
-    }
-    typename CxA<A>::T o;
-    o.x = ar;
-    o.y = ai;
-    part[(uint64_t)blockIdx.y * dim + m] = o;
+    return __uint_as_float(__float_as_uint(c) ^ ((uint32_t)__popc(v) << 31));
+}
+__device__ __forceinline__ double uniform_sign(double c, uint32_t v)
+{
+    return __hiloint2double(__double2hiint(c) ^ (int)((uint32_t)__popc(v) << 31), __double2loint(c));
+}
+// +-1 by the lane's bit of `neg`
+__device__ __forceinline__ float lane_sign(uint64_t neg, float)
+{
+    return __builtin_amdgcn_inverse_ballot_w64(neg) ? -1.f : 1.f;
+}
+__device__ __forceinline__ double lane_sign(uint64_t neg, double)
+{
+    return __hiloint2double(__builtin_amdgcn_inverse_ballot_w64(neg) ? 0xbff00000 : 0x3ff00000, 0);
 }
 
-template <typename R, typename A>
-__global__ void __launch_bounds__(kSmallThreads)
-k_split_reduce(const typename CxA<A>::T *__restrict__ part, typename CxA<R>::T *__restrict__ out,
-               uint32_t dim, int slices, int accumulate, const int *__restrict__ stop)
+// d[r] += one term (BYROW: it has phase bits among the row bits; otherwise
+// only d[0], which the caller copies); m0: the wavefront's first amplitude
+template <typename A, int ROWS, bool BYROW>
+__device__ __forceinline__ void add_term(const TermW<A> &C, uint32_t m0, A (&d)[ROWS])
 {
-    if (stop && *stop) return;
-    for (uint32_t m = blockIdx.x * kSmallThreads + threadIdx.x; m < dim;
-         m += gridDim.x * kSmallThreads) {
-        A ar = 0, ai = 0;
-        for (int sl = 0; sl < slices; sl++) {
-            const auto p = part[(uint64_t)sl * dim + m];
-            ar += p.x;
-            ai += p.y;
+    const A sg = lane_sign(C.lanes, A(0));
+#pragma unroll
+    for (int r = 0; r < (BYROW ? ROWS : 1); r++)
+        d[r] = fma(sg, uniform_sign(C.c, (m0 | (r * 64)) & C.z), d[r]);
+}
+
+template <typename A, int ROWS, bool BYROW>
+__device__ __forceinline__ void sum_terms(const TermW<A> *__restrict__ p, uint32_t n, uint32_t m0,
+                                          A (&d)[ROWS])
+{
+    uint32_t t = 0;
+    for (; t + 4 <= n; t += 4) {     // four records in flight
+        const TermW<A> C[4] = {p[t], p[t + 1], p[t + 2], p[t + 3]};
+#pragma unroll
+        for (int i = 0; i < 4; i++) add_term<A, ROWS, BYROW>(C[i], m0, d);
+    }
+    for (; t < n; t++) add_term<A, ROWS, BYROW>(p[t], m0, d);
+}
+
+// the coefficient of one flip mask at the wavefront's amplitudes: na terms
+// shared by all rows, nb by row
+template <typename A, int ROWS>
+__device__ __forceinline__ void sum_coef(const TermW<A> *__restrict__ p, uint32_t na, uint32_t nb,
+                                         uint32_t m0, A (&d)[ROWS])
+{
+    A one[1] = {0};
+    sum_terms<A, 1, false>(p, na, m0, one);
+#pragma unroll
+    for (int r = 0; r < ROWS; r++) d[r] = one[0];
+    if (ROWS > 1 && nb) sum_terms<A, ROWS, true>(p + na, nb, m0, d);
+}
+
+// acc += d v, or i d v
+template <typename T, typename A, int ROWS>
+__device__ __forceinline__ void add_rows(const A (&d)[ROWS], const T (&v)[ROWS], bool imag,
+                                         A (&ar)[ROWS], A (&ai)[ROWS])
+{
+    if (!imag) {
+#pragma unroll
+        for (int r = 0; r < ROWS; r++) {
+            ar[r] = fma(d[r], (A)v[r].x, ar[r]);
+            ai[r] = fma(d[r], (A)v[r].y, ai[r]);
         }
+    } else {
+#pragma unroll
+        for (int r = 0; r < ROWS; r++) {
+            ar[r] = fma(-d[r], (A)v[r].y, ar[r]);
+            ai[r] = fma(d[r], (A)v[r].x, ai[r]);
+        }
+    }
+}
+
+// W wavefronts per workgroup: with one slice each its own amplitudes, else
+// slices of the same ones
+template <typename R, typename A, int ROWS, int W>
+__global__ void __launch_bounds__(64 * W)
+k_apply_wave(const typename CxA<R>::T *__restrict__ in, typename CxA<R>::T *__restrict__ out,
+             uint64_t dim, const uint32_t *__restrict__ flips, const SubW<A> *__restrict__ subs,
+             const TermW<A> *__restrict__ terms, const uint32_t *__restrict__ cut, int depth,
+             int accumulate, double *__restrict__ part, unsigned *__restrict__ count,
+             const int *__restrict__ stop)
+{
+    using T = typename CxA<R>::T;
+    constexpr int U = ROWS == 1 ? 4 : 2;       // flip masks whose gathers go out together
+    constexpr bool SLICED = W > 4;
+    __shared__ A sh[SLICED ? 2 * ROWS : 1][W][64];
+    if (stop && *stop) return;
+    const uint32_t lane = threadIdx.x & 63;
+    const uint32_t wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // one slice: each XCD a contiguous range of amplitudes
+    const uint32_t chunk = SLICED ? blockIdx.x : xcd_tile_index() * W + wid;
+    const uint32_t slice = SLICED ? blockIdx.y * W + wid : 0;
+    const uint32_t m0 = chunk * (64 * ROWS);
+    if (!SLICED && m0 >= dim) return;          // the grid is whole workgroups
+    // fewer than 64 amplitudes: the upper lanes repeat the lower ones
+    const uint32_t ll = dim < 64 ? lane & ((uint32_t)dim - 1) : lane;
+    A ar[ROWS], ai[ROWS];
+#pragma unroll
+    for (int r = 0; r < ROWS; r++) { ar[r] = 0; ai[r] = 0; }
+    const uint32_t s0 = cut[slice], s1 = cut[slice + 1];
+
+    auto gather = [&](const uint32_t (&x)[U], T (&v)[U][ROWS]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+            for (int r = 0; r < ROWS; r++)
+                v[u][r] = (in + ((m0 | (r * 64)) ^ (x[u] & ~63u)))[ll ^ (x[u] & 63u)];
+    };
+    auto load_flips = [&](uint32_t s, uint32_t (&x)[U]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < U; u++) x[u] = flips[s + u];
+    };
+    auto apply = [&](const SubW<A> &S, const T (&v)[ROWS]) __attribute__((always_inline)) {
+        A d[ROWS];
+        if (S.kind & kWaveMulti) {
+            const uint32_t n2 = (uint32_t)S.l0, n3 = (uint32_t)(S.l0 >> 32);
+            const TermW<A> *p = terms + S.term;
+            if (S.z0 + S.z1) {
+                sum_coef<A, ROWS>(p, S.z0, S.z1, m0, d);
+                add_rows<T, A, ROWS>(d, v, false, ar, ai);
+            }
+            if (n2 + n3) {
+                sum_coef<A, ROWS>(p + S.z0 + S.z1, n2, n3, m0, d);
+                add_rows<T, A, ROWS>(d, v, true, ar, ai);
+            }
+            return;
+        }
+        const A g0 = lane_sign(S.l0, A(0)), g1 = lane_sign(S.l1, A(0));
+        if (ROWS > 1 && (S.kind & kWaveRow)) {
+#pragma unroll
+            for (int r = 0; r < ROWS; r++) {
+                d[r] = g0 * uniform_sign(S.c0, (m0 | (r * 64)) & S.z0);
+                d[r] = fma(g1, uniform_sign(S.c1, (m0 | (r * 64)) & S.z1), d[r]);
+            }
+        } else {
+            d[0] = g0 * uniform_sign(S.c0, m0 & S.z0);
+            if (S.kind & kWaveTwo) d[0] = fma(g1, uniform_sign(S.c1, m0 & S.z1), d[0]);
+#pragma unroll
+            for (int r = 1; r < ROWS; r++) d[r] = d[0];
+        }
+        add_rows<T, A, ROWS>(d, v, S.kind & kWaveImag, ar, ai);
+    };
+    // the gathers of the next U flip masks are in flight while the current
+    // ones are used, their masks loaded one step earlier
+    uint32_t xn[U];
+    T va[U][ROWS], vb[U][ROWS];
+    load_flips(s0, xn);
+    gather(xn, va);
+    load_flips(s0 + U, xn);
+    auto step = [&](uint32_t s, T (&cur)[U][ROWS], T (&nxt)[U][ROWS]) __attribute__((always_inline)) {
+        // the records as words: an array of the struct itself goes to scratch
+        constexpr int NW = sizeof(SubW<A>) / 4;
+        uint32_t S[U][NW];
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+            for (int i = 0; i < NW; i++) S[u][i] = ((const uint32_t *)(subs + s + u))[i];
+        if (s + U < s1) gather(xn, nxt);
+        load_flips(s + 2 * U, xn);
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (s + u < s1) apply(__builtin_bit_cast(SubW<A>, S[u]), cur[u]);
+    };
+    for (uint32_t s = s0; s < s1; s += 2 * U) {
+        step(s, va, vb);
+        if (s + U < s1) step(s + U, vb, va);
+    }
+
+    if constexpr (SLICED) {
+        // the slices of this workgroup, then those of the others
+#pragma unroll
+        for (int r = 0; r < ROWS; r++) {
+            sh[2 * r][wid][lane] = ar[r];
+            sh[2 * r + 1][wid][lane] = ai[r];
+        }
+        __syncthreads();
+        if (wid) return;
+#pragma unroll
+        for (int r = 0; r < ROWS; r++) {
+            ar[r] = sh[2 * r][0][lane];
+            ai[r] = sh[2 * r + 1][0][lane];
+#pragma unroll
+            for (int w = 1; w < W; w++) {
+                ar[r] += sh[2 * r][w][lane];
+                ai[r] += sh[2 * r + 1][w][lane];
+            }
+        }
+        const uint32_t nw = gridDim.y;
+        if constexpr (W == 16) {
+            double *row = part + (size_t)chunk * nw * (128 * ROWS) + lane;
+#pragma unroll
+            for (int r = 0; r < ROWS; r++) {
+                double *q = row + (size_t)blockIdx.y * (128 * ROWS) + r * 128;
+                put_shared(q, (double)ar[r]);
+                put_shared(q + 64, (double)ai[r]);
+            }
+            if (!arrive_last(count + chunk, nw)) return;
+            // at most 8 workgroups: all their sums in flight
+            double p[8][2 * ROWS];
+#pragma unroll
+            for (int i = 0; i < 8; i++)
+#pragma unroll
+                for (int r = 0; r < 2 * ROWS; r++)
+                    p[i][r] = (uint32_t)i < nw
+                                  ? get_shared(row + (size_t)i * (128 * ROWS) + r * 64)
+                                  : 0.0;
+            if (lane == 0) count[chunk] = 0;
+#pragma unroll
+            for (int r = 0; r < ROWS; r++) {
+                double sr = p[0][2 * r], si = p[0][2 * r + 1];
+#pragma unroll
+                for (int i = 1; i < 8; i++) {
+                    sr += p[i][2 * r];
+                    si += p[i][2 * r + 1];
+                }
+                ar[r] = (A)sr;
+                ai[r] = (A)si;
+            }
+        }
+    }
+    if (lane >= dim) return;
+#pragma unroll
+    for (int r = 0; r < ROWS; r++) {
+        T *o = out + (size_t)m0 + r * 64 + lane;
+        A xr = ar[r], xi = ai[r];
         if (accumulate) {
-            const auto o = out[m];
-            ar += (A)o.x;
-            ai += (A)o.y;
+            const T b = *o;
+            xr += (A)b.x;
+            xi += (A)b.y;
         }
-        typename CxA<R>::T o;
-        o.x = (R)ar;
-        o.y = (R)ai;
-        out[m] = o;
+        T e;
+        e.x = (R)xr;
+        e.y = (R)xi;
+        *o = e;
     }
 }
+
+// wavefronts per workgroup of k_apply_wave: for 8 slices one workgroup, for
+// 32 and 128 two and eight of 16 wavefronts
+static int wave_width(int depth) { return depth == 1 ? 4 : depth == 8 ? 8 : 16; }
 
 template <typename R, int TB, int NT, int D = 2>
 constexpr int apply_waves_per_eu()
@@ -518,14 +715,6 @@ __device__ __forceinline__ void apply_tile(const typename CxA<R>::T *__restrict_
         out[m] = o;
         wv[r] = o;
     }
-}
-
-// XCD-aware numbering: consecutive workgroup ids go to different XCDs, so
-// give each XCD a contiguous range of tiles
-__device__ __forceinline__ uint32_t xcd_tile_index()
-{
-    const uint32_t nb = gridDim.x, b = blockIdx.x;
-    return (nb & 7u) == 0 ? (b & 7u) * (nb >> 3) + (b >> 3) : b;
 }
 
 // the workgroup's output tile under the map tm (rp_tables.h): index bits
@@ -932,8 +1121,8 @@ constexpr int tiling_key(int tb, int nt, int d) { return tb * 100000 + nt * 10 +
 // the tilings the tiled kernel is instantiated for: {tile bits, threads,
 // pipeline depth, element bytes (0: both precisions)}
 struct TilingDesc { int tb, nt, depth, esz; };
-// Tile bits 0 is the small kernel, its depth the number of term slices.
-constexpr int kSplitMaxLen = 16;
+// Tile bits 0 is the kernel without tiles, its depth the number of term slices.
+constexpr int kSplitMaxLen = 16;       // rp_terms_set_tiling takes it up to here
 constexpr TilingDesc kTilings[] = {
     {0, kSmallThreads, 1, 0}, {0, kSmallThreads, 8, 0}, {0, kSmallThreads, 32, 0},
     {0, kSmallThreads, 128, 0},
@@ -949,28 +1138,54 @@ static bool tiling_instantiated(int prec, int tb, int nt, int d)
     return false;
 }
 
-// default tiling (RP_TERMS_AUTOTUNE measures the alternatives).  Up to 16
-// sites the small kernel, its terms split into slices when 2^len / 256
-// workgroups are too few for the term count: the largest power-of-two slice
-// count up to 128 that keeps at most 2048 workgroups and 32 terms per slice.
-// Beyond, the tiled kernel: 8 amplitudes per thread, smaller tiles and
-// workgroups for shorter chains so that there are enough workgroups.
-static void choose_tiling(int prec, int len, uint64_t nterms, int group_acc, int *tb, int *nt,
-                          int *depth)
+// distinct flip masks of a term list (zero coefficients included)
+static uint64_t count_flips(const uint64_t *bits, uint64_t n)
+{
+    std::vector<uint32_t> x(n);
+    for (uint64_t t = 0; t < n; t++) x[t] = pext_even(bits[t]);
+    std::sort(x.begin(), x.end());
+    return (uint64_t)(std::unique(x.begin(), x.end()) - x.begin());
+}
+
+// slices of the flip masks for the kernel without tiles: the most that keep
+// about 8192 wavefronts (the GPU holds that many; with 8 slices each lane has
+// four amplitudes from 17 sites on) and the work of 24 terms a slice
+static int wave_depth(int len, uint64_t flips, uint64_t nterms)
+{
+    const uint64_t chunks = len > 6 ? 1ull << (len - 6) : 1;
+    int d = 1;
+    for (int s : {8, 32, 128})
+        if (chunks * s <= (s == 8 ? 32768 : 8192) && flips >= (uint64_t)s &&
+            6 * flips + nterms >= (uint64_t)(24 * s))
+            d = s;
+    return d;
+}
+
+// default tiling (RP_TERMS_AUTOTUNE measures the alternatives)
+static void choose_tiling(int prec, int len, uint64_t flips, uint64_t nterms, int group_acc,
+                          int *tb, int *nt, int *depth)
 {
     *depth = 2;
-    if (len <= kSplitMaxLen) {
-        uint64_t blocks = std::max<uint64_t>(1, (1ull << len) / kSmallThreads);
-        int sl = 1;
-        while (sl < 128 && blocks * (uint64_t)(2 * sl) <= 2048 && nterms >= (uint64_t)(64 * sl))
-            sl *= 2;
-        if (sl > 1 || len < 10) {
-            *tb = 0;
-            *nt = kSmallThreads;
-            *depth = sl;
-            return;
-        }
+    // No tiles for short chains, nor for few flip masks with several terms
+    // each, whose sums the tiled kernel forms for every row.  us per apply
+    // without tiles / with (12, 512, 2), FP64 sums, default upload:
+    //   sparse SYK, k = 8, complex<float>:  16 sites 19 / 93, 18 sites 48 / 110
+    //   XXZ with fields (4 terms a mask):   20 sites 21 / 40, 24 sites 241 / 431,
+    //     26 sites 1072 / 1814, complex<double> 24 sites 392 / 728
+    //   XY chain (2 a mask):                20 sites 16 / 28, 24 sites 196 / 297
+    //   transverse Ising (under 2):         22 sites 54 / 60, 24 sites 205 / 204
+    //   one a mask, 20 masks:               22 sites 54 / 50, 24 sites 249 / 189
+    // and with group accumulation XY 20 sites 16 / 23, 24 sites 199 / 244, but
+    // 26 sites (beyond the Infinity Cache) 1071 / 1030, XXZ there 1072 / 1461.
+    const bool several = nterms >= 2 * flips &&
+                         !(group_acc && len >= 25 && 2 * nterms < 5 * flips);
+    if (len <= kWaveMaxLen || (flips <= kWaveMaxFlips && several)) {
+        *tb = 0;
+        *nt = kSmallThreads;
+        *depth = wave_depth(len, flips, nterms);
+        return;
     }
+    // Beyond, the tiled kernel: 8 amplitudes per thread.
     // 2^12-amplitude tiles with 512 threads: for complex<float> sparse SYK at
     // 24 qubits faster than 2^13 tiles (more groups, but two workgroups per
     // CU instead of one); for complex<double> the largest tile in 128 KiB.
@@ -979,10 +1194,8 @@ static void choose_tiling(int prec, int len, uint64_t nterms, int group_acc, int
     // sparse SYK at 30 qubits takes 197 ms there against 260 ms with 2^12
     // tiles
     if (prec == RP_C64 && group_acc && len >= 28) { *tb = 13; *nt = 1024; return; }
-    if (len >= 18) { *tb = 12; *nt = 512; return; }
-    if (len >= 14) { *tb = 10; *nt = 128; return; }
-    *tb = 8;
-    *nt = 128;
+    *tb = 12;
+    *nt = 512;
 }
 
 // the compact lists of the tiled tables (complex<float> states, FP64 term
@@ -1028,6 +1241,15 @@ static bool compact_stream(const Tables<double> &tab, std::vector<GroupC> &cg,
     return true;
 }
 
+// bytes of the partial sums of k_apply_wave: (re, im) of every amplitude from
+// each workgroup of its slices, where there are several
+static size_t wave_part_bytes(const rp_terms *h)
+{
+    const int wgs = h->depth / wave_width(h->depth);
+    const uint64_t dim = std::max<uint64_t>(64ull * h->rows, 1ull << h->len);
+    return wgs > 1 ? (size_t)dim * 2 * sizeof(double) * wgs : 0;
+}
+
 // log2 of the tiled kernel's resident workgroups per XCD (32 CUs) at the
 // occupancy apply_waves_per_eu gives it: the p of its output-tile map
 static int xcd_resident_bits(int prec, int tb, int nt, int depth)
@@ -1039,6 +1261,93 @@ static int xcd_resident_bits(int prec, int tb, int nt, int depth)
     int p = 5;
     while ((2 << p) <= 32 * wg) p++;
     return p;
+}
+
+// The tables of k_apply_wave from the x-sorted terms: one record per flip
+// mask, its terms by class, and the cuts of the flip masks into h->depth
+// slices of about equal work (a flip mask costs about as much as six terms:
+// the gather, its address and the products).
+template <typename A, typename UP>
+static int upload_wave(rp_terms *h, const std::vector<FlatTerm<A>> &flat, UP &&up)
+{
+    const uint64_t dim = 1ull << h->len;
+    // four amplitudes per lane where that leaves enough wavefronts
+    h->rows = h->depth <= 8 && dim * (uint64_t)h->depth >= (1ull << 20) ? 4 : 1;
+    std::vector<SubW<A>> subs;
+    std::vector<TermW<A>> terms;
+    std::vector<uint32_t> flips;
+    std::vector<uint64_t> cost(1, 0);
+    auto lanes = [](uint32_t z) {
+        uint64_t m = 0;
+        for (uint32_t l = 0; l < 64; l++) m |= (uint64_t)(__builtin_popcount(l & z) & 1) << l;
+        return m;
+    };
+    const uint32_t rowbits = 64u * (h->rows - 1);
+    for (size_t i = 0; i < flat.size();) {
+        size_t j = i;
+        bool re = true, im = true;
+        for (; j < flat.size() && flat[j].x == flat[i].x; j++) {
+            re = re && flat[j].ci == 0;
+            im = im && flat[j].cr == 0;
+        }
+        SubW<A> S{};
+        uint64_t work = 6;
+        if (j - i <= 2 && (re || im)) {
+            const FlatTerm<A> &a = flat[i], &b = flat[j - 1];
+            S.kind = (re ? 0 : kWaveImag) | (((a.z | b.z) & rowbits) ? kWaveRow : 0);
+            S.c0 = re ? a.cr : a.ci;
+            S.z0 = a.z;
+            S.l0 = lanes(a.z);
+            if (j - i == 2) {
+                S.kind |= kWaveTwo;
+                S.c1 = re ? b.cr : b.ci;
+                S.z1 = b.z;
+                S.l1 = lanes(b.z);
+            }
+            work += j - i;
+        } else {
+            uint32_t n[4] = {0, 0, 0, 0};
+            S.kind = kWaveMulti;
+            S.term = (uint32_t)terms.size();
+            for (int k = 0; k < 4; k++)
+                for (size_t q = i; q < j; q++) {
+                    const A c = k < 2 ? flat[q].cr : flat[q].ci;
+                    const bool byrow = (flat[q].z & rowbits) != 0;
+                    if (c == 0 || byrow != (k & 1)) continue;
+                    terms.push_back({lanes(flat[q].z), c, flat[q].z, 0});
+                    n[k]++;
+                }
+            S.z0 = n[0];
+            S.z1 = n[1];
+            S.l0 = (uint64_t)n[3] << 32 | n[2];
+            work += n[0] + n[2] + (uint64_t)h->rows * (n[1] + n[3]);
+        }
+        cost.push_back(cost.back() + work);
+        subs.push_back(S);
+        flips.push_back(flat[i].x);
+        i = j;
+    }
+    const size_t nsubs = subs.size();
+    flips.resize(nsubs + kWavePad, 0);
+    subs.resize(nsubs + kWavePad);
+    std::vector<uint32_t> cut;
+    for (int s = 0; s <= h->depth; s++) {
+        const uint64_t want = cost.back() * (uint64_t)s / (uint64_t)h->depth;
+        cut.push_back((uint32_t)(std::lower_bound(cost.begin(), cost.end(), want) - cost.begin()));
+    }
+    int st;
+    if ((st = up(&h->d_wflips, flips.data(), flips.size() * sizeof(uint32_t)))) return st;
+    if ((st = up(&h->d_wsubs, subs.data(), subs.size() * sizeof(SubW<A>)))) return st;
+    if ((st = up(&h->d_wterms, terms.data(), terms.size() * sizeof(TermW<A>)))) return st;
+    if ((st = up(&h->d_wcut, cut.data(), cut.size() * sizeof(uint32_t)))) return st;
+    if (wave_part_bytes(h)) {
+        const size_t chunks = std::max<uint64_t>(1, dim / (64 * h->rows));
+        std::vector<char> z(wave_part_bytes(h) + chunks * sizeof(unsigned), 0);
+        if ((st = up(&h->d_split, z.data(), z.size()))) return st;
+    }
+    // the tables are host temporaries
+    RP_CHECK_HIP(hipStreamSynchronize(ctx().stream));
+    return RP_OK;
 }
 
 template <typename R, typename A>
@@ -1071,22 +1380,7 @@ static int upload_impl(rp_terms *h, const uint64_t *bits, const double *coeff, u
         RP_CHECK_HIP(hipMemcpyAsync(*dst, src, bytes, hipMemcpyHostToDevice, c.stream));
         return RP_OK;
     };
-    if ((st = up(&h->d_flat, flat.data(), flat.size() * sizeof(FlatTerm<A>)))) return st;
-    if (tb == 0 && h->depth > 1) {
-        size_t need = (size_t)h->depth * (1ull << h->len) * sizeof(typename CxA<A>::T);
-        if (h->split_bytes < need) {
-            if (h->d_split) (void)hipFree(h->d_split);
-            h->d_split = nullptr;
-            h->split_bytes = 0;
-            if (dev_malloc((void **)&h->d_split, need) != hipSuccess) {
-                (void)hipGetLastError();
-                h->d_split = nullptr;
-                return set_error(RP_ERR_OUT_OF_MEMORY, "Failed to allocate %zu bytes on GPU device.",
-                                 need);
-            }
-            h->split_bytes = need;
-        }
-    }
+    if (!tb && (st = upload_wave<A>(h, flat, up))) return st;
     if (tb) {
         if ((st = up(&h->d_groups, groups.data(), groups.size() * sizeof(GroupRuns)))) return st;
         if ((st = up(&h->d_subs, subs.data(), subs.size() * sizeof(SubRec<A>)))) return st;
@@ -1112,9 +1406,8 @@ static void free_handle(rp_terms *h)
     if (h->d_groups) (void)hipFree(h->d_groups);
     if (h->d_subs) (void)hipFree(h->d_subs);
     if (h->d_terms) (void)hipFree(h->d_terms);
-    if (h->d_flat) (void)hipFree(h->d_flat);
-    if (h->d_split) (void)hipFree(h->d_split);
-    for (void *p : {h->d_cgroups, h->d_csubs, h->d_cterms})
+    for (void *p : {h->d_cgroups, h->d_csubs, h->d_cterms, h->d_wflips, h->d_wsubs,
+                    h->d_wterms, h->d_wcut, h->d_split})
         if (p) (void)hipFree(p);
     delete h;
 }
@@ -1157,22 +1450,22 @@ static int apply_impl(rp_terms *h, void *res, const void *vec, int accumulate, c
         return RP_OK;
     }
     if (h->tile_bits == 0) {
-        int grid = (int)((dim + kSmallThreads - 1) / kSmallThreads);
-        if (h->depth > 1) {
-            using P = typename CxA<A>::T;
-            const int slices = h->depth;
-            const int per = (int)((h->nterms + slices - 1) / slices);
-            RP_LAUNCH(RP_KERNEL_APPLY, (k_apply_split<R, A>), dim3(grid, slices),
-                      dim3(kSmallThreads), 0, (const T *)vec, (P *)h->d_split, (uint32_t)dim,
-                      (const FlatTerm<A> *)h->d_flat, (int)h->nterms, per, stop);
-            RP_LAUNCH(RP_KERNEL_APPLY, (k_split_reduce<R, A>), dim3(grid), dim3(kSmallThreads), 0,
-                      (const P *)h->d_split, (T *)res, (uint32_t)dim, slices, accumulate,
-                      stop);
-            return RP_OK;
-        }
-        RP_LAUNCH(RP_KERNEL_APPLY, (k_apply_small<R, A>), dim3(grid), dim3(kSmallThreads), 0,
-                  (const T *)vec, (T *)res, (uint32_t)dim, (const FlatTerm<A> *)h->d_flat,
-                  (int)h->nterms, accumulate, stop);
+        const uint64_t chunks = std::max<uint64_t>(1, dim / (64 * h->rows));
+        const int w = wave_width(h->depth);
+        const dim3 grid = h->depth == 1 ? dim3((unsigned)((chunks + w - 1) / w))
+                                        : dim3((unsigned)chunks, h->depth / w);
+        unsigned *count = (unsigned *)((char *)h->d_split + wave_part_bytes(h));
+#define RP_WAVE(ROWS, W)                                                          \
+    RP_LAUNCH(RP_KERNEL_APPLY, (k_apply_wave<R, A, ROWS, W>), grid, dim3(64 * W), 0,              \
+              (const T *)vec, (T *)res, dim, (const uint32_t *)h->d_wflips,                      \
+              (const SubW<A> *)h->d_wsubs, (const TermW<A> *)h->d_wterms,                        \
+              (const uint32_t *)h->d_wcut, h->depth, accumulate, (double *)h->d_split, count, stop)
+        if (w == 16) RP_WAVE(1, 16);
+        else if (w == 8 && h->rows == 1) RP_WAVE(1, 8);
+        else if (w == 8) RP_WAVE(4, 8);
+        else if (h->rows == 1) RP_WAVE(1, 4);
+        else RP_WAVE(4, 4);
+#undef RP_WAVE
         return RP_OK;
     }
     switch (tiling_key(h->tile_bits, h->threads, h->depth)) {
@@ -1245,8 +1538,8 @@ static int upload_any(rp_terms *h, const uint64_t *bits, const double *coeff, ui
 
 static void free_tables(rp_terms *h)
 {
-    for (void **p : {&h->d_groups, &h->d_subs, &h->d_terms, &h->d_flat, &h->d_cgroups, &h->d_csubs,
-                     &h->d_cterms})
+    for (void **p : {&h->d_groups, &h->d_subs, &h->d_terms, &h->d_cgroups, &h->d_csubs,
+                     &h->d_cterms, &h->d_wflips, &h->d_wsubs, &h->d_wterms, &h->d_wcut, &h->d_split})
         if (*p) { (void)hipFree(*p); *p = nullptr; }
 }
 
@@ -1297,7 +1590,10 @@ static int autotune(rp_terms *h)
     for (const TilingDesc &cd : kTilings) {
         if (st) break;
         if (cd.tb > h->len || !tiling_instantiated(h->prec, cd.tb, cd.nt, cd.depth)) continue;
-        if (cd.tb == 0 && (h->len > kSplitMaxLen || h->nterms < (uint64_t)(2 * cd.depth))) continue;
+        if (cd.tb == 0 && (cd.depth == 1 ? h->len > kWaveMaxLen && h->nflips > kWaveMaxFlips
+                                         : h->len > kWaveMaxLen ||
+                                               h->nterms < (uint64_t)(2 * cd.depth)))
+            continue;
         if ((st = retile(h, cd.tb, cd.nt, cd.depth))) break;
         if ((st = apply_dispatch(h, y, x, 0))) break;
         if (hipEventRecord(e0, c.stream) != hipSuccess) { st = RP_ERR_RUNTIME; break; }
@@ -1356,7 +1652,7 @@ int rp_terms_upload_ex(rp_terms_t *out, int prec, int len, const uint64_t *bits,
     h->len = len;
     h->acc64 = (prec == RP_C128 || !(flags & RP_TERMS_ACC_NATIVE)) ? 1 : 0;
     h->group_acc = (prec == RP_C64 && (flags & RP_TERMS_ACC_GROUP)) ? 1 : 0;
-    choose_tiling(prec, len, nterms, h->group_acc, &h->tile_bits, &h->threads, &h->depth);
+    choose_tiling(prec, len, count_flips(bits, nterms), nterms, h->group_acc, &h->tile_bits, &h->threads, &h->depth);
     h->raw_bits.assign(bits, bits + nterms);
     h->raw_coeff.assign(coeff, coeff + 2 * nterms);
     st = upload_any(h, bits, coeff, nterms);
@@ -1392,10 +1688,8 @@ int rp_terms_set_tiling(rp_terms_t h, int tile_bits, int threads, int depth)
     if (st) return st;
     RP_REQUIRE(h, "null term handle");
     RP_REQUIRE(tile_bits <= h->len, "tile bits exceed the chain length");
-    // the one-thread-per-amplitude kernels index 32-bit amplitudes and the
-    // sliced one keeps depth * 2^len partial sums
-    RP_REQUIRE(tile_bits != 0 || h->len <= kSplitMaxLen,
-               "tile bits 0 (one thread per amplitude) only up to len 16");
+    // the sliced kernel keeps depth / 4 * 2^len partial sums
+    RP_REQUIRE(tile_bits != 0 || h->len <= kSplitMaxLen, "tile bits 0 only up to len 16");
     RP_REQUIRE(tiling_instantiated(h->prec, tile_bits, threads, depth),
                "tiling not instantiated for this precision");
     RP_CHECK_HIP(hipStreamSynchronize(ctx().stream));

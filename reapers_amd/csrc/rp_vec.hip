@@ -228,32 +228,6 @@ __device__ __forceinline__ void wave_multi_sum(double (&v)[NV])
     for (; off > 0; off >>= 1) v[0] += __shfl_xor(v[0], off, 64);
 }
 
-// Partials that another workgroup of the same launch reads: written through
-// to memory and read past the caches (device-scope accesses), with a wait
-// for the writes before the arrival is counted.  A device-scope fence would
-// order them too, but it writes the whole L2 back: with one in each of 2048
-// workgroups a dot sweep over 12 vectors of 2^23 complex<float> took 267 us
-// instead of 172.
-__device__ __forceinline__ void put_shared(double *p, double v)
-{
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ double get_shared(const double *p)
-{
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-// count this workgroup's arrival, its writes by put_shared complete (called
-// by the wavefront that made them); true in the last of n workgroups
-__device__ __forceinline__ bool arrive_last(unsigned *count, unsigned n)
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    __builtin_amdgcn_s_waitcnt(0);
-    unsigned before = 0;
-    if ((threadIdx.x & 63) == 0)
-        before = __hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    return __builtin_amdgcn_readfirstlane(before) == n - 1;
-}
-
 constexpr int pow2_at_least(int v) { return v <= 1 ? 1 : 2 * pow2_at_least((v + 1) / 2); }
 
 // Dots of one Gram-Schmidt pass: workgroup (x, y) forms the FP64 partials of

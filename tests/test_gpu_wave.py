@@ -1,0 +1,67 @@
+"""The apply without tiles (rp_terms_info kernel RP_APPLY_SMALL) at the edges
+of its range: chains below one wavefront, every slice count, one and four
+amplitudes per lane, and flip masks with one, two and many terms whose
+coefficients are real, imaginary, complex and mixed, with phase bits in the
+lane, the row and the remaining index bits.
+
+Tolerance: FP64 sums of the terms (n of them, each off by at most
+eps64 |c v|) and one rounding to the state's precision."""
+import numpy as np
+import pytest
+
+from conftest import random_state
+from gpu_util import DeviceBuffer, Terms, prec_of
+
+pytestmark = pytest.mark.gpu
+
+
+def _terms(rng, L, masks, fp):
+    """`masks` flip masks with 1, 2, 3, 1, 2, 9, ... terms of every kind."""
+    bits, co = [], []
+    xs = {0} | {int(v) for v in rng.integers(0, 1 << L, masks - 1)}
+    for i, x in enumerate(sorted(xs)):
+        nt = (1, 2, 3, 1, 2, 9)[i % 6]
+        kind = (i // 6) % 4
+        for q in range(nt):
+            z = int(rng.integers(0, 1 << L))
+            b = 0
+            for s in range(L):
+                b |= (x >> s & 1) << (2 * s) | (z >> s & 1) << (2 * s + 1)
+            c = rng.standard_normal() + 1j * rng.standard_normal()
+            c = (c.real, 1j * c.imag, c, c.real if q % 2 else 1j * c.imag)[kind]
+            bits.append(b)
+            co.append(c)
+    co = np.array(co, np.complex128)
+    return np.array(bits, np.uint64), co.astype(np.complex64).astype(np.complex128) if fp == 32 else co
+
+
+@pytest.mark.parametrize("fp,native", [(32, False), (32, True), (64, False)])
+@pytest.mark.parametrize("L,masks", [(1, 2), (2, 4), (5, 9), (6, 30), (7, 40), (9, 120), (12, 300),
+                                     (15, 70), (16, 3), (17, 12), (18, 40), (20, 16)])
+def test_apply_without_tiles(gpu, orc, fp, native, L, masks):
+    rng = np.random.default_rng(1000 * L + masks + fp)
+    dt = np.complex64 if fp == 32 else np.complex128
+    bits, co = _terms(rng, L, masks, fp)
+    psi, prior = random_state(rng, L, dt), random_state(rng, L, dt)
+    ref = orc.apply(L, bits, co, psi.astype(np.complex128), fp=64)
+    t = Terms(L, bits, co, prec_of(dt), gpu.RP_TERMS_ACC_NATIVE if native else 0)
+    info = t.info()
+    assert info.kernel == gpu.RP_APPLY_SMALL and info.tile_bits == 0
+    vin = DeviceBuffer.from_array(psi)
+    depths = [info.depth] + ([1, 8, 32, 128] if L <= 16 else [])
+    # |sum| error: terms times the rounding of the sums, plus the output's
+    eps = 1.2e-7 if native else 2.3e-16
+    tol = len(bits) * eps * np.abs(co).sum() * np.abs(psi).max() + \
+        (6e-8 if fp == 32 else 1.2e-16) * (np.abs(ref).max() + np.abs(prior).max())
+    for d in depths:
+        if d != info.depth:
+            gpu.check(gpu.hip().rp_terms_set_tiling(t.h, 0, 256, d))
+        out = DeviceBuffer.from_array(prior)
+        for acc in (1, 0, 0):      # twice over the same workspace
+            gpu.check(gpu.hip().rp_apply_ops(t.h, out.ptr, vin.ptr, acc))
+            got = out.to_array(dt, len(psi)).astype(np.complex128)
+            want = ref + prior if acc else ref
+            assert np.abs(got - want).max() <= tol, (L, d, acc)
+        out.free()
+    vin.free()
+    t.free()
