@@ -86,10 +86,17 @@ int prof_collect();   // must be called after a stream synchronization
 // blocks of the persistent-style reduction kernels
 constexpr int kRedBlocks = 1024;
 constexpr int kRedThreads = 256;
+// the device workspace: reduction partials and results (kRedBlocks columns of
+// 2 RP_MAX_SWEEP_VECS + 1 doubles and 64 KiB), then the partial rows of the
+// proposer network's gradient
+constexpr size_t kMlpOffset =
+    (size_t)kRedBlocks * (2 * RP_MAX_SWEEP_VECS + 1) * sizeof(double) + 64 * 1024;
+constexpr int kMlpRows = 128, kMlpRowFloats = RP_MLP_NPARAMS + 1;
 // the pinned host buffer: scalars of one call in [0, kHostSteps), then a slot
 // of results for each of the up to 64 queued steps of a Krylov recurrence
 constexpr int kHostSteps = 4096;
 constexpr int kHostSlot = 136;
+constexpr int kHostLoss = kHostSteps + RP_MAX_SWEEP_VECS * kHostSlot;   // the training loss
 
 // Partials that another workgroup of the same launch reads: written through
 // to memory and read past the caches (device-scope accesses), with a wait

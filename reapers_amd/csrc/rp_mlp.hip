@@ -6,15 +6,15 @@
 //   W1[64][12] @ 0, b1[64] @ 768, W2[64][64] @ 832, b2[64] @ 4928,
 //   W3[2][64] @ 4992, b3[2] @ 5120.
 //
-// One 64-wide wavefront evaluates one sample: lane j owns hidden unit j of
-// both layers, so the 64x64 layer is one LDS-broadcast dot product per lane
-// (W2 is staged transposed so that the 64 lanes read 64 consecutive words)
-// and the 2 outputs are wavefront reductions.  The gradient kernel keeps the
-// per-lane slice of the gradient (row j of W1 and W2, b1[j], b2[j], column j
-// of W3) in registers over the wave's samples, sums the 4 waves of a block in
-// LDS and writes one partial row per block; a second kernel adds the block
-// rows in a fixed order, so gradients are bitwise deterministic for a given
-// sample count.
+// Forward: one 64-wide wavefront evaluates one sample: lane j owns hidden unit
+// j of both layers, so the 64x64 layer is one LDS-broadcast dot product per
+// lane (W2 is staged transposed so that the 64 lanes read 64 consecutive
+// words) and the 2 outputs are wavefront reductions.
+//
+// Gradient: a workgroup takes tiles of 64 samples and forms every product of
+// the two passes with the FP32 matrix instructions; it writes one partial row
+// of gradients, and a second kernel adds the rows in a fixed order, so
+// gradients are bitwise deterministic for a given sample count.
 #include "rp_internal.h"
 
 #include <math.h>
@@ -32,14 +32,12 @@ static_assert(kNP == RP_MLP_NPARAMS, "parameter layout");
 static_assert(kHid == 64, "one lane per hidden unit of a 64-wide wavefront");
 
 constexpr int kWaves = 4, kThreads = 64 * kWaves;
-constexpr int kMaxGradBlocks = 32;
+constexpr int kMaxGradBlocks = kMlpRows;
 
 struct Shared {
     float w1t[kIn * kHid];     // w1t[i*64 + j] = W1[j][i]
     float w2t[kHid * kHid];    // w2t[k*64 + j] = W2[j][k]
-    float w2[kHid * kHid];     // W2[j][k]
     float h1[kWaves][kHid];
-    float dz2[kWaves][kHid];
     float x[kWaves][kIn];
 };
 
@@ -49,7 +47,7 @@ __device__ inline float wave_sum(float v)
     return v;
 }
 
-__device__ inline void stage_weights(Shared &sh, const float *__restrict__ p, bool need_w2)
+__device__ inline void stage_weights(Shared &sh, const float *__restrict__ p)
 {
     for (int e = threadIdx.x; e < kHid * kIn; e += kThreads) {
         int j = e / kIn, i = e % kIn;
@@ -57,9 +55,7 @@ __device__ inline void stage_weights(Shared &sh, const float *__restrict__ p, bo
     }
     for (int e = threadIdx.x; e < kHid * kHid; e += kThreads) {
         int j = e / kHid, k = e % kHid;
-        float w = p[oW2 + e];
-        sh.w2t[k * kHid + j] = w;
-        if (need_w2) sh.w2[e] = w;
+        sh.w2t[k * kHid + j] = p[oW2 + e];
     }
 }
 
@@ -86,7 +82,7 @@ __global__ __launch_bounds__(kThreads) void k_mlp_forward(const float *__restric
                                                           float *__restrict__ Y)
 {
     __shared__ Shared sh;
-    stage_weights(sh, p, false);
+    stage_weights(sh, p);
     __syncthreads();
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
     for (long s = (long)blockIdx.x * kWaves + wv; s < n; s += (long)gridDim.x * kWaves) {
@@ -97,99 +93,222 @@ __global__ __launch_bounds__(kThreads) void k_mlp_forward(const float *__restric
     }
 }
 
-// loss = sum_s sum_o w[s,o] (y[s,o] - t[s,o])^2 / n and its gradient
+// Loss and gradient of tiles of 64 samples: loss = sum_s sum_o w[s,o]
+// (y[s,o] - t[s,o])^2 / n.  The layers' products are 16x16x4 FP32 matrix
+// instructions (operand A: lane l holds row l mod 16 at k = l / 16; B: column
+// l mod 16 at k = l / 16; result register r: row 4 (l / 16) + r, column l mod
+// 16), all operands from LDS, whose rows are padded by one word against bank
+// conflicts.  Wavefront w takes the samples 16 w .. 16 w + 15 in the passes
+// and the rows 16 w .. of dW1, dW2 in the sums over samples, which stay in
+// registers over the workgroup's tiles.
+//
+// Bound by latency: 2792 samples are 44 workgroups.  One wavefront per sample
+// with LDS dot products, on 32 workgroups, took 61 us there (22 samples in
+// series, 2.8 us each).
+constexpr int kTile = 64, kPad = kHid + 1, kXPad = 17;
+using f4 = __attribute__((ext_vector_type(4))) float;
+
+// c += A B over K (a multiple of 4); a(row, k), b(k, column) for rows and
+// columns 0..15 of this tile
+template <int K, typename FA, typename FB>
+__device__ __forceinline__ f4 tile_mma(f4 c, int lane, FA &&a, FB &&b)
+{
+#pragma unroll
+    for (int k = 0; k < K; k += 4)
+        c = __builtin_amdgcn_mfma_f32_16x16x4f32(a(lane & 15, k + (lane >> 4)),
+                                                 b(k + (lane >> 4), lane & 15), c, 0, 0, 0);
+    return c;
+}
+
 __global__ __launch_bounds__(kThreads) void k_mlp_grad(const float *__restrict__ p,
                                                        const float *__restrict__ X,
                                                        const float *__restrict__ T,
                                                        const float *__restrict__ W, long n,
                                                        float *__restrict__ part)
 {
-    __shared__ Shared sh;
-    __shared__ float red[kWaves][kHid];
-    stage_weights(sh, p, true);
-    __syncthreads();
-    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    __shared__ float w1[kHid][kXPad], w2[kHid][kPad];     // W1 with zero columns 12..15
+    __shared__ float x[kTile][kXPad], h1[kTile][kPad], dz2[kTile][kPad], dz1[kTile][kPad];
+    __shared__ float red[kWaves][5 * kHid + 4];           // gb1, gb2, gw3[2], loss and gb3
+    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63, col = lane & 15, grp = lane >> 4;
+    for (int e = threadIdx.x; e < kHid * 16; e += kThreads) {
+        const int j = e >> 4, i = e & 15;
+        w1[j][i] = i < kIn ? p[oW1 + j * kIn + i] : 0.f;
+    }
+    for (int e = threadIdx.x; e < kHid * kHid; e += kThreads) w2[e >> 6][e & 63] = p[oW2 + e];
+    float b1[4], b2[4], w3[kOut][4], b3[kOut];
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+        b1[t] = p[oB1 + 16 * t + col];
+        b2[t] = p[oB2 + 16 * t + col];
+        for (int o = 0; o < kOut; o++) w3[o][t] = p[oW3 + o * kHid + 16 * t + col];
+    }
+    for (int o = 0; o < kOut; o++) b3[o] = p[oB3 + o];
     const float inv_n = 1.0f / (float)n;
-    float gw1[kIn], gw2[kHid], gb1 = 0, gb2 = 0, gw3[kOut], gb3 = 0, loss = 0;
-    for (int i = 0; i < kIn; i++) gw1[i] = 0;
-    for (int k = 0; k < kHid; k++) gw2[k] = 0;
-    for (int o = 0; o < kOut; o++) gw3[o] = 0;
-    float w3[kOut];
-    for (int o = 0; o < kOut; o++) w3[o] = p[oW3 + o * kHid + lane];
-    for (long s = (long)blockIdx.x * kWaves + wv; s < n; s += (long)gridDim.x * kWaves) {
-        float h1, h2, y[kOut];
-        wave_forward(sh, wv, lane, p, X + s * kIn, h1, h2, y);
-        float dy[kOut], dh2 = 0;
-        for (int o = 0; o < kOut; o++) {
-            float w = W ? W[s * kOut + o] : 1.0f;
-            float e = y[o] - T[s * kOut + o];
-            loss += w * e * e;
-            dy[o] = 2.0f * w * e * inv_n;
-            gw3[o] += dy[o] * h2;
-            dh2 += w3[o] * dy[o];
-            if (lane == o) gb3 += dy[o];
-        }
-        float dz2 = dh2 * (1.0f - h2 * h2);
-        gb2 += dz2;
-        for (int k = 0; k < kHid; k++) gw2[k] += dz2 * sh.h1[wv][k];
-        sh.dz2[wv][lane] = dz2;
-        __builtin_amdgcn_wave_barrier();
-        float dh1 = 0;
-        for (int j = 0; j < kHid; j++) dh1 += sh.w2[j * kHid + lane] * sh.dz2[wv][j];
-        float dz1 = dh1 * (1.0f - h1 * h1);
-        gb1 += dz1;
-        for (int i = 0; i < kIn; i++) gw1[i] += dz1 * sh.x[wv][i];
-        __builtin_amdgcn_wave_barrier();
+    f4 gw2[4], gw1 = {0, 0, 0, 0};
+    float gb1[4], gb2[4], gw3[kOut][4], gb3[kOut] = {0, 0}, loss = 0;
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+        gw2[t] = f4{0, 0, 0, 0};
+        gb1[t] = gb2[t] = gw3[0][t] = gw3[1][t] = 0;
     }
-    // sum the waves of the block: one parameter group at a time through LDS
+    const long tiles = (n + kTile - 1) / kTile;
+    const int row0 = 16 * wv;
+    for (long tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+        const long s0 = tile * kTile;
+        __syncthreads();     // the last tile's reads are done (first: w1, w2 follow)
+        for (int e = threadIdx.x; e < kTile * 16; e += kThreads) {
+            const int r = e >> 4, i = e & 15;
+            x[r][i] = i < kIn && s0 + r < n ? X[(s0 + r) * kIn + i] : 0.f;
+        }
+        __syncthreads();
+        // forward, layer 1
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            const f4 z = tile_mma<16>(f4{b1[t], b1[t], b1[t], b1[t]}, lane,
+                                      [&](int r, int k) { return x[row0 + r][k]; },
+                                      [&](int k, int c) { return w1[16 * t + c][k]; });
+#pragma unroll
+            for (int r = 0; r < 4; r++) h1[row0 + 4 * grp + r][16 * t + col] = tanhf(z[r]);
+        }
+        // (a wavefront reads only its own rows of h1 until the sums below)
+        __builtin_amdgcn_wave_barrier();
+        // layer 2 and the outputs; the 16 lanes of a group hold 4 samples
+        float h2[4][4], y[kOut][4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) y[0][r] = y[1][r] = 0;
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            const f4 z = tile_mma<kHid>(f4{b2[t], b2[t], b2[t], b2[t]}, lane,
+                                        [&](int r, int k) { return h1[row0 + r][k]; },
+                                        [&](int k, int c) { return w2[16 * t + c][k]; });
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                h2[t][r] = tanhf(z[r]);
+                y[0][r] += w3[0][t] * h2[t][r];
+                y[1][r] += w3[1][t] * h2[t][r];
+            }
+        }
+        float dy[kOut][4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const long smp = s0 + row0 + 4 * grp + r;
+#pragma unroll
+            for (int o = 0; o < kOut; o++) {
+                float v = y[o][r];
+                for (int off = 8; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+                float d = 0;
+                if (smp < n) {
+                    const float w = W ? W[smp * kOut + o] : 1.0f;
+                    const float e = v + b3[o] - T[smp * kOut + o];
+                    d = 2.0f * w * e * inv_n;
+                    if (col == 0) {
+                        loss += w * e * e;
+                        gb3[o] += d;
+                    }
+                }
+                dy[o][r] = d;
+            }
+        }
+        // backward, layer 2
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const float h = h2[t][r];
+                const float d = (w3[0][t] * dy[0][r] + w3[1][t] * dy[1][r]) * (1.0f - h * h);
+                gw3[0][t] += dy[0][r] * h;
+                gw3[1][t] += dy[1][r] * h;
+                gb2[t] += d;
+                dz2[row0 + 4 * grp + r][16 * t + col] = d;
+            }
+        __builtin_amdgcn_wave_barrier();
+        // layer 1
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            const f4 d = tile_mma<kHid>(f4{0, 0, 0, 0}, lane,
+                                        [&](int r, int k) { return dz2[row0 + r][k]; },
+                                        [&](int k, int c) { return w2[k][16 * t + c]; });
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const float h = h1[row0 + 4 * grp + r][16 * t + col];
+                const float v = d[r] * (1.0f - h * h);
+                gb1[t] += v;
+                dz1[row0 + 4 * grp + r][16 * t + col] = v;
+            }
+        }
+        __syncthreads();
+        // the sums over the tile's samples
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+            gw2[t] = tile_mma<kTile>(gw2[t], lane, [&](int r, int k) { return dz2[k][row0 + r]; },
+                                     [&](int k, int c) { return h1[k][16 * t + c]; });
+        gw1 = tile_mma<kTile>(gw1, lane, [&](int r, int k) { return dz1[k][row0 + r]; },
+                              [&](int k, int c) { return x[k][c]; });
+    }
     float *row = part + (size_t)blockIdx.x * (kNP + 1);
-    auto block_sum = [&](float v, int dst_index) {
-        red[wv][lane] = v;
-        __syncthreads();
-        if (wv == 0) {
-            float a = red[0][lane];
-            for (int q = 1; q < kWaves; q++) a += red[q][lane];
-            row[dst_index] = a;
-        }
-        __syncthreads();
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+            row[oW2 + (row0 + 4 * grp + r) * kHid + 16 * t + col] = gw2[t][r];
+    if (col < kIn)
+#pragma unroll
+        for (int r = 0; r < 4; r++) row[oW1 + (row0 + 4 * grp + r) * kIn + col] = gw1[r];
+    // per-unit sums: over the four groups of lanes, then the wavefronts
+    auto groups = [](float v) {
+        v += __shfl_xor(v, 16, 64);
+        return v + __shfl_xor(v, 32, 64);
     };
-    for (int i = 0; i < kIn; i++) block_sum(gw1[i], oW1 + lane * kIn + i);
-    block_sum(gb1, oB1 + lane);
-    for (int k = 0; k < kHid; k++) block_sum(gw2[k], oW2 + lane * kHid + k);
-    block_sum(gb2, oB2 + lane);
-    for (int o = 0; o < kOut; o++) block_sum(gw3[o], oW3 + o * kHid + lane);
-    // b3 lives in lane o of each wave
-    red[wv][lane] = gb3;
-    __syncthreads();
-    if (threadIdx.x < kOut) {
-        float a = red[0][threadIdx.x];
-        for (int q = 1; q < kWaves; q++) a += red[q][threadIdx.x];
-        row[oB3 + threadIdx.x] = a;
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+        const float a = groups(gb1[t]), b = groups(gb2[t]), c = groups(gw3[0][t]),
+                    d = groups(gw3[1][t]);
+        if (grp == 0) {
+            float *q = red[wv] + 16 * t + col;
+            q[0] = a;
+            q[kHid] = b;
+            q[2 * kHid] = c;
+            q[3 * kHid] = d;
+        }
+    }
+    const float l = groups(loss), g0 = groups(gb3[0]), g1 = groups(gb3[1]);
+    if (lane == 0) {
+        red[wv][4 * kHid] = g0;
+        red[wv][4 * kHid + 1] = g1;
+        red[wv][4 * kHid + 2] = l;
     }
     __syncthreads();
-    loss = __shfl(loss, 0, 64);   // every lane holds the same loss sum
-    red[wv][lane] = loss;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        float a = red[0][0];
-        for (int q = 1; q < kWaves; q++) a += red[q][0];
-        row[kNP] = a;
+    for (int e = threadIdx.x; e < 4 * kHid + 3; e += kThreads) {
+        float a = red[0][e];
+        for (int q = 1; q < kWaves; q++) a += red[q][e];
+        row[e < kHid ? oB1 + e : e < 2 * kHid ? oB2 + e - kHid : e < 4 * kHid ? oW3 + e - 2 * kHid
+            : e < 4 * kHid + 2 ? oB3 + e - 4 * kHid : kNP] = a;
     }
 }
 
-// out[e] = sum over blocks b (in order) of part[b][e]; the loss sums, at
-// index kNP of each row, go to loss_out divided by n
-__global__ void k_mlp_reduce(const float *__restrict__ part, int nb, float *__restrict__ out,
-                             double *__restrict__ loss_out, long n)
+// out[e] = sum over blocks b of part[b][e], each of a workgroup's kRedRows
+// groups of threads every kRedRows-th row, then the groups in order; the loss
+// sums, at index kNP of each row, go to loss_out divided by n
+constexpr int kRedRows = 8, kRedCols = 32;
+__global__ __launch_bounds__(kRedRows *kRedCols) void k_mlp_reduce(
+    const float *__restrict__ part, int nb, float *__restrict__ out, double *__restrict__ loss_out,
+    long n)
 {
-    for (int e = blockIdx.x * blockDim.x + threadIdx.x; e <= kNP; e += gridDim.x * blockDim.x) {
-        float a = 0;
-        for (int b = 0; b < nb; b++) a += part[(size_t)b * (kNP + 1) + e];
-        if (e < kNP)
-            out[e] = a;
-        else
-            loss_out[0] = (double)a / (double)n;
-    }
+    __shared__ float sh[kRedRows][kRedCols];
+    const int c = threadIdx.x % kRedCols, g = threadIdx.x / kRedCols;
+    const int e = blockIdx.x * kRedCols + c;
+    float a = 0;
+    if (e <= kNP)
+#pragma unroll 8
+        for (int b = g; b < nb; b += kRedRows) a += part[(size_t)b * (kNP + 1) + e];
+    sh[g][c] = a;
+    __syncthreads();
+    if (g || e > kNP) return;
+    for (int q = 1; q < kRedRows; q++) a += sh[q][c];
+    if (e < kNP)
+        out[e] = a;
+    else
+        loss_out[0] = (double)a / (double)n;
 }
 
 __global__ void k_mlp_adam(float *__restrict__ p, const float *__restrict__ g,
@@ -208,7 +327,7 @@ __global__ void k_mlp_adam(float *__restrict__ p, const float *__restrict__ g,
     }
 }
 
-int grad_blocks(long n) { return (int)std::min<long>(kMaxGradBlocks, (n + kWaves - 1) / kWaves); }
+int grad_blocks(long n) { return (int)std::min<long>(kMaxGradBlocks, (n + kTile - 1) / kTile); }
 
 }  // namespace
 }  // namespace rp
@@ -238,24 +357,22 @@ int rp_mlp_loss_grad(const float *params, const float *X, const float *T, const 
     RP_REQUIRE(params && X && T && grad, "null argument");
     Context &c = ctx();
     const int nb = grad_blocks((long)n);
-    float *part = (float *)c.work;
-    double *dloss = (double *)((char *)c.work + c.work_bytes - 64 * 1024);
-    static_assert(kMaxGradBlocks * (kNP + 1) * sizeof(float) + 64 * 1024 <=
-                      (size_t)kRedBlocks * (2 * 64 + 1) * sizeof(double) + 64 * 1024,
-                  "gradient partials fit the workspace");
+    float *part = (float *)((char *)c.work + kMlpOffset);
+    static_assert(kMlpRowFloats == kNP + 1, "gradient partial rows");
     RP_LAUNCH(RP_KERNEL_OTHER, k_mlp_grad, dim3(nb), dim3(kThreads), 0, params, X, T, W,
               (long)n, part);
-    RP_LAUNCH(RP_KERNEL_OTHER, k_mlp_reduce, dim3(21), dim3(256), 0, (const float *)part, nb,
-              grad, dloss, (long)n);
+    // the loss straight to pinned memory, in a place of its own: without a
+    // wait (loss null) it may still be written while others use the buffer
+    double *host_loss = c.pinned + kHostLoss;
+    RP_LAUNCH(RP_KERNEL_OTHER, k_mlp_reduce, dim3(kNP / kRedCols + 1), dim3(kRedRows * kRedCols), 0,
+              (const float *)part, nb, grad, host_loss, (long)n);
     if (loss) {
-        RP_CHECK_HIP(hipMemcpyAsync(c.pinned, dloss, sizeof(double), hipMemcpyDeviceToHost,
-                                    c.stream));
         RP_CHECK_HIP(hipStreamSynchronize(c.stream));
         if (c.prof) {
             st = prof_collect();
             if (st) return st;
         }
-        *loss = c.pinned[0];
+        *loss = *host_loss;
     }
     return RP_OK;
 }
@@ -286,7 +403,7 @@ int rp_mlp_infer(const float *params, const float *x_host, int n, float *y_host)
     // staging: inputs and outputs in the pinned buffer and in the tail of the
     // workspace (stream order keeps them apart from reduction partials)
     float *hin = (float *)c.pinned, *hout = hin + RP_MLP_MAX_INFER * kIn;
-    float *din = (float *)((char *)c.work + c.work_bytes - 32 * 1024);
+    float *din = (float *)((char *)c.work + kMlpOffset - 32 * 1024);
     float *dout = din + RP_MLP_MAX_INFER * kIn;
     // the previous user of the pinned buffer has completed: every entry point
     // that fills it synchronizes before returning

@@ -109,11 +109,9 @@ int rp_init(int device)
     c.name = prop.gcnArchName;
     // default-priority stream, not synchronizing with the legacy null stream
     RP_CHECK_HIP(hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking));
-    // partials for up to 64 complex FP64 values and one norm per reduction
-    // block, plus room for the reduced results
-    c.work_bytes = (size_t)kRedBlocks * (2 * 64 + 1) * sizeof(double) + 64 * 1024;
+    c.work_bytes = kMlpOffset + (size_t)kMlpRows * kMlpRowFloats * sizeof(float);
     RP_CHECK_HIP(dev_malloc(&c.work, c.work_bytes));
-    c.pinned_doubles = kHostSteps + RP_MAX_SWEEP_VECS * kHostSlot;
+    c.pinned_doubles = kHostLoss + 8;
     RP_CHECK_HIP(hipHostMalloc((void **)&c.pinned, c.pinned_doubles * sizeof(double),
                                hipHostMallocDefault));
     int st = vec_scratch_setup(device);
