@@ -223,11 +223,11 @@ class Krylov {
             dense::CMat tH = Hfull;
             const cd z{-t_imag, -t_real};
             for (auto &v : tH.a) v *= z;
-            dense::CMat E = dense::expm(tH);
+            const std::vector<cd> E = dense::expm_col0(tH);
             std::vector<cd> c(m);
             double nrm2 = 0;
             for (int i = 0; i < m; i++) {
-                cd e = E(off + i, 0);
+                cd e = E[off + i];
                 c[i] = beta0 * e;
                 nrm2 += std::norm(e);
             }

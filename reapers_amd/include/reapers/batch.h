@@ -280,10 +280,10 @@ private:
                             i == j + 1 ? cd(Hget(r, i, j).real()) : i <= j ? Hget(r, i, j) : 0.0;
                 dense::CMat tH = F;
                 for (auto &v : tH.a) v *= z;
-                dense::CMat E = dense::expm(tH);
+                const std::vector<cd> E = dense::expm_col0(tH);
                 double nrm2 = 0;
                 for (int i = 0; i < mr; i++) {
-                    cd e = E(off_blk + i, 0);
+                    cd e = E[off_blk + i];
                     cd c = beta0[r] * e;
                     ch[(size_t)2 * kmax * r + 2 * i] = c.real();
                     ch[(size_t)2 * kmax * r + 2 * i + 1] = c.imag();
