@@ -108,7 +108,7 @@ template <typename A> struct alignas(16) SubW { uint64_t l0, l1; A c0, c1; uint3
 enum : uint32_t { kWaveImag = 1, kWaveRow = 2, kWaveTwo = 4, kWaveMulti = 8 };
 template <typename A> struct TermW { uint64_t lanes; A c; uint32_t z, pad; };
 
-constexpr int kWaveMaxLen = 18, kWaveMaxFlips = 40;
+constexpr int kWaveMaxLen = 19, kWaveMaxFlips = 40;
 constexpr int kWavePad = 16;       // flip masks read past the end of the list
 
 // c with the sign of (-1)^popcount(v), v uniform
@@ -189,7 +189,8 @@ __device__ __forceinline__ void add_rows(const A (&d)[ROWS], const T (&v)[ROWS],
 
 // W wavefronts per workgroup: with one slice each its own amplitudes, else
 // slices of the same ones
-template <typename R, typename A, int ROWS, int W>
+// BIG: states of 4 GiB and more, whose gathers need 64-bit offsets
+template <typename R, typename A, int ROWS, int W, bool BIG>
 __global__ void __launch_bounds__(64 * W)
 k_apply_wave(const typename CxA<R>::T *__restrict__ in, typename CxA<R>::T *__restrict__ out,
              uint64_t dim, const uint32_t *__restrict__ flips, const SubW<A> *__restrict__ subs,
@@ -216,12 +217,18 @@ k_apply_wave(const typename CxA<R>::T *__restrict__ in, typename CxA<R>::T *__re
     for (int r = 0; r < ROWS; r++) { ar[r] = 0; ai[r] = 0; }
     const uint32_t s0 = cut[slice], s1 = cut[slice + 1];
 
+    // byte offset of the lane's amplitude in row 0; a flip mask and a row
+    // change bits of it: one scalar and one vector instruction per gather
+    const uint32_t own = (m0 | ll) * (uint32_t)sizeof(T);
     auto gather = [&](const uint32_t (&x)[U], T (&v)[U][ROWS]) __attribute__((always_inline)) {
 #pragma unroll
         for (int u = 0; u < U; u++)
 #pragma unroll
-            for (int r = 0; r < ROWS; r++)
-                v[u][r] = (in + ((m0 | (r * 64)) ^ (x[u] & ~63u)))[ll ^ (x[u] & 63u)];
+            for (int r = 0; r < ROWS; r++) {
+                const uint32_t f = x[u] ^ (uint32_t)(r * 64);
+                if constexpr (BIG) v[u][r] = in[(uint64_t)((m0 | ll) ^ f)];
+                else v[u][r] = *(const T *)((const char *)in + (own ^ f * (uint32_t)sizeof(T)));
+            }
     };
     auto load_flips = [&](uint32_t s, uint32_t (&x)[U]) __attribute__((always_inline)) {
 #pragma unroll
@@ -291,16 +298,18 @@ k_apply_wave(const typename CxA<R>::T *__restrict__ in, typename CxA<R>::T *__re
             sh[2 * r + 1][wid][lane] = ai[r];
         }
         __syncthreads();
+        for (uint32_t i = threadIdx.x; i < 128 * ROWS; i += 64 * W) {
+            A *q = &sh[i >> 6][0][i & 63], a = q[0];
+#pragma unroll
+            for (int w = 1; w < W; w++) a += q[w * 64];
+            q[0] = a;
+        }
+        __syncthreads();
         if (wid) return;
 #pragma unroll
         for (int r = 0; r < ROWS; r++) {
             ar[r] = sh[2 * r][0][lane];
             ai[r] = sh[2 * r + 1][0][lane];
-#pragma unroll
-            for (int w = 1; w < W; w++) {
-                ar[r] += sh[2 * r][w][lane];
-                ai[r] += sh[2 * r + 1][w][lane];
-            }
         }
         const uint32_t nw = gridDim.y;
         if constexpr (W == 16) {
@@ -1155,7 +1164,7 @@ static int wave_depth(int len, uint64_t flips, uint64_t nterms)
     const uint64_t chunks = len > 6 ? 1ull << (len - 6) : 1;
     int d = 1;
     for (int s : {8, 32, 128})
-        if (chunks * s <= (s == 8 ? 32768 : 8192) && flips >= (uint64_t)s &&
+        if (chunks * s <= (s == 8 ? 65536 : 8192) && flips >= (uint64_t)s &&
             6 * flips + nterms >= (uint64_t)(24 * s))
             d = s;
     return d;
@@ -1169,9 +1178,11 @@ static void choose_tiling(int prec, int len, uint64_t flips, uint64_t nterms, in
     // No tiles for short chains, nor for few flip masks with several terms
     // each, whose sums the tiled kernel forms for every row.  us per apply
     // without tiles / with (12, 512, 2), FP64 sums, default upload:
-    //   sparse SYK, k = 8, complex<float>:  16 sites 19 / 93, 18 sites 48 / 110
-    //   XXZ with fields (4 terms a mask):   20 sites 21 / 40, 24 sites 241 / 431,
-    //     26 sites 1072 / 1814, complex<double> 24 sites 392 / 728
+    //   sparse SYK, k = 8, complex<float>:  16 sites 17 / 93, 18 sites 41 / 110,
+    //     19 sites 80 / 136 (group accumulation 80 / 87), 20 sites 154 / 153,
+    //     21 sites 321 / 210; complex<double> 19 sites 92 / 137, 20 191 / 160
+    //   XXZ with fields (4 terms a mask):   20 sites 21 / 40, 24 sites 209 / 431,
+    //     26 sites 1072 / 1814, complex<double> 24 sites 388 / 728
     //   XY chain (2 a mask):                20 sites 16 / 28, 24 sites 196 / 297
     //   transverse Ising (under 2):         22 sites 54 / 60, 24 sites 205 / 204
     //   one a mask, 20 masks:               22 sites 54 / 50, 24 sites 249 / 189
@@ -1455,16 +1466,18 @@ static int apply_impl(rp_terms *h, void *res, const void *vec, int accumulate, c
         const dim3 grid = h->depth == 1 ? dim3((unsigned)((chunks + w - 1) / w))
                                         : dim3((unsigned)chunks, h->depth / w);
         unsigned *count = (unsigned *)((char *)h->d_split + wave_part_bytes(h));
-#define RP_WAVE(ROWS, W)                                                          \
-    RP_LAUNCH(RP_KERNEL_APPLY, (k_apply_wave<R, A, ROWS, W>), grid, dim3(64 * W), 0,              \
+        const bool big = dim * sizeof(T) >= (1ull << 32);
+#define RP_WAVE(ROWS, W, BIG)                                                     \
+    RP_LAUNCH(RP_KERNEL_APPLY, (k_apply_wave<R, A, ROWS, W, BIG>), grid, dim3(64 * W), 0,         \
               (const T *)vec, (T *)res, dim, (const uint32_t *)h->d_wflips,                      \
               (const SubW<A> *)h->d_wsubs, (const TermW<A> *)h->d_wterms,                        \
               (const uint32_t *)h->d_wcut, h->depth, accumulate, (double *)h->d_split, count, stop)
-        if (w == 16) RP_WAVE(1, 16);
-        else if (w == 8 && h->rows == 1) RP_WAVE(1, 8);
-        else if (w == 8) RP_WAVE(4, 8);
-        else if (h->rows == 1) RP_WAVE(1, 4);
-        else RP_WAVE(4, 4);
+        if (w == 16) RP_WAVE(1, 16, false);
+        else if (w == 8 && h->rows == 1) RP_WAVE(1, 8, false);
+        else if (w == 8) RP_WAVE(4, 8, false);
+        else if (h->rows == 1) RP_WAVE(1, 4, false);
+        else if (!big) RP_WAVE(4, 4, false);
+        else RP_WAVE(4, 4, true);
 #undef RP_WAVE
         return RP_OK;
     }

@@ -40,16 +40,19 @@ constexpr int kWaves = kRedThreads / 64;
 struct VecPtrs { const void *p[kMaxVecs]; };
 struct Coefs { double c[2 * kMaxVecs]; };
 
-// Workspace of the reductions (doubles): the partials, up to kDotBlocks for
-// each of 2 kMaxVecs + 1 columns (kRedBlocks are reserved), then the results of the pass in flight:
+// Workspace of the reductions (doubles): the partials, kDotCols for each of up
+// to kDotBlocks workgroups of each row of vectors (kRedBlocks x 2 kMaxVecs + 1
+// are reserved), then the results of the pass in flight:
 //   [0, 2k) coefficients h; kResNorm (host only) the norm after the pass when
 //   it was not fused; kResIn ||w||^2 before it; kResBeta the fused norm (0: not
 //   fused); kResStop (an int) set by an Arnoldi step that needs the host;
-//   kResCount arrival counters of the dot workgroups, zero between launches.
+//   kResCount arrival counters of the dot workgroups, zero between launches
+//   (for each row of workgroups one, and 16 below it, 64 bytes apart).
 // The pinned host copy that the kernels write has the layout up to kResStop.
 constexpr int kResNorm = 2 * kMaxVecs, kResIn = kResNorm + 1, kResBeta = kResNorm + 2,
               kResStop = kResNorm + 4, kResCount = kResNorm + 8;
-constexpr int kResDoubles = kResCount + kMaxVecs / 2;
+constexpr int kDotRows = 16, kCountStep = 8;      // counters: doubles apart
+constexpr int kResDoubles = kResCount + kDotRows * 17 * kCountStep;
 static_assert(kResBeta < kHostSlot && (size_t)kResDoubles * sizeof(double) < 32 * 1024,
               "result slots");
 
@@ -244,8 +247,11 @@ constexpr int pow2_at_least(int v) { return v <= 1 ? 1 : 2 * pow2_at_least((v + 
 // pass), the recursive halving the shuffles of the workgroup's reduction.
 // At most kDotBlocks workgroups a row, so that every thread of the last one
 // has all its partials in flight at once (past the caches each read takes
-// about 1 us); from 2^16 elements they have 1024 threads.
-constexpr int kDotBlocks = 256;
+// about 1 us); from 2^19 elements they have 1024 threads.
+constexpr int kDotBlocks = 256, kDotCols = 24;
+static_assert(2 * kDotChunk + 1 <= kDotCols &&
+                  kDotRows * kDotBlocks * kDotCols <= kRedBlocks * (2 * kMaxVecs + 1),
+              "dot partials");
 template <typename R, int KC, int NT>
 __global__ void __launch_bounds__(NT)
 k_gs_dots(VecPtrs V, int k, const typename Cx<R>::T *__restrict__ w, uint64_t n,
@@ -289,9 +295,9 @@ k_gs_dots(VecPtrs V, int k, const typename Cx<R>::T *__restrict__ w, uint64_t n,
         if (lane == 0) sh[wid][NV] = wn;
     }
     __syncthreads();
-    // columns of this row: 2 per vector, and ||w||^2 (column kResNorm)
+    // columns of this row: 2 per vector, and ||w||^2
     const int nv = KC ? 2 * min(KC, k - q0) : 0, ncol = nv + (y == 0 ? 1 : 0);
-    auto column = [&](int c) { return part + (size_t)(c < nv ? 2 * q0 + c : kResNorm) * kDotBlocks; };
+    double *rows = part + (size_t)y * kDotBlocks * kDotCols;
     auto store = [&](int c, double v) {
         const int at = c < nv ? 2 * q0 + c : kResIn;
         if (real && c < nv && (c & 1)) v = 0.0;
@@ -305,31 +311,46 @@ k_gs_dots(VecPtrs V, int k, const typename Cx<R>::T *__restrict__ w, uint64_t n,
 #pragma unroll
             for (int q = 0; q < W; q++) v += sh[q][c];
             if (nb == 1) store(lane, v);
-            else put_shared(column(lane) + blockIdx.x, v);
+            else put_shared(rows + blockIdx.x * kDotCols + lane, v);
         }
         if (nb > 1) {
-            const bool l = arrive_last((unsigned *)(res + kResCount) + y, (unsigned)nb);
+            // Arrivals at one counter are served one after the other (256 of
+            // them took 15 us): 16 counters, whose last arrivals meet at one
+            double *cnt = res + kResCount + (size_t)y * 17 * kCountStep;
+            const unsigned sub = blockIdx.x & 15u, subs = min(nb, 16);
+            unsigned *leaf = (unsigned *)(cnt + (1 + sub) * kCountStep);
+            bool l = arrive_last(leaf, ((unsigned)nb - sub + 15u) / 16u);
+            if (l) {
+                if (lane == 0) *leaf = 0;
+                l = arrive_last((unsigned *)cnt, subs);
+            }
             if (lane == 0) last = l;
         }
     }
     if (nb == 1) return;
     __syncthreads();
     if (!last) return;
-    // G threads per column (32 column slots for at most 17 columns)
+    // thread (g, c): column c of every (NT / 32)-th workgroup's partials
     constexpr int G = NT / 32, PER = kDotBlocks / G;
-    const int c = threadIdx.x / G, g = threadIdx.x % G;
+    __shared__ double sums[G][kDotCols];
+    const int c = threadIdx.x & 31, g = threadIdx.x >> 5;
     if (c < ncol) {
-        const double *col = column(c);
         double p[PER], v = 0;
 #pragma unroll
-        for (int i = 0; i < PER; i++) p[i] = g + i * G < nb ? get_shared(col + g + i * G) : 0.0;
+        for (int i = 0; i < PER; i++)
+            p[i] = g + i * G < nb ? get_shared(rows + (g + i * G) * kDotCols + c) : 0.0;
 #pragma unroll
         for (int i = 0; i < PER; i++) v += p[i];
-#pragma unroll
-        for (int off = G / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-        if (g == 0) store(c, v);
+        sums[g][c] = v;
     }
-    if (threadIdx.x == 0) ((unsigned *)(res + kResCount))[y] = 0;
+    __syncthreads();
+    if ((int)threadIdx.x < ncol) {
+        double v = 0;
+#pragma unroll
+        for (int i = 0; i < G; i++) v += sums[i][threadIdx.x];
+        store(threadIdx.x, v);
+    }
+    if (threadIdx.x == 0) *(unsigned *)(res + kResCount + (size_t)y * 17 * kCountStep) = 0;
 }
 
 // sum over q of h_q x_q for the KC vectors from p on, added to (yr, yi) or
@@ -559,7 +580,7 @@ static int dots_launch(int cls, const VecPtrs &P, int k, const void *w, uint64_t
     const int most = n <= (1u << 15) ? kDotChunk / 2 : kDotChunk;
     const int rows = k > 0 ? (k + most - 1) / most : 1;
     const int kc = (k + rows - 1) / rows;
-    const int nt = n <= (1u << 16) ? 256 : 1024;
+    const int nt = n <= (1u << 19) ? 256 : 1024;
     const dim3 grid((unsigned)std::min<uint64_t>((n + nt - 1) / nt, kDotBlocks), rows);
     double *res = work + kPartDoubles;
 #define RP_DOTS(KC)                                                               \
