@@ -775,8 +775,10 @@ k_apply_tiled(const typename CxA<R>::T *__restrict__ in, typename CxA<R>::T *__r
 // row flip (uniform) to a code path whose LDS row reads are immediate
 // offsets from one lane address.
 // ---------------------------------------------------------------------------
+// xl: bytes that the flip moves the lane by (bits 0..15), the row flip (16..)
+// and the phase bits among the row bits (24..)
 struct SubC { uint32_t xl, z; float c0, c1; };
-struct TermC { uint32_t z; float cr, ci; uint32_t pad; };
+struct TermC { uint32_t z; float cr, ci; uint32_t zr; };
 // group header: tile index above the tile bits, first sub, subs per class
 // run (kRunReal0 .. kRunMulti)
 struct GroupC { uint32_t xh, begin; uint8_t n[kRuns]; uint8_t pad[8 - kRuns]; };
@@ -817,38 +819,41 @@ __device__ __forceinline__ void with_row_flip(uint32_t xr, F &&f)
 
 // all RP row values of a sub loaded before any is used: the reads go out
 // back to back and one wait covers them
-template <int RP> __device__ __forceinline__ void pin_rows(float2 (&v)[RP])
+template <int PR> __device__ __forceinline__ void pin_rows(float4 (&v)[PR])
 {
-    if constexpr (RP == 8)
-        asm volatile("" : "+v"(v[0].x), "+v"(v[0].y), "+v"(v[1].x), "+v"(v[1].y), "+v"(v[2].x),
-                     "+v"(v[2].y), "+v"(v[3].x), "+v"(v[3].y), "+v"(v[4].x), "+v"(v[4].y),
-                     "+v"(v[5].x), "+v"(v[5].y), "+v"(v[6].x), "+v"(v[6].y), "+v"(v[7].x),
-                     "+v"(v[7].y));
-    else if constexpr (RP == 4)
-        asm volatile("" : "+v"(v[0].x), "+v"(v[0].y), "+v"(v[1].x), "+v"(v[1].y), "+v"(v[2].x),
-                     "+v"(v[2].y), "+v"(v[3].x), "+v"(v[3].y));
-    else if constexpr (RP == 2)
-        asm volatile("" : "+v"(v[0].x), "+v"(v[0].y), "+v"(v[1].x), "+v"(v[1].y));
-    else
-        asm volatile("" : "+v"(v[0].x), "+v"(v[0].y));
+#pragma unroll
+    for (int i = 0; i + 1 < PR; i += 2)
+        asm volatile("" : "+v"(v[i].x), "+v"(v[i].y), "+v"(v[i].z), "+v"(v[i].w), "+v"(v[i + 1].x),
+                     "+v"(v[i + 1].y), "+v"(v[i + 1].z), "+v"(v[i + 1].w));
+    if constexpr (PR & 1)
+        asm volatile("" : "+v"(v[PR - 1].x), "+v"(v[PR - 1].y), "+v"(v[PR - 1].z), "+v"(v[PR - 1].w));
 }
 
-// One single-term sub with the row flip XR fixed: input row j of the
-// lane's column (row base `row`, immediate offsets) feeds output row
-// j ^ XR.  c (and ci for the complex class) carry the lane's phase sign; zr
-// = the phase bits among the row bits (classes 1 and complex).
+// The rows of a thread in the streamed kernel: amplitude r = 2 p + h of
+// thread tid is element p 2 NT + 2 tid + h of the tile.  Neighbouring pairs
+// make every LDS read 16 bytes wide: ds_read_b128 delivers 212 bytes per
+// clock and CU, ds_read2st64_b64 120.  Flip masks and phase masks in these
+// terms: bits 1 .. log2 NT move the lane, bit 0 and the top log2 (RP / 2)
+// bits the row.
+static inline uint32_t stream_row(uint32_t v, int tb, int nt)
+{
+    return (v & 1u) | (((v & ((1u << tb) - 1)) / (2u * (unsigned)nt)) << 1);
+}
+
+// One single-term sub with the row flip XR fixed: input amplitude j of the
+// lane feeds output amplitude j ^ XR.  c (and ci for the complex class) carry
+// the lane's phase sign; zr = the phase bits among the row bits (classes 1
+// and complex).
 template <int RP, int NT, uint32_t CLS, int XR>
-__device__ __forceinline__ void sub_rows(const float2 *row, float c, float ci, uint32_t zr,
+__device__ __forceinline__ void sub_rows(float4 (&vv)[RP / 2], float c, float ci, uint32_t zr,
                                          float (&gr)[RP], float (&gi)[RP])
 {
-    float2 vv[RP];
-#pragma unroll
-    for (int j = 0; j < RP; j++) vv[j] = row[j * NT];
-    pin_rows<RP>(vv);
+    pin_rows<RP / 2>(vv);
 #pragma unroll
     for (int j = 0; j < RP; j++) {
         const int r = j ^ XR;
-        const float2 v = vv[j];
+        const float4 q = vv[j / 2];
+        const float2 v = (j & 1) ? float2{q.z, q.w} : float2{q.x, q.y};
         // explicit fused multiply-adds: one rounding each, and no product
         // that the compiler could share between the row-flip paths
         if constexpr (CLS == kRunReal0) {
@@ -881,32 +886,41 @@ __device__ __forceinline__ void sub_rows(const float2 *row, float c, float ci, u
 // term list.  S is the record at s on entry and at end on exit.
 template <int TB, int NT, uint32_t CLS>
 __device__ __forceinline__ void stream_run(uint32_t &s, uint32_t end, SubC &S,
-                                           const SubC *__restrict__ subs, const float2 *buf,
-                                           uint32_t lane8, uint32_t lanebits,
+                                           const SubC *__restrict__ subs, const float4 *buf,
+                                           uint32_t lane16, uint32_t lanebits,
                                            const TermC *__restrict__ terms,
                                            float (&gr)[(1 << TB) / NT], float (&gi)[(1 << TB) / NT])
 {
-    using T = float2;
     constexpr int RP = (1 << TB) / NT;
-    constexpr int LB = NT == 1024 ? 10 : NT == 512 ? 9 : NT == 256 ? 8 : 7;
     for (; s < end; s++) {
         const SubC Sn = subs[s + 1];     // the list has one sentinel record
-        const T *row = sub_lane_base<T, NT>(buf, lane8, S.xl);
-        const uint32_t xr = S.xl >> LB;
+        // the lane's address: one xor, kept opaque, so that each row is an
+        // immediate offset from it
+        uint32_t la = lane16 ^ (S.xl & 0xffffu);
+        asm volatile("" : "+v"(la));
+        const float4 *row = (const float4 *)((const char *)buf + la);
+        const uint32_t xr = (S.xl >> 16) & (RP - 1);
         if constexpr (CLS != kRunMulti) {
+            // the reads go out first: the sign and the branch on the row flip
+            // run while they are under way
+            float4 vv[RP / 2];
+#pragma unroll
+            for (int p = 0; p < RP / 2; p++) vv[p] = row[p * NT];
+            asm volatile("" ::: "memory");
             const uint32_t lsb = parity_sign(lanebits & S.z);
-            const uint32_t zr = (S.z >> LB) & (RP - 1);
+            const uint32_t zr = S.xl >> 24;
             float c = flip_sign(S.c0, lsb), ci = 0.f;
             // a lane-signed coefficient that each row flips again stays in a
             // register (one xor per row instead of the popcount per row)
             if constexpr (CLS == kRunReal1 || CLS == kRunImag1 || CLS == kRunCplx) c = opaque(c);
             if constexpr (CLS == kRunCplx) ci = opaque(flip_sign(S.c1, lsb));
             with_row_flip<RP>(xr, [&](auto X) {
-                sub_rows<RP, NT, CLS, decltype(X)::value>(row, c, ci, zr, gr, gi);
+                sub_rows<RP, NT, CLS, decltype(X)::value>(vv, c, ci, zr, gr, gi);
             });
         } else {
-            constexpr int RC = RP < 4 ? RP : 4;
             const uint32_t tb = S.z, te = __float_as_uint(S.c0);
+            // d(m) = sum_t c_t (-1)^popcount(m & z_t), two pairs at a time
+            constexpr int RC = RP < 4 ? RP : 4;
 #pragma unroll
             for (int r0 = 0; r0 < RP; r0 += RC) {
                 float dr[RC], di[RC];
@@ -916,17 +930,17 @@ __device__ __forceinline__ void stream_run(uint32_t &s, uint32_t end, SubC &S,
                     const TermC C = terms[t];
                     const uint32_t lsb = parity_sign(lanebits & C.z);
                     const float cr = flip_sign(C.cr, lsb), ci = flip_sign(C.ci, lsb);
-                    const uint32_t zr = (C.z >> LB) & (RP - 1);
 #pragma unroll
                     for (int q = 0; q < RC; q++) {
-                        const uint32_t rsb = parity_sign((r0 + q) & zr);
+                        const uint32_t rsb = parity_sign((r0 + q) & C.zr);
                         dr[q] += flip_sign(cr, rsb);
                         di[q] += flip_sign(ci, rsb);
                     }
                 }
 #pragma unroll
                 for (int q = 0; q < RC; q++) {
-                    const T v = row[((r0 + q) ^ xr) * NT];
+                    const uint32_t j = (uint32_t)(r0 + q) ^ xr;
+                    const float2 v = ((const float2 *)(row + (j >> 1) * NT))[j & 1];
                     gr[r0 + q] = __builtin_fmaf(dr[q], v.x, __builtin_fmaf(-di[q], v.y, gr[r0 + q]));
                     gi[r0 + q] = __builtin_fmaf(dr[q], v.y, __builtin_fmaf(di[q], v.x, gi[r0 + q]));
                 }
@@ -946,20 +960,20 @@ __device__ __forceinline__ void stream_phase(int g, int ngroups, const float2 *_
                                              const GroupC *__restrict__ groups,
                                              const SubC *__restrict__ subs,
                                              const TermC *__restrict__ terms, uint32_t t0,
-                                             uint32_t tid, const float2 *cur, float2 *nxt,
+                                             uint32_t tid, const float4 *cur, float4 *nxt,
                                              SubC &S, uint32_t &s, GroupC &Gc, GroupC &Gn,
                                              float (&gr)[(1 << TB) / NT],
                                              float (&gi)[(1 << TB) / NT])
 {
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
-    if (g + 1 < ngroups) tile_dma<float2, TB, NT>(in, t0 ^ (Gn.xh << TB), nxt);
+    if (g + 1 < ngroups) tile_dma<float2, TB, NT>(in, t0 ^ (Gn.xh << TB), (float2 *)nxt);
     const GroupC Gnn = groups[g + 2];
-    const uint32_t lane8 = tid * (uint32_t)sizeof(float2), lb = t0 | tid;
+    const uint32_t lane16 = tid * (uint32_t)sizeof(float4), lb = t0 | (tid << 1);
     uint32_t e = Gc.begin;
 #define RP_STREAM_RUN(CLS)                                                                  \
     e += Gc.n[CLS];                                                                         \
-    stream_run<TB, NT, CLS>(s, e, S, subs, cur, lane8, lb, terms, gr, gi);
+    stream_run<TB, NT, CLS>(s, e, S, subs, cur, lane16, lb, terms, gr, gi);
     RP_STREAM_RUN(kRunReal0)
     RP_STREAM_RUN(kRunReal1)
     RP_STREAM_RUN(kRunImag0)
@@ -978,7 +992,7 @@ __device__ __forceinline__ void stream_tile(const float2 *__restrict__ in, float
                                             const GroupC *__restrict__ groups, int ngroups,
                                             const SubC *__restrict__ subs,
                                             const TermC *__restrict__ terms, int accumulate,
-                                            uint32_t t0, float2 *tile0, float2 *tile1)
+                                            uint32_t t0, float4 *tile0, float4 *tile1)
 {
     using T = float2;
     constexpr int RP = (1 << TB) / NT;
@@ -996,7 +1010,7 @@ __device__ __forceinline__ void stream_tile(const float2 *__restrict__ in, float
     GroupC Gc = groups[0], Gn = groups[1];
     uint32_t s = 0;
     SubC S = subs[0];
-    tile_dma<T, TB, NT>(in, t0 ^ (Gc.xh << TB), tile0);
+    tile_dma<T, TB, NT>(in, t0 ^ (Gc.xh << TB), (float2 *)tile0);
     for (int g = 0; g < ngroups; g += 2) {
         stream_phase<TB, NT>(g, ngroups, in, groups, subs, terms, t0, tid, tile0, tile1, S, s, Gc,
                              Gn, gr, gi);
@@ -1007,19 +1021,24 @@ __device__ __forceinline__ void stream_tile(const float2 *__restrict__ in, float
         if ((g / 2) & 1) flush_partials(accr, acci, gr, gi);
     }
     flush_partials(accr, acci, gr, gi);
+    // vectors are aligned to their elements, 8 bytes
+    typedef float Pair __attribute__((ext_vector_type(4), aligned(8)));
 #pragma unroll
-    for (int r = 0; r < RP; r++) {
-        const uint64_t m = (uint64_t)t0 + r * NT + tid;
-        T o;
+    for (int p = 0; p < RP / 2; p++) {
+        Pair *at = (Pair *)(out + (uint64_t)t0 + p * (2 * NT) + 2 * tid), o;
         if (accumulate) {
-            const T p = out[m];
-            o.x = (float)(accr[r] + (double)p.x);
-            o.y = (float)(acci[r] + (double)p.y);
+            const Pair b = *at;
+            o.x = (float)(accr[2 * p] + (double)b.x);
+            o.y = (float)(acci[2 * p] + (double)b.y);
+            o.z = (float)(accr[2 * p + 1] + (double)b.z);
+            o.w = (float)(acci[2 * p + 1] + (double)b.w);
         } else {
-            o.x = (float)accr[r];
-            o.y = (float)acci[r];
+            o.x = (float)accr[2 * p];
+            o.y = (float)acci[2 * p];
+            o.z = (float)accr[2 * p + 1];
+            o.w = (float)acci[2 * p + 1];
         }
-        out[m] = o;
+        *at = o;
     }
 }
 
@@ -1031,8 +1050,8 @@ k_apply_stream(const float2 *__restrict__ in, float2 *__restrict__ out,
                const int *__restrict__ stop)
 {
     if (stop && *stop) return;
-    __shared__ float2 tile0[1 << TB];
-    __shared__ float2 tile1[1 << TB];
+    __shared__ float4 tile0[1 << (TB - 1)];
+    __shared__ float4 tile1[1 << (TB - 1)];
     stream_tile<TB, NT>(in, out, groups, ngroups, subs, terms, accumulate, tile_index(tm) << TB,
                         tile0, tile1);
 }
@@ -1215,20 +1234,25 @@ static void choose_tiling(int prec, int len, uint64_t flips, uint64_t nterms, in
 // per group, two sentinel headers; the multi-sub terms in FP32.  False when
 // a class run of some group has more than 255 subs (the header's count
 // width): the handle then keeps the SubRec kernel.
-static bool compact_stream(const Tables<double> &tab, std::vector<GroupC> &cg,
+static bool compact_stream(const Tables<double> &tab, int tb, int nt, std::vector<GroupC> &cg,
                            std::vector<SubC> &cs, std::vector<TermC> &ct)
 {
-    for (const TermRec<double> &t : tab.terms) ct.push_back({t.z, (float)t.cr, (float)t.ci, 0});
+    for (const TermRec<double> &t : tab.terms)
+        ct.push_back({t.z, (float)t.cr, (float)t.ci, stream_row(t.z, tb, nt)});
     for (const GroupRuns &G : tab.groups) {
         GroupC h{};
         h.xh = G.xh;
         h.begin = G.b[0];
+        // this kernel's row bits are not the SubRec kernel's: the single-term
+        // real and imaginary subs are classed again
+        std::vector<SubC> run[kRuns];
         for (uint32_t k = 0; k < kRuns; k++) {
-            if (G.b[k + 1] - G.b[k] > 255) return false;
-            h.n[k] = (uint8_t)(G.b[k + 1] - G.b[k]);
             for (uint32_t i = G.b[k]; i < G.b[k + 1]; i++) {
                 const SubRec<double> &S = tab.subs[i];
-                SubC c{S.xl, S.z, 0.f, 0.f};
+                const uint32_t zr = k == kRunMulti ? 0 : stream_row(S.z, tb, nt);
+                SubC c{(S.xl & (2u * nt - 2u)) * 8u | stream_row(S.xl, tb, nt) << 16 | zr << 24, S.z,
+                       0.f, 0.f};
+                const uint32_t cls = k >= kRunCplx ? k : (k & ~1u) | (zr ? 1u : 0u);
                 if (k == kRunMulti) {
                     c.z = S.term_begin;
                     memcpy(&c.c0, &S.term_end, sizeof(float));
@@ -1238,8 +1262,13 @@ static bool compact_stream(const Tables<double> &tab, std::vector<GroupC> &cg,
                     c.c0 = S.fr;
                     c.c1 = S.fi;
                 }
-                cs.push_back(c);
+                run[cls].push_back(c);
             }
+        }
+        for (uint32_t k = 0; k < kRuns; k++) {
+            if (run[k].size() > 255) return false;
+            h.n[k] = (uint8_t)run[k].size();
+            cs.insert(cs.end(), run[k].begin(), run[k].end());
         }
         cg.push_back(h);
     }
@@ -1248,7 +1277,7 @@ static bool compact_stream(const Tables<double> &tab, std::vector<GroupC> &cg,
     cg.push_back(end);
     cg.push_back(end);
     cs.push_back({0, 0, 0.f, 0.f});
-    if (ct.empty()) ct.push_back({0, 0.f, 0.f, 0});
+    if (ct.empty()) ct.push_back(TermC{});
     return true;
 }
 
@@ -1401,7 +1430,7 @@ static int upload_impl(rp_terms *h, const uint64_t *bits, const double *coeff, u
         std::vector<GroupC> cg;
         std::vector<SubC> cs;
         std::vector<TermC> ct;
-        if (tb && compact_stream(tab, cg, cs, ct)) {
+        if (tb && compact_stream(tab, tb, h->threads, cg, cs, ct)) {
             if ((st = up(&h->d_cgroups, cg.data(), cg.size() * sizeof(GroupC)))) return st;
             if ((st = up(&h->d_csubs, cs.data(), cs.size() * sizeof(SubC)))) return st;
             if ((st = up(&h->d_cterms, ct.data(), ct.size() * sizeof(TermC)))) return st;
