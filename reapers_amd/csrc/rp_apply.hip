@@ -1057,6 +1057,159 @@ k_apply_stream(const float2 *__restrict__ in, float2 *__restrict__ out,
 }
 
 // ---------------------------------------------------------------------------
+// The same with FP64 sums throughout (complex<double>, and complex<float>
+// without group accumulation): 16-byte records {flip, phase, coefficient} of
+// the real and imaginary single-term subs, one list in group order, the next
+// one loaded while the current one is in use; complex coefficients and flip
+// masks with several terms go through the term list.  The rows are the SubRec
+// kernel's; each sub branches once on its row flip, so that its row reads are
+// immediate offsets, and the reads go out before its sign is formed.  The
+// SubRec kernel's 48-byte records (17 KiB for sparse SYK at 23 qubits) do not
+// fit the 16 KiB scalar cache and its rows need an address each.
+// ---------------------------------------------------------------------------
+struct SubD { uint32_t xl, z; double c; };
+static_assert(sizeof(SubD) == 16, "16-byte record");
+
+template <typename T, int RP, int NT, uint32_t CLS, int XR>
+__device__ __forceinline__ void wide_rows(const T (&v)[RP], double c, uint32_t zr,
+                                          double (&ar)[RP], double (&ai)[RP])
+{
+#pragma unroll
+    for (int j = 0; j < RP; j++) {
+        const int r = j ^ XR;
+        const double x = (double)v[j].x, y = (double)v[j].y;
+        double cc = c;
+        if constexpr (CLS == kRunReal1 || CLS == kRunImag1)
+            cc = flip_sign(c, parity_sign((uint32_t)r & zr));
+        if constexpr (CLS == kRunReal0 || CLS == kRunReal1) {
+            ar[r] = fmadd(cc, x, ar[r]);
+            ai[r] = fmadd(cc, y, ai[r]);
+        } else {
+            ar[r] = fmadd(-cc, y, ar[r]);
+            ai[r] = fmadd(cc, x, ai[r]);
+        }
+    }
+}
+
+template <typename T, int TB, int NT, uint32_t CLS>
+__device__ __forceinline__ void wide_run(uint32_t &s, uint32_t end, SubD &S,
+                                         const SubD *__restrict__ subs, const T *buf, uint32_t lane,
+                                         uint32_t lanebits, const TermRec<double> *__restrict__ terms,
+                                         double (&ar)[(1 << TB) / NT], double (&ai)[(1 << TB) / NT])
+{
+    constexpr int RP = (1 << TB) / NT;
+    constexpr int LB = NT == 1024 ? 10 : NT == 512 ? 9 : NT == 256 ? 8 : 7;
+    for (; s < end; s++) {
+        const T *row = sub_lane_base<T, NT>(buf, lane, S.xl);
+        const uint32_t xr = S.xl >> LB;
+        if constexpr (CLS != kRunMulti) {
+            T v[RP];
+#pragma unroll
+            for (int j = 0; j < RP; j++) v[j] = row[j * NT];
+            asm volatile("" ::: "memory");
+            const SubD Sn = subs[s + 1];     // the list has one sentinel record
+            const uint32_t zr = (S.z >> LB) & (RP - 1);
+            double c = flip_sign(S.c, parity_sign(lanebits & S.z));
+            if constexpr (CLS == kRunReal1 || CLS == kRunImag1) c = opaque(c);
+            with_row_flip<RP>(xr, [&](auto X) {
+                wide_rows<T, RP, NT, CLS, decltype(X)::value>(v, c, zr, ar, ai);
+            });
+            S = Sn;
+        } else {
+            const SubD Sn = subs[s + 1];
+            const uint32_t tb = S.z, te = (uint32_t)__double2loint(S.c);
+            constexpr int RC = RP < 4 ? RP : 4;
+#pragma unroll
+            for (int r0 = 0; r0 < RP; r0 += RC) {
+                double dr[RC], di[RC];
+#pragma unroll
+                for (int q = 0; q < RC; q++) { dr[q] = 0; di[q] = 0; }
+                for (uint32_t t = tb; t < te; t++) {
+                    const TermRec<double> C = terms[t];
+                    const uint32_t lsb = parity_sign(lanebits & C.z);
+                    const double cr = flip_sign(C.cr, lsb), ci = flip_sign(C.ci, lsb);
+                    const uint32_t zr = (C.z >> LB) & (RP - 1);
+#pragma unroll
+                    for (int q = 0; q < RC; q++) {
+                        const uint32_t rsb = parity_sign((r0 + q) & zr);
+                        dr[q] += flip_sign(cr, rsb);
+                        di[q] += flip_sign(ci, rsb);
+                    }
+                }
+#pragma unroll
+                for (int q = 0; q < RC; q++) {
+                    const T v = row[((r0 + q) ^ xr) * NT];
+                    const double x = (double)v.x, y = (double)v.y;
+                    ar[r0 + q] = fmadd(dr[q], x, fmadd(-di[q], y, ar[r0 + q]));
+                    ai[r0 + q] = fmadd(dr[q], y, fmadd(di[q], x, ai[r0 + q]));
+                }
+            }
+            S = Sn;
+        }
+    }
+}
+
+template <typename R, int TB, int NT>
+__global__ void __launch_bounds__(NT, (apply_waves_per_eu<R, TB, NT, 2>()))
+k_apply_wide(const typename CxA<R>::T *__restrict__ in, typename CxA<R>::T *__restrict__ out,
+             const GroupC *__restrict__ groups, int ngroups, const SubD *__restrict__ subs,
+             const TermRec<double> *__restrict__ terms, int accumulate, TileMap tm,
+             const int *__restrict__ stop)
+{
+    using T = typename CxA<R>::T;
+    constexpr int RP = (1 << TB) / NT;
+    if (stop && *stop) return;
+    __shared__ T tile0[1 << TB];
+    __shared__ T tile1[1 << TB];
+    const uint32_t tid = threadIdx.x, t0 = tile_index(tm) << TB;
+    const uint32_t lane = tid * (uint32_t)sizeof(T), lb = t0 | tid;
+    double ar[RP], ai[RP];
+#pragma unroll
+    for (int r = 0; r < RP; r++) { ar[r] = 0; ai[r] = 0; }
+    GroupC Gc = groups[0], Gn = groups[1];
+    uint32_t s = 0;
+    SubD S = subs[0];
+    tile_dma<T, TB, NT>(in, t0 ^ (Gc.xh << TB), tile0);
+    auto stage = [&](int g, const T *cur, T *nxt) __attribute__((always_inline)) {
+        __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();
+        if (g + 1 < ngroups) tile_dma<T, TB, NT>(in, t0 ^ (Gn.xh << TB), nxt);
+        const GroupC Gnn = groups[g + 2];
+        uint32_t e = Gc.begin;
+#define RP_WIDE_RUN(CLS)                                                                    \
+    e += Gc.n[CLS];                                                                         \
+    wide_run<T, TB, NT, CLS>(s, e, S, subs, cur, lane, lb, terms, ar, ai);
+        RP_WIDE_RUN(kRunReal0)
+        RP_WIDE_RUN(kRunReal1)
+        RP_WIDE_RUN(kRunImag0)
+        RP_WIDE_RUN(kRunImag1)
+        RP_WIDE_RUN(kRunMulti)
+#undef RP_WIDE_RUN
+        Gc = Gn;
+        Gn = Gnn;
+    };
+    for (int g = 0; g < ngroups; g += 2) {
+        stage(g, tile0, tile1);
+        if (g + 1 >= ngroups) break;
+        stage(g + 1, tile1, tile0);
+    }
+#pragma unroll
+    for (int r = 0; r < RP; r++) {
+        T *at = out + (uint64_t)t0 + r * NT + tid;
+        double x = ar[r], y = ai[r];
+        if (accumulate) {
+            const T b = *at;
+            x += (double)b.x;
+            y += (double)b.y;
+        }
+        T o;
+        o.x = (R)x;
+        o.y = (R)y;
+        *at = o;
+    }
+}
+
+// ---------------------------------------------------------------------------
 // The apply with the first Gram-Schmidt pass's coefficients formed in its
 // epilogue: after writing its output tile w, the workgroup reads the same
 // rows of V_0..V_{k-1} and writes its FP64 partials of <V_q|w> (columns
@@ -1191,7 +1344,7 @@ static int wave_depth(int len, uint64_t flips, uint64_t nterms)
 
 // default tiling (RP_TERMS_AUTOTUNE measures the alternatives)
 static void choose_tiling(int prec, int len, uint64_t flips, uint64_t nterms, int group_acc,
-                          int *tb, int *nt, int *depth)
+                          int acc64, int *tb, int *nt, int *depth)
 {
     *depth = 2;
     // No tiles for short chains, nor for few flip masks with several terms
@@ -1215,17 +1368,24 @@ static void choose_tiling(int prec, int len, uint64_t flips, uint64_t nterms, in
         *depth = wave_depth(len, flips, nterms);
         return;
     }
-    // Beyond, the tiled kernel: 8 amplitudes per thread.
-    // 2^12-amplitude tiles with 512 threads: for complex<float> sparse SYK at
-    // 24 qubits faster than 2^13 tiles (more groups, but two workgroups per
-    // CU instead of one); for complex<double> the largest tile in 128 KiB.
-    // For complex<float> with group accumulation from 28 sites (states of
-    // 2 GiB and more, beyond every cache) 2^13 tiles with 1024 threads:
-    // sparse SYK at 30 qubits takes 197 ms there against 260 ms with 2^12
-    // tiles
-    if (prec == RP_C64 && group_acc && len >= 28) { *tb = 13; *nt = 1024; return; }
+    // Beyond, tiles of 2^12 amplitudes; for complex<double> the largest in two
+    // 64 KiB buffers.  Sparse SYK, us per apply with 12/512, 12/1024, 13/1024:
+    //   group accumulation: 20 sites 101, 89, 118; 21 sites 140, 161, 139;
+    //     25 sites 3283, 3635, 3325; 26 sites (beyond the Infinity Cache, where
+    //     the workgroups of a CU drift apart and the larger tile has fewer
+    //     passes) 10579, 8946, 7899; 28 sites 59465, 51047, 40086
+    //   FP64 sums: 20 sites 137, 116, 178; 24 sites 1896, 1842, 1984; 26 sites
+    //     9655, 9546, 10130; 27 sites 22901, 21967, 22013; 28 sites 51281,
+    //     53053, 49537
     *tb = 12;
     *nt = 512;
+    if (prec == RP_C64 && group_acc) {
+        if (len >= 26) *tb = 13;
+        if (len >= 26 || len == 20) *nt = 1024;
+    } else if (prec == RP_C64 && acc64) {
+        if (len >= 27) *tb = 13;
+        *nt = 1024;
+    }
 }
 
 // the compact lists of the tiled tables (complex<float> states, FP64 term
@@ -1278,6 +1438,60 @@ static bool compact_stream(const Tables<double> &tab, int tb, int nt, std::vecto
     cg.push_back(end);
     cs.push_back({0, 0, 0.f, 0.f});
     if (ct.empty()) ct.push_back(TermC{});
+    return true;
+}
+
+// Where k_apply_wide takes the place of the SubRec kernel: for complex<float>
+// in every pipeline of two tiles (sparse SYK, 24 qubits: 12/512 1.96 -> 1.90
+// ms, 12/1024 1.97 -> 1.84, 13/1024 2.19 -> 1.98), for complex<double> with 2^12
+// tiles (24 qubits 4.01 -> 3.39 ms); with 2^10 tiles of 128 threads its
+// workgroups drift apart in group order and lose each other's tiles in L2
+// (24 qubits 3.79 -> 5.78 ms), and so do those of complex<float> 2^12 tiles
+// beyond the Infinity Cache (12/512 at 26 qubits 9.65 -> 10.01 ms).
+static bool wide_table(int prec, int acc64, int len, int tb, int depth)
+{
+    return acc64 && depth == 2 && (prec == RP_C64 ? tb > 12 || len <= 25 : tb == 12);
+}
+template <typename R, typename A, int TB, int D> constexpr bool wide_tiling()
+{
+    return sizeof(A) == 8 && D == 2 && (sizeof(R) == 4 || TB == 12);
+}
+
+// the lists of k_apply_wide, in the SubRec order; a complex single term is
+// appended to the term list.  False as for compact_stream.
+static bool compact_wide(Tables<double> &tab, std::vector<GroupC> &cg, std::vector<SubD> &cs)
+{
+    for (const GroupRuns &G : tab.groups) {
+        GroupC h{};
+        h.xh = G.xh;
+        h.begin = G.b[0];
+        for (uint32_t k = 0; k < kRuns; k++) {
+            const uint32_t cls = k == kRunCplx ? (uint32_t)kRunMulti : k;
+            if (h.n[cls] + (G.b[k + 1] - G.b[k]) > 255) return false;
+            h.n[cls] += (uint8_t)(G.b[k + 1] - G.b[k]);
+            for (uint32_t i = G.b[k]; i < G.b[k + 1]; i++) {
+                const SubRec<double> &S = tab.subs[i];
+                SubD c{S.xl, S.z, k == kRunImag0 || k == kRunImag1 ? S.ci : S.cr};
+                if (cls == kRunMulti) {
+                    uint64_t end = S.term_end;
+                    c.z = S.term_begin;
+                    if (k == kRunCplx) {
+                        c.z = (uint32_t)tab.terms.size();
+                        tab.terms.push_back({S.z, 0, S.cr, S.ci});
+                        end = tab.terms.size();
+                    }
+                    memcpy(&c.c, &end, sizeof(double));
+                }
+                cs.push_back(c);
+            }
+        }
+        cg.push_back(h);
+    }
+    GroupC end{};
+    end.begin = (uint32_t)cs.size();
+    cg.push_back(end);
+    cg.push_back(end);
+    cs.push_back({0, 0, 0.0});
     return true;
 }
 
@@ -1421,6 +1635,16 @@ static int upload_impl(rp_terms *h, const uint64_t *bits, const double *coeff, u
         return RP_OK;
     };
     if (!tb && (st = upload_wave<A>(h, flat, up))) return st;
+    if constexpr (sizeof(A) == 8) {
+        std::vector<GroupC> cg;
+        std::vector<SubD> cs;
+        if (tb && !h->group_acc && wide_table(h->prec, h->acc64, h->len, tb, h->depth) &&
+            compact_wide(tab, cg, cs)) {
+            if ((st = up(&h->d_cgroups, cg.data(), cg.size() * sizeof(GroupC)))) return st;
+            if ((st = up(&h->d_csubs, cs.data(), cs.size() * sizeof(SubD)))) return st;
+            RP_CHECK_HIP(hipStreamSynchronize(c.stream));     // host temporaries
+        }
+    }
     if (tb) {
         if ((st = up(&h->d_groups, groups.data(), groups.size() * sizeof(GroupRuns)))) return st;
         if ((st = up(&h->d_subs, subs.data(), subs.size() * sizeof(SubRec<A>)))) return st;
@@ -1430,7 +1654,7 @@ static int upload_impl(rp_terms *h, const uint64_t *bits, const double *coeff, u
         std::vector<GroupC> cg;
         std::vector<SubC> cs;
         std::vector<TermC> ct;
-        if (tb && compact_stream(tab, tb, h->threads, cg, cs, ct)) {
+        if (tb && h->group_acc && compact_stream(tab, tb, h->threads, cg, cs, ct)) {
             if ((st = up(&h->d_cgroups, cg.data(), cg.size() * sizeof(GroupC)))) return st;
             if ((st = up(&h->d_csubs, cs.data(), cs.size() * sizeof(SubC)))) return st;
             if ((st = up(&h->d_cterms, ct.data(), ct.size() * sizeof(TermC)))) return st;
@@ -1470,6 +1694,15 @@ static int launch_tiled(rp_terms *h, void *res, const void *vec, int accumulate,
                       dim3(NT), 0, (const T *)vec, (T *)res, (const GroupRuns *)h->d_groups,
                       (int)h->ngroups, (const SubRec<A> *)h->d_subs,
                       (const TermRec<A> *)h->d_terms, accumulate, h->tmap, stop);
+            return RP_OK;
+        }
+    }
+    if constexpr (wide_tiling<R, A, TB, D>()) {
+        if (h->d_csubs) {
+            RP_LAUNCH(RP_KERNEL_APPLY, (k_apply_wide<R, TB, NT>), dim3((unsigned)grid), dim3(NT), 0,
+                      (const T *)vec, (T *)res, (const GroupC *)h->d_cgroups, (int)h->ngroups,
+                      (const SubD *)h->d_csubs, (const TermRec<double> *)h->d_terms, accumulate,
+                      h->tmap, stop);
             return RP_OK;
         }
     }
@@ -1694,7 +1927,8 @@ int rp_terms_upload_ex(rp_terms_t *out, int prec, int len, const uint64_t *bits,
     h->len = len;
     h->acc64 = (prec == RP_C128 || !(flags & RP_TERMS_ACC_NATIVE)) ? 1 : 0;
     h->group_acc = (prec == RP_C64 && (flags & RP_TERMS_ACC_GROUP)) ? 1 : 0;
-    choose_tiling(prec, len, count_flips(bits, nterms), nterms, h->group_acc, &h->tile_bits, &h->threads, &h->depth);
+    choose_tiling(prec, len, count_flips(bits, nterms), nterms, h->group_acc, h->acc64,
+                  &h->tile_bits, &h->threads, &h->depth);
     h->raw_bits.assign(bits, bits + nterms);
     h->raw_coeff.assign(coeff, coeff + 2 * nterms);
     st = upload_any(h, bits, coeff, nterms);

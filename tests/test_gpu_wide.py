@@ -1,0 +1,79 @@
+"""The tiled apply with FP64 sums over compact records, and the streamed
+apply with group accumulation, at every two-tile tiling: all classes of subs
+(real, imaginary and complex single terms with and without phase bits in the
+row, lane and tile bits, flip masks with several terms), every row flip, one
+and two groups, against the oracle.
+
+Tolerance: FP64 sums of n terms and one rounding of the output; with group
+accumulation FP32 sums of the terms of four groups."""
+import numpy as np
+import pytest
+
+from conftest import random_state
+from gpu_util import DeviceBuffer, Terms, prec_of
+
+pytestmark = pytest.mark.gpu
+
+TILINGS = {32: [(8, 128, 2), (10, 128, 2), (12, 512, 2), (12, 1024, 2), (13, 1024, 2)],
+           64: [(8, 128, 2), (10, 128, 2), (12, 512, 2)]}
+
+
+def _list(rng, L, tb, groups):
+    """Flip masks in `groups` groups: every combination of bit 0 and the top
+    tile bits with a random rest, 1 to 3 terms each."""
+    bits, co = [], []
+    highs = [0] + [int(h) for h in rng.choice(np.arange(1, 1 << (L - tb)), groups - 1, False)]
+    for i in range(64):
+        x = highs[i % groups] << tb | int(rng.integers(0, 1 << tb))
+        x = x & ~1 | i & 1
+        for _ in range((1, 1, 1, 2, 1, 3)[i % 6]):
+            z = int(rng.integers(0, 1 << L)) & (~0, 0x3e, -1 << 6, -1 << tb)[(i // 2) % 4]
+            b = 0
+            for s in range(L):
+                b |= (x >> s & 1) << (2 * s) | (z >> s & 1) << (2 * s + 1)
+            c = rng.standard_normal() + 1j * rng.standard_normal()
+            bits.append(b)
+            co.append((c.real, 1j * c.imag, c)[(i // 6) % 3])
+    return np.array(bits, np.uint64), np.array(co, np.complex128)
+
+
+@pytest.mark.parametrize("fp,group", [(32, False), (32, True), (64, False)])
+@pytest.mark.parametrize("groups", [1, 2, 5])
+def test_two_tile_tilings(gpu, orc, fp, group, groups):
+    L = 16
+    dt = np.complex64 if fp == 32 else np.complex128
+    for tb, nt, d in TILINGS[fp]:
+        rng = np.random.default_rng(tb * nt + groups)
+        bits, co = _list(rng, L, tb, groups)
+        if fp == 32:
+            co = co.astype(np.complex64).astype(np.complex128)
+        psi, prior = random_state(rng, L, dt), random_state(rng, L, dt)
+        ref = orc.apply(L, bits, co, psi.astype(np.complex128), fp=64)
+        t = Terms(L, bits, co, prec_of(dt), gpu.RP_TERMS_ACC_GROUP if group else 0)
+        gpu.check(gpu.hip().rp_terms_set_tiling(t.h, tb, nt, d))
+        vin = DeviceBuffer.from_array(psi)
+        out = DeviceBuffer.from_array(prior)
+        eps = 1.2e-7 if group else 2.3e-16
+        tol = len(bits) * eps * np.abs(co).sum() * np.abs(psi).max() + \
+            (6e-8 if fp == 32 else 1.2e-16) * (np.abs(ref).max() + np.abs(prior).max())
+        for acc in (1, 0):
+            gpu.check(gpu.hip().rp_apply_ops(t.h, out.ptr, vin.ptr, acc))
+            got = out.to_array(dt, len(psi)).astype(np.complex128)
+            assert np.abs(got - (ref + prior if acc else ref)).max() <= tol, (tb, nt, acc)
+        vin.free()
+        out.free()
+        t.free()
+
+
+@pytest.mark.parametrize("fp,group,L", [(32, False, 20), (32, True, 20), (64, False, 20),
+                                        (32, False, 26), (32, True, 26), (32, False, 27)])
+def test_default_tilings(gpu, fp, group, L):
+    """The default layout's choice at the sizes where it changes."""
+    rng = np.random.default_rng(L)
+    bits = np.array([int(rng.integers(1, 1 << (2 * L))) for _ in range(60)], np.uint64)
+    t = Terms(L, bits, np.ones(60), gpu.RP_C64 if fp == 32 else gpu.RP_C128,
+              gpu.RP_TERMS_ACC_GROUP if group else 0)
+    i = t.info()
+    want = {(64, False): (12, 512), (32, True): (12, 1024) if L == 20 else (13, 1024),
+            (32, False): (13, 1024) if L >= 27 else (12, 1024)}[fp, group]
+    assert (i.tile_bits, i.threads, i.depth) == want + (2,)
