@@ -1596,8 +1596,18 @@ static int upload_wave(rp_terms *h, const std::vector<FlatTerm<A>> &flat, UP &&u
     if ((st = up(&h->d_wcut, cut.data(), cut.size() * sizeof(uint32_t)))) return st;
     if (wave_part_bytes(h)) {
         const size_t chunks = std::max<uint64_t>(1, dim / (64 * h->rows));
-        std::vector<char> z(wave_part_bytes(h) + chunks * sizeof(unsigned), 0);
-        if ((st = up(&h->d_split, z.data(), z.size()))) return st;
+        // the partial sums are written before they are read: only the arrival
+        // counters behind them start at zero
+        const std::vector<unsigned> zero(chunks, 0u);
+        const size_t at = wave_part_bytes(h), bytes = at + chunks * sizeof(unsigned);
+        if (dev_malloc(&h->d_split, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            return set_error(RP_ERR_OUT_OF_MEMORY, "Failed to allocate %zu bytes on GPU device.",
+                             bytes);
+        }
+        RP_CHECK_HIP(hipMemcpyAsync((char *)h->d_split + at, zero.data(), bytes - at,
+                                    hipMemcpyHostToDevice, ctx().stream));
+        RP_CHECK_HIP(hipStreamSynchronize(ctx().stream));     // zero is a host temporary
     }
     // the tables are host temporaries
     RP_CHECK_HIP(hipStreamSynchronize(ctx().stream));
@@ -1862,11 +1872,14 @@ static int autotune(rp_terms *h)
     if (hipMemsetAsync(x, 0, bytes, c.stream) != hipSuccess ||
         hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess)
         st = set_error(RP_ERR_RUNTIME, "rp_terms_upload_ex: autotuning set-up failed");
+    // Without tiles, 32 and 128 slices only up to 16 sites: beyond, they are
+    // at least eight times the wavefronts the GPU holds, and their partial sums
+    // (67 MB at 19 sites) cost the upload more than the rest of it.
     for (const TilingDesc &cd : kTilings) {
         if (st) break;
         if (cd.tb > h->len || !tiling_instantiated(h->prec, cd.tb, cd.nt, cd.depth)) continue;
         if (cd.tb == 0 && (cd.depth == 1 ? h->len > kWaveMaxLen && h->nflips > kWaveMaxFlips
-                                         : h->len > kWaveMaxLen ||
+                                         : h->len > (cd.depth == 8 ? kWaveMaxLen : kSplitMaxLen) ||
                                                h->nterms < (uint64_t)(2 * cd.depth)))
             continue;
         if ((st = retile(h, cd.tb, cd.nt, cd.depth))) break;
