@@ -222,7 +222,7 @@ int rp_gs_pass_fused(int prec, const void *const *V, int k, void *w, uint64_t n,
  * device memory (code under HIP graph capture, tight serving loops, harnesses
  * that forbid it); no counterpart in the reference.  Same arguments and
  * results as rp_gs_pass_fused; its reduction partials and results live in a
- * fixed 1.06 MB device array of the library (one per GPU, taken at rp_init)
+ * fixed 1.08 MB device array of the library (one per GPU, taken at rp_init)
  * instead of the library workspace, which limits k to 64 (larger k is
  * rejected with RP_ERR_INVALID_ARGUMENT; n is unlimited).  Every call on a
  * GPU shares that GPU's array and leaves its last contents there: calls that

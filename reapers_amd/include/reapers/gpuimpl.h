@@ -357,10 +357,11 @@ public:
 
     // Apply through the dense matrix when the term count reaches 2^len (the
     // reference's switch in DevSumOps::upload, inc/gpuimpl.h:1068-1084), up
-    // to 15 sites.  Off by default: at those sizes the term-split kernel is
-    // faster (a dense SYK N=24 evolution: 3.8 ms against 11.2 ms in FP64,
-    // 7.3 ms against 37.8 ms in FP32) and sums FP32 states in FP64, where
-    // the matrix-vector product sums in the state's precision.
+    // to 15 sites.  Off by default: at those sizes the kernel without
+    // tiles is faster (a dense SYK N=24 evolution in FP64: 2.7 ms against
+    // 11.2 ms; its slower predecessor took 7.3 ms in FP32 against 37.8 ms)
+    // and sums FP32 states in FP64, where the matrix-vector product sums in
+    // the state's precision.
     static bool &dense_apply() {
         static bool on = false;
         return on;
