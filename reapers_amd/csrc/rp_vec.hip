@@ -45,7 +45,8 @@ struct Coefs { double c[2 * kMaxVecs]; };
 // are reserved), then the results of the pass in flight:
 //   [0, 2k) coefficients h; kResNorm (host only) the norm after the pass when
 //   it was not fused; kResIn ||w||^2 before it; kResBeta the fused norm (0: not
-//   fused); kResStop (an int) set by an Arnoldi step that needs the host;
+//   fused); kResStop (an int) set by an Arnoldi step that needs the host, to
+//   the step's number;
 //   kResCount arrival counters of the dot workgroups, zero between launches
 //   (for each row of workgroups one, and 16 below it, 64 bytes apart).
 // The pinned host copy that the kernels write has the layout up to kResStop.
@@ -454,10 +455,14 @@ k_gs_update(VecPtrs V, int k, typename Cx<R>::T *__restrict__ w, uint64_t n,
 template <typename R>
 __global__ void __launch_bounds__(kRedThreads)
 k_gs_finish(typename Cx<R>::T *__restrict__ w, uint64_t n, const double *__restrict__ part, int nb,
-            double *res, int scale, double min_norm, double *__restrict__ host, int *stop)
+            double *res, int scale, double min_norm, double *__restrict__ host, int *stop, int step)
 {
     __shared__ double sh[(kWaves + 1) * 1];
-    if ((stop && *(volatile int *)stop) || res[kResBeta] > 0) return;
+    if (res[kResBeta] > 0) return;
+    if (stop) {
+        const int s = *(volatile int *)stop;
+        if (s && s != step) return;
+    }
     double v[1] = {0.0};
     for (int p = threadIdx.x; p < nb; p += kRedThreads) v[0] += part[p];
     block_reduce<1>(v, sh);
@@ -467,7 +472,7 @@ k_gs_finish(typename Cx<R>::T *__restrict__ w, uint64_t n, const double *__restr
         res[2] = norm;
         res[3] = 0.0;
         host[kResNorm] = norm;
-        if (scale && !ok && stop) *stop = 1;
+        if (scale && !ok && stop) *(volatile int *)stop = step;
     }
     if (!scale || !ok) return;
     const R f = (R)(1.0 / norm);
@@ -609,7 +614,7 @@ static int dots_launch(int cls, const VecPtrs &P, int k, const void *w, uint64_t
 // queue the update of w by V[0..k) and the end of the pass
 template <typename R>
 static int update_launch(const VecPtrs &P, int k, void *w, uint64_t n, double *work, double *host,
-                         double fuse_min, int scale, double min_norm, int *stop)
+                         double fuse_min, int scale, double min_norm, int *stop, int step)
 {
     using T = typename Cx<R>::T;
     const int nb = red_blocks(n), kr = (k - 1) % kUpdChunk + 1;
@@ -628,7 +633,7 @@ static int update_launch(const VecPtrs &P, int k, void *w, uint64_t n, double *w
 #undef RP_UPD
 #undef RP_UPD_LONG
     RP_LAUNCH(RP_KERNEL_GS, k_gs_finish<R>, dim3(scale ? nb : 1), dim3(kRedThreads), 0, (T *)w, n,
-              (const double *)work, nb, res, scale, min_norm, host, stop);
+              (const double *)work, nb, res, scale, min_norm, host, stop, step);
     return RP_OK;
 }
 
@@ -658,7 +663,7 @@ static int gs_pass_impl(const void *const *V, int k, void *w, uint64_t n, double
         return st;
     }
     if (k > 0 &&
-        (st = update_launch<R>(P, k, w, n, work, host, fuse_min, 0, 0.0, (int *)nullptr)))
+        (st = update_launch<R>(P, k, w, n, work, host, fuse_min, 0, 0.0, (int *)nullptr, 0)))
         return st;
     if ((st = wait_results())) return st;
     for (int q = 0; q < 2 * k; q++) h[q] = host[q];
@@ -721,12 +726,13 @@ static int steps_impl(rp_terms_t hd, void *const *V, int j0, int m, uint64_t n, 
             P.p[1] = j > j0 ? V[j - 1] : nullptr;
             if ((st = dots_launch<R>(RP_KERNEL_GS, P, 1, V[j + 1], n, work, 1, host, stop))) break;
             if (j == m - 1) break;
-            st = update_launch<R>(P, j > j0 ? 2 : 1, V[j + 1], n, work, host, 0.0, 1, 0.0, stop);
+            st = update_launch<R>(P, j > j0 ? 2 : 1, V[j + 1], n, work, host, 0.0, 1, 0.0, stop, 0);
         } else {
             P.p[j] = V[j];
             if ((st = dots_launch<R>(RP_KERNEL_GS, P, j + 1, V[j + 1], n, work, 0, nullptr,
                                      stop))) break;
-            st = update_launch<R>(P, j + 1, V[j + 1], n, work, host, min_norm, 1, min_norm, stop);
+            st = update_launch<R>(P, j + 1, V[j + 1], n, work, host, min_norm, 1, min_norm, stop,
+                                  j + 1);
         }
         if (st) break;
     }

@@ -119,6 +119,40 @@ def test_arnoldi_steps_stop(gpu, dtype):
             assert np.array_equal(bufs[j].to_array(dtype, 4), mark)
 
 
+@pytest.mark.parametrize("dtype", [np.complex64, np.complex128])
+@pytest.mark.parametrize("length", [9, 18, 20])
+def test_arnoldi_steps_stop_leaves_the_pass_result(gpu, dtype, length):
+    """The step that stops leaves its vector unscaled, also where the pass's
+    last kernel runs in up to 1024 workgroups and one of them raises the stop
+    flag while others start.  H = Z0 + 2 X1 + X2 / 20 on |000> times a random
+    state of the other sites: step 1 leaves X1 X2 V0 / (5 b0), b0 = H(1, 0), of
+    norm below 0.25."""
+    n, m = 1 << length, 4
+    rng = np.random.default_rng(length)
+    bits = np.array([2, 1 << 2, 1 << 4], np.uint64)
+    t = Terms(length, bits, np.array([1.0, 2.0, 0.05]), prec_of(dtype))
+    v = np.zeros(n, np.complex128)
+    v[::8] = rng.standard_normal(n // 8) + 1j * rng.standard_normal(n // 8)
+    v = (v / np.linalg.norm(v)).astype(dtype)
+    b0 = np.hypot(2, 0.05)
+    want = np.zeros(n, np.complex128)
+    want[6::8] = v[::8] * (0.2 / b0)
+    mark = np.full(n, 7, dtype)
+    for _ in range(4):
+        bufs = [DeviceBuffer.from_array(v if j == 0 else mark) for j in range(m + 1)]
+        out, done = np.zeros((m, STEP)), ctypes.c_int()
+        gpu.check(gpu.hip().rp_arnoldi_steps(t.h, _ptrs(bufs), 0, m, 0.25,
+                                             out.ctypes.data_as(_vp), ctypes.byref(done)))
+        assert done.value == 2 and out[1, 129] == 0
+        # roundings of the stored V0, V1 and V2, of norms 1, 1 and 0.1, carried
+        # through H of norm 3.05
+        tol = 16 * EPS[dtype]
+        assert abs(out[0, 128] - b0) <= tol and abs(out[1, 128] - 0.2 / b0) <= tol
+        assert np.linalg.norm(bufs[2].to_array(dtype, n) - want) <= tol
+        for j in (3, 4):
+            assert np.array_equal(bufs[j].to_array(dtype, n), mark)
+
+
 @pytest.mark.parametrize("length,m", [(3, 1), (3, 2), (8, 12), (10, 30)])
 def test_lanczos_steps(gpu, length, m):
     rng = np.random.default_rng(length)
