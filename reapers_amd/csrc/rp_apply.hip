@@ -1723,13 +1723,31 @@ static int launch_tiled(rp_terms *h, void *res, const void *vec, int accumulate,
     return RP_OK;
 }
 
+// res = 0: the apply of an operator without terms
+template <typename T>
+__global__ void __launch_bounds__(kSmallThreads)
+k_apply_none(T *__restrict__ out, uint64_t dim, const int *__restrict__ stop)
+{
+    if (stop && *stop) return;
+    for (uint64_t i = blockIdx.x * (uint64_t)kSmallThreads + threadIdx.x; i < dim;
+         i += (uint64_t)gridDim.x * kSmallThreads) {
+        T e;
+        e.x = 0;
+        e.y = 0;
+        out[i] = e;
+    }
+}
+
 template <typename R, typename A>
 static int apply_impl(rp_terms *h, void *res, const void *vec, int accumulate, const int *stop)
 {
     using T = typename CxA<R>::T;
     const uint64_t dim = 1ull << h->len;
     if (h->nterms == 0) {
-        if (!accumulate) RP_CHECK_HIP(hipMemsetAsync(res, 0, dim * sizeof(T), ctx().stream));
+        if (accumulate) return RP_OK;
+        const uint64_t wgs = (dim + kSmallThreads - 1) / kSmallThreads;
+        RP_LAUNCH(RP_KERNEL_APPLY, k_apply_none<T>, dim3((unsigned)std::min<uint64_t>(wgs, 8192)),
+                  dim3(kSmallThreads), 0, (T *)res, dim, stop);
         return RP_OK;
     }
     if (h->tile_bits == 0) {

@@ -680,8 +680,7 @@ int setup_planes(rp_batch *b, const uint64_t *bits, const double *coeff, uint64_
 {
     const int fl = (autotune ? RP_TERMS_AUTOTUNE : 0) | (b->group_acc ? RP_TERMS_ACC_GROUP : 0);
     int st = rp_terms_upload_ex(&b->plane_terms, b->prec, b->len[0], bits, coeff, nterms, fl);
-    // no term left (H = 0): the single-state apply would clear its output
-    // with a memset, which a captured restart must not hold; the batched
+    // no term left (H = 0): nothing that planes would serve; the batched
     // kernel takes it
     rp_terms_info_t ti;
     if (!st && !(st = rp_terms_info(b->plane_terms, &ti)) && ti.nterms == 0) {

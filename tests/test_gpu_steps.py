@@ -153,6 +153,29 @@ def test_arnoldi_steps_stop_leaves_the_pass_result(gpu, dtype, length):
             assert np.array_equal(bufs[j].to_array(dtype, n), mark)
 
 
+@pytest.mark.parametrize("dtype", [np.complex64, np.complex128])
+@pytest.mark.parametrize("length", [2, 13])
+def test_arnoldi_steps_without_terms(gpu, dtype, length):
+    """H = 0 stops at its first step: V[1] is zero and the rest untouched."""
+    n, m = 1 << length, 4
+    t = Terms(length, np.array([2], np.uint64), np.zeros(1), prec_of(dtype))
+    mark = np.full(n, 7, dtype)
+    v = np.zeros(n, dtype)
+    v[1] = 1
+    bufs = [DeviceBuffer.from_array(v if j == 0 else mark) for j in range(m + 1)]
+    out, done = np.zeros((m, STEP)), ctypes.c_int()
+    gpu.check(gpu.hip().rp_arnoldi_steps(t.h, _ptrs(bufs), 0, m, 0.25, out.ctypes.data_as(_vp),
+                                         ctypes.byref(done)))
+    assert done.value == 1 and out[0, 128] == 0
+    assert not bufs[1].to_array(dtype, n).any()
+    for j in range(2, m + 1):
+        assert np.array_equal(bufs[j].to_array(dtype, n), mark), j
+    gpu.check(gpu.hip().rp_apply_ops(t.h, bufs[2].ptr, bufs[0].ptr, 1))
+    assert np.array_equal(bufs[2].to_array(dtype, n), mark)
+    gpu.check(gpu.hip().rp_apply_ops(t.h, bufs[2].ptr, bufs[0].ptr, 0))
+    assert not bufs[2].to_array(dtype, n).any()
+
+
 @pytest.mark.parametrize("length,m", [(3, 1), (3, 2), (8, 12), (10, 30)])
 def test_lanczos_steps(gpu, length, m):
     rng = np.random.default_rng(length)
