@@ -93,9 +93,9 @@ __device__ __forceinline__ uint32_t xcd_tile_index()
 //
 // For chains of up to kWaveMaxLen sites, whose tiles are too few to fill the
 // 256 CUs, the flip masks are cut into `depth` slices of about equal work,
-// one per wavefront, so that all CUs have several wavefronts; the four of a
-// workgroup add their sums in LDS, workgroups through memory, the last one to
-// arrive in slice order.  Bound by latency there: dense SYK N=24 FP64 (10626
+// one per wavefront, so that all CUs have several wavefronts; the 8 or 16 of
+// a workgroup add their sums in LDS, workgroups through memory, the last one
+// to arrive in slice order.  Bound by latency there: dense SYK N=24 FP64 (10626
 // terms, 4096 amplitudes) took 33 us in one chain of loads per term and slice
 // and 14 us in a second launch that added the slices.
 // ---------------------------------------------------------------------------
@@ -111,14 +111,27 @@ template <typename A> struct TermW { uint64_t lanes; A c; uint32_t z, pad; };
 constexpr int kWaveMaxLen = 19, kWaveMaxFlips = 40;
 constexpr int kWavePad = 16;       // flip masks read past the end of the list
 
-// c with the sign of (-1)^popcount(v), v uniform
-__device__ __forceinline__ float uniform_sign(float c, uint32_t v)
+__device__ __forceinline__ float flip_bit31(float c, uint32_t b)
 {
-    return __uint_as_float(__float_as_uint(c) ^ ((uint32_t)__popc(v) << 31));
+    return __uint_as_float(__float_as_uint(c) ^ b);
 }
-__device__ __forceinline__ double uniform_sign(double c, uint32_t v)
+__device__ __forceinline__ double flip_bit31(double c, uint32_t b)
 {
-    return __hiloint2double(__double2hiint(c) ^ (int)((uint32_t)__popc(v) << 31), __double2loint(c));
+    return __hiloint2double(__double2hiint(c) ^ (int)b, __double2loint(c));
+}
+// c with the sign of (-1)^popcount(m & z), uniform, for the first amplitude
+// m = m0 of each row r of 64 (index bits 6 and 7 number four rows)
+template <typename A, int ROWS>
+__device__ __forceinline__ void row_signs(A c, uint32_t m0, uint32_t z, A (&s)[ROWS])
+{
+    static_assert(ROWS == 1 || ROWS == 4, "rows");
+    s[0] = flip_bit31(c, (uint32_t)__popc(m0 & z) << 31);
+    if constexpr (ROWS == 4) {
+        const uint32_t b0 = (z << 25) & 0x80000000u, b1 = (z << 24) & 0x80000000u;
+        s[1] = flip_bit31(s[0], b0);
+        s[2] = flip_bit31(s[0], b1);
+        s[3] = flip_bit31(s[1], b1);
+    }
 }
 // +-1 by the lane's bit of `neg`
 __device__ __forceinline__ float lane_sign(uint64_t neg, float)
@@ -136,9 +149,10 @@ template <typename A, int ROWS, bool BYROW>
 __device__ __forceinline__ void add_term(const TermW<A> &C, uint32_t m0, A (&d)[ROWS])
 {
     const A sg = lane_sign(C.lanes, A(0));
+    A c[BYROW ? ROWS : 1];
+    row_signs<A, BYROW ? ROWS : 1>(C.c, m0, C.z, c);
 #pragma unroll
-    for (int r = 0; r < (BYROW ? ROWS : 1); r++)
-        d[r] = fma(sg, uniform_sign(C.c, (m0 | (r * 64)) & C.z), d[r]);
+    for (int r = 0; r < (BYROW ? ROWS : 1); r++) d[r] = fma(sg, c[r], d[r]);
 }
 
 template <typename A, int ROWS, bool BYROW>
@@ -172,17 +186,26 @@ template <typename T, typename A, int ROWS>
 __device__ __forceinline__ void add_rows(const A (&d)[ROWS], const T (&v)[ROWS], bool imag,
                                          A (&ar)[ROWS], A (&ai)[ROWS])
 {
+    // the components as values first: sunk below the branch, their loads from
+    // v became one load at a chosen address, and v an array in scratch memory
+    A x[ROWS], y[ROWS];
+#pragma unroll
+    for (int r = 0; r < ROWS; r++) {
+        x[r] = v[r].x;
+        y[r] = v[r].y;
+        if constexpr (ROWS == 1 && sizeof(A) == 4) asm volatile("" : "+v"(x[r]), "+v"(y[r]));
+    }
     if (!imag) {
 #pragma unroll
         for (int r = 0; r < ROWS; r++) {
-            ar[r] = fma(d[r], (A)v[r].x, ar[r]);
-            ai[r] = fma(d[r], (A)v[r].y, ai[r]);
+            ar[r] = fma(d[r], x[r], ar[r]);
+            ai[r] = fma(d[r], y[r], ai[r]);
         }
     } else {
 #pragma unroll
         for (int r = 0; r < ROWS; r++) {
-            ar[r] = fma(-d[r], (A)v[r].y, ar[r]);
-            ai[r] = fma(d[r], (A)v[r].x, ai[r]);
+            ar[r] = fma(-d[r], y[r], ar[r]);
+            ai[r] = fma(d[r], x[r], ai[r]);
         }
     }
 }
@@ -249,16 +272,26 @@ k_apply_wave(const typename CxA<R>::T *__restrict__ in, typename CxA<R>::T *__re
             }
             return;
         }
-        const A g0 = lane_sign(S.l0, A(0)), g1 = lane_sign(S.l1, A(0));
+        const A g0 = lane_sign(S.l0, A(0));
         if (ROWS > 1 && (S.kind & kWaveRow)) {
+            A c[ROWS];
+            row_signs<A, ROWS>(S.c0, m0, S.z0, c);
 #pragma unroll
-            for (int r = 0; r < ROWS; r++) {
-                d[r] = g0 * uniform_sign(S.c0, (m0 | (r * 64)) & S.z0);
-                d[r] = fma(g1, uniform_sign(S.c1, (m0 | (r * 64)) & S.z1), d[r]);
+            for (int r = 0; r < ROWS; r++) d[r] = g0 * c[r];
+            if (S.kind & kWaveTwo) {
+                const A g1 = lane_sign(S.l1, A(0));
+                row_signs<A, ROWS>(S.c1, m0, S.z1, c);
+#pragma unroll
+                for (int r = 0; r < ROWS; r++) d[r] = fma(g1, c[r], d[r]);
             }
         } else {
-            d[0] = g0 * uniform_sign(S.c0, m0 & S.z0);
-            if (S.kind & kWaveTwo) d[0] = fma(g1, uniform_sign(S.c1, m0 & S.z1), d[0]);
+            A c[1];
+            row_signs<A, 1>(S.c0, m0, S.z0, c);
+            d[0] = g0 * c[0];
+            if (S.kind & kWaveTwo) {
+                row_signs<A, 1>(S.c1, m0, S.z1, c);
+                d[0] = fma(lane_sign(S.l1, A(0)), c[0], d[0]);
+            }
 #pragma unroll
             for (int r = 1; r < ROWS; r++) d[r] = d[0];
         }
@@ -321,26 +354,28 @@ k_apply_wave(const typename CxA<R>::T *__restrict__ in, typename CxA<R>::T *__re
                 put_shared(q + 64, (double)ai[r]);
             }
             if (!arrive_last(count + chunk, nw)) return;
-            // at most 8 workgroups: all their sums in flight
-            double p[8][2 * ROWS];
+            // at most 8 workgroups, the sums of 8 / ROWS of them in flight
+            constexpr int PER = 8 / ROWS;
+            double sum[2 * ROWS] = {};
+            for (uint32_t i0 = 0; i0 < nw; i0 += PER) {
+                double p[PER][2 * ROWS];
 #pragma unroll
-            for (int i = 0; i < 8; i++)
+                for (int i = 0; i < PER; i++)
 #pragma unroll
-                for (int r = 0; r < 2 * ROWS; r++)
-                    p[i][r] = (uint32_t)i < nw
-                                  ? get_shared(row + (size_t)i * (128 * ROWS) + r * 64)
-                                  : 0.0;
+                    for (int r = 0; r < 2 * ROWS; r++)
+                        p[i][r] = i0 + i < nw
+                                      ? get_shared(row + (size_t)(i0 + i) * (128 * ROWS) + r * 64)
+                                      : 0.0;
+#pragma unroll
+                for (int i = 0; i < PER; i++)
+#pragma unroll
+                    for (int r = 0; r < 2 * ROWS; r++) sum[r] += p[i][r];
+            }
             if (lane == 0) count[chunk] = 0;
 #pragma unroll
             for (int r = 0; r < ROWS; r++) {
-                double sr = p[0][2 * r], si = p[0][2 * r + 1];
-#pragma unroll
-                for (int i = 1; i < 8; i++) {
-                    sr += p[i][2 * r];
-                    si += p[i][2 * r + 1];
-                }
-                ar[r] = (A)sr;
-                ai[r] = (A)si;
+                ar[r] = (A)sum[2 * r];
+                ai[r] = (A)sum[2 * r + 1];
             }
         }
     }
@@ -1328,17 +1363,51 @@ static uint64_t count_flips(const uint64_t *bits, uint64_t n)
     return (uint64_t)(std::unique(x.begin(), x.end()) - x.begin());
 }
 
-// slices of the flip masks for the kernel without tiles: the most that keep
-// about 8192 wavefronts (the GPU holds that many; with 8 slices each lane has
-// four amplitudes from 17 sites on) and the work of 24 terms a slice
-static int wave_depth(int len, uint64_t flips, uint64_t nterms)
+// Amplitudes per lane of the kernel without tiles: four where that leaves
+// enough wavefronts.  Every term's sign and record is then shared by four
+// amplitudes, and the scalar instructions of a flip mask (about 35), which
+// bound the lists of many masks, by 256 instead of 64.
+static int wave_rows(int len, int depth, uint64_t flips, uint64_t nterms)
+{
+    if (len > kSplitMaxLen || depth == 1)
+        return depth <= 8 && ((uint64_t)depth << len) >= (1ull << 20) ? 4 : 1;
+    return len > 8 && ((uint64_t)depth << (len - 8)) >= 2048 &&
+                   flips + nterms >= (uint64_t)(10 * depth)
+               ? 4 : 1;
+}
+
+// Slices of the flip masks for the kernel without tiles.  With one amplitude
+// per lane the most that keep about 8192 wavefronts (the GPU holds that many;
+// with 8 slices each lane has four amplitudes from 17 sites on) and the work
+// of 22 terms a slice.  From 13 to 16 sites longer lists take four amplitudes
+// per lane and the slices that give at least 2048 wavefronts; more of them
+// only where the list is long enough to pay for adding the sums of 8 to 16
+// times as many workgroups.  us per apply, one amplitude a lane (8 slices at
+// 15 and 16 sites, 32 below) / four, masks x terms a mask, complex<float>:
+//   13 sites: 300 x 1  6.3 / 7.8 (not taken), 300 x 4  12.4 / 10.1, 1000 x 4  30.5 / 17.8
+//   14 sites: 100 x 4  10.4 / 9.6 (32 slices), 1000 x 1  18.8 / 15.7, 4000 x 4  216 / 99
+//   15 sites: 300 x 1  11.5 / 9.6, 1000 x 1  31.8 / 20.4, 1000 x 4  108 / 48.8
+//   16 sites: 300 x 1  18.4 / 12.9 (8 slices), 1000 x 1  53 / 37, 4000 x 4  765 / 357
+// and FP32 sums, whose wavefronts need half the registers, 128 slices at 15
+// sites: 4000 x 1  64.4 (32) / 61.8, 4000 x 4  155 / 129, 1000 x 1  19.3 / 20.2.
+static int wave_depth(int len, uint64_t flips, uint64_t nterms, int acc64)
 {
     const uint64_t chunks = len > 6 ? 1ull << (len - 6) : 1;
     int d = 1;
     for (int s : {8, 32, 128})
         if (chunks * s <= (s == 8 ? 65536 : 8192) && flips >= (uint64_t)s &&
-            6 * flips + nterms >= (uint64_t)(24 * s))
+            6 * flips + nterms >= (uint64_t)(22 * s))
             d = s;
+    if (len < 13 || len > kSplitMaxLen) return d;
+    uint64_t more = 0;             // list length from which more slices pay
+    for (int s : {8, 32, 128}) {
+        const uint64_t waves = (uint64_t)s << (len - 8);
+        if (waves < 2048 || flips < (uint64_t)s) continue;
+        if (waves > (acc64 ? 8192u : 16384u)) break;
+        if (waves > 8192) more = 4096;
+        if (flips + nterms >= std::max<uint64_t>(10 * s, more)) d = s;
+        more = 1280;
+    }
     return d;
 }
 
@@ -1365,7 +1434,7 @@ static void choose_tiling(int prec, int len, uint64_t flips, uint64_t nterms, in
     if (len <= kWaveMaxLen || (flips <= kWaveMaxFlips && several)) {
         *tb = 0;
         *nt = kSmallThreads;
-        *depth = wave_depth(len, flips, nterms);
+        *depth = wave_depth(len, flips, nterms, acc64);
         return;
     }
     // Beyond, tiles of 2^12 amplitudes; for complex<double> the largest in two
@@ -1525,8 +1594,7 @@ template <typename A, typename UP>
 static int upload_wave(rp_terms *h, const std::vector<FlatTerm<A>> &flat, UP &&up)
 {
     const uint64_t dim = 1ull << h->len;
-    // four amplitudes per lane where that leaves enough wavefronts
-    h->rows = h->depth <= 8 && dim * (uint64_t)h->depth >= (1ull << 20) ? 4 : 1;
+    h->rows = wave_rows(h->len, h->depth, h->nflips, h->nterms);
     std::vector<SubW<A>> subs;
     std::vector<TermW<A>> terms;
     std::vector<uint32_t> flips;
@@ -1762,7 +1830,8 @@ static int apply_impl(rp_terms *h, void *res, const void *vec, int accumulate, c
               (const T *)vec, (T *)res, dim, (const uint32_t *)h->d_wflips,                      \
               (const SubW<A> *)h->d_wsubs, (const TermW<A> *)h->d_wterms,                        \
               (const uint32_t *)h->d_wcut, h->depth, accumulate, (double *)h->d_split, count, stop)
-        if (w == 16) RP_WAVE(1, 16, false);
+        if (w == 16 && h->rows == 1) RP_WAVE(1, 16, false);
+        else if (w == 16) RP_WAVE(4, 16, false);
         else if (w == 8 && h->rows == 1) RP_WAVE(1, 8, false);
         else if (w == 8) RP_WAVE(4, 8, false);
         else if (h->rows == 1) RP_WAVE(1, 4, false);

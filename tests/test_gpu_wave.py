@@ -65,3 +65,28 @@ def test_apply_without_tiles(gpu, orc, fp, native, L, masks):
         out.free()
     vin.free()
     t.free()
+
+
+@pytest.mark.parametrize("fp,native", [(32, False), (32, True), (64, False)])
+@pytest.mark.parametrize("L,masks,depth", [(13, 400, 128), (14, 160, 32), (14, 400, 128),
+                                           (15, 150, 32), (15, 1250, None), (16, 40, 8),
+                                           (16, 400, 32)])
+def test_long_lists(gpu, orc, fp, native, L, masks, depth):
+    """The slices and four amplitudes a lane that lists of many terms get from
+    13 to 16 sites, with phase bits in the row bits (sites 6 and 7)."""
+    rng = np.random.default_rng(1000 * L + masks + fp)
+    dt = np.complex64 if fp == 32 else np.complex128
+    bits, co = _terms(rng, L, masks, fp)
+    psi, prior = random_state(rng, L, dt), random_state(rng, L, dt)
+    ref = orc.apply(L, bits, co, psi.astype(np.complex128), fp=64)
+    t = Terms(L, bits, co, prec_of(dt), gpu.RP_TERMS_ACC_NATIVE if native else 0)
+    info = t.info()
+    assert info.kernel == gpu.RP_APPLY_SMALL and info.depth == (depth or (128 if native else 32))
+    vin, out = DeviceBuffer.from_array(psi), DeviceBuffer.from_array(prior)
+    eps = 1.2e-7 if native else 2.3e-16
+    tol = len(bits) * eps * np.abs(co).sum() * np.abs(psi).max() + \
+        (6e-8 if fp == 32 else 1.2e-16) * (np.abs(ref).max() + np.abs(prior).max())
+    for acc in (1, 0, 0):
+        gpu.check(gpu.hip().rp_apply_ops(t.h, out.ptr, vin.ptr, acc))
+        got = out.to_array(dt, len(psi)).astype(np.complex128)
+        assert np.abs(got - (ref + prior if acc else ref)).max() <= tol, acc
