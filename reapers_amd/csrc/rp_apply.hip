@@ -99,7 +99,7 @@ __device__ __forceinline__ uint32_t xcd_tile_index()
 // terms, 4096 amplitudes) took 33 us in one chain of loads per term and slice
 // and 14 us in a second launch that added the slices.
 // ---------------------------------------------------------------------------
-// One flip mask.  One or two terms of one kind (real, or kWaveImag imaginary
+// One flip mask, or a piece of one.  One or two terms of one kind (real, or kWaveImag imaginary
 // coefficients) stand in the record itself (kWaveTwo: two); kWaveRow: one of
 // them has phase bits among the row bits.  Otherwise (kWaveMulti) the terms
 // from `term` on: real ones without and with such bits, then imaginary ones
@@ -110,6 +110,12 @@ template <typename A> struct TermW { uint64_t lanes; A c; uint32_t z, pad; };
 
 constexpr int kWaveMaxLen = 19, kWaveMaxFlips = 40;
 constexpr int kWavePad = 16;       // flip masks read past the end of the list
+// Where the list is cut into slices, a flip mask of more terms than this is
+// cut into records of its own, each with its gather (worth about six terms),
+// so that few masks of many terms fill the slices too: one mask of 300 terms
+// at 14 sites 15.0 us in one slice, 6.1 in 8 (the
+// kernel of one record a term it replaced: 10.4).
+constexpr uint32_t kWavePiece = 32;
 
 __device__ __forceinline__ float flip_bit31(float c, uint32_t b)
 {
@@ -1354,25 +1360,36 @@ static bool tiling_instantiated(int prec, int tb, int nt, int d)
     return false;
 }
 
-// distinct flip masks of a term list (zero coefficients included)
-static uint64_t count_flips(const uint64_t *bits, uint64_t n)
+// what the choice of a layout looks at in a term list (zero coefficients
+// included)
+struct ListShape {
+    uint64_t terms, flips;    // terms, distinct flip masks
+    uint64_t pieces;          // flip masks in pieces of kWavePiece terms
+};
+static ListShape list_shape(const uint64_t *bits, uint64_t n)
 {
     std::vector<uint32_t> x(n);
     for (uint64_t t = 0; t < n; t++) x[t] = pext_even(bits[t]);
     std::sort(x.begin(), x.end());
-    return (uint64_t)(std::unique(x.begin(), x.end()) - x.begin());
+    ListShape L{n, 0, 0};
+    for (uint64_t i = 0, j; i < n; i = j) {
+        for (j = i; j < n && x[j] == x[i];) j++;
+        L.flips++;
+        L.pieces += (j - i + kWavePiece - 1) / kWavePiece;
+    }
+    return L;
 }
 
 // Amplitudes per lane of the kernel without tiles: four where that leaves
 // enough wavefronts.  Every term's sign and record is then shared by four
 // amplitudes, and the scalar instructions of a flip mask (about 35), which
 // bound the lists of many masks, by 256 instead of 64.
-static int wave_rows(int len, int depth, uint64_t flips, uint64_t nterms)
+static int wave_rows(int len, int depth, uint64_t pieces, uint64_t nterms)
 {
     if (len > kSplitMaxLen || depth == 1)
         return depth <= 8 && ((uint64_t)depth << len) >= (1ull << 20) ? 4 : 1;
     return len > 8 && ((uint64_t)depth << (len - 8)) >= 2048 &&
-                   flips + nterms >= (uint64_t)(10 * depth)
+                   pieces + nterms >= (uint64_t)(10 * depth)
                ? 4 : 1;
 }
 
@@ -1390,31 +1407,32 @@ static int wave_rows(int len, int depth, uint64_t flips, uint64_t nterms)
 //   16 sites: 300 x 1  18.4 / 12.9 (8 slices), 1000 x 1  53 / 37, 4000 x 4  765 / 357
 // and FP32 sums, whose wavefronts need half the registers, 128 slices at 15
 // sites: 4000 x 1  64.4 (32) / 61.8, 4000 x 4  155 / 129, 1000 x 1  19.3 / 20.2.
-static int wave_depth(int len, uint64_t flips, uint64_t nterms, int acc64)
+static int wave_depth(int len, uint64_t pieces, uint64_t nterms, int acc64)
 {
     const uint64_t chunks = len > 6 ? 1ull << (len - 6) : 1;
     int d = 1;
     for (int s : {8, 32, 128})
-        if (chunks * s <= (s == 8 ? 65536 : 8192) && flips >= (uint64_t)s &&
-            6 * flips + nterms >= (uint64_t)(22 * s))
+        if (chunks * s <= (s == 8 ? 65536 : 8192) && pieces >= (uint64_t)s &&
+            6 * pieces + nterms >= (uint64_t)(22 * s))
             d = s;
     if (len < 13 || len > kSplitMaxLen) return d;
     uint64_t more = 0;             // list length from which more slices pay
     for (int s : {8, 32, 128}) {
         const uint64_t waves = (uint64_t)s << (len - 8);
-        if (waves < 2048 || flips < (uint64_t)s) continue;
+        if (waves < 2048 || pieces < (uint64_t)s) continue;
         if (waves > (acc64 ? 8192u : 16384u)) break;
         if (waves > 8192) more = 4096;
-        if (flips + nterms >= std::max<uint64_t>(10 * s, more)) d = s;
+        if (pieces + nterms >= std::max<uint64_t>(10 * s, more)) d = s;
         more = 1280;
     }
     return d;
 }
 
 // default tiling (RP_TERMS_AUTOTUNE measures the alternatives)
-static void choose_tiling(int prec, int len, uint64_t flips, uint64_t nterms, int group_acc,
-                          int acc64, int *tb, int *nt, int *depth)
+static void choose_tiling(int prec, int len, const ListShape &L, int group_acc, int acc64, int *tb,
+                          int *nt, int *depth)
 {
+    const uint64_t flips = L.flips, nterms = L.terms;
     *depth = 2;
     // No tiles for short chains, nor for few flip masks with several terms
     // each, whose sums the tiled kernel forms for every row.  us per apply
@@ -1434,7 +1452,7 @@ static void choose_tiling(int prec, int len, uint64_t flips, uint64_t nterms, in
     if (len <= kWaveMaxLen || (flips <= kWaveMaxFlips && several)) {
         *tb = 0;
         *nt = kSmallThreads;
-        *depth = wave_depth(len, flips, nterms, acc64);
+        *depth = wave_depth(len, L.pieces, nterms, acc64);
         return;
     }
     // Beyond, tiles of 2^12 amplitudes; for complex<double> the largest in two
@@ -1587,14 +1605,22 @@ static int xcd_resident_bits(int prec, int tb, int nt, int depth)
 }
 
 // The tables of k_apply_wave from the x-sorted terms: one record per flip
-// mask, its terms by class, and the cuts of the flip masks into h->depth
+// mask (or piece of it), its terms by class, and the cuts of the flip masks into h->depth
 // slices of about equal work (a flip mask costs about as much as six terms:
 // the gather, its address and the products).
 template <typename A, typename UP>
 static int upload_wave(rp_terms *h, const std::vector<FlatTerm<A>> &flat, UP &&up)
 {
     const uint64_t dim = 1ull << h->len;
-    h->rows = wave_rows(h->len, h->depth, h->nflips, h->nterms);
+    const size_t piece = h->depth > 1 ? kWavePiece : flat.size();
+    auto run_end = [&](size_t i) {
+        size_t j = i;
+        while (j < flat.size() && flat[j].x == flat[i].x && j - i < piece) j++;
+        return j;
+    };
+    uint64_t pieces = 0;
+    for (size_t i = 0; i < flat.size(); i = run_end(i)) pieces++;
+    h->rows = wave_rows(h->len, h->depth, pieces, flat.size());
     std::vector<SubW<A>> subs;
     std::vector<TermW<A>> terms;
     std::vector<uint32_t> flips;
@@ -1606,11 +1632,11 @@ static int upload_wave(rp_terms *h, const std::vector<FlatTerm<A>> &flat, UP &&u
     };
     const uint32_t rowbits = 64u * (h->rows - 1);
     for (size_t i = 0; i < flat.size();) {
-        size_t j = i;
+        const size_t j = run_end(i);
         bool re = true, im = true;
-        for (; j < flat.size() && flat[j].x == flat[i].x; j++) {
-            re = re && flat[j].ci == 0;
-            im = im && flat[j].cr == 0;
+        for (size_t q = i; q < j; q++) {
+            re = re && flat[q].ci == 0;
+            im = im && flat[q].cr == 0;
         }
         SubW<A> S{};
         uint64_t work = 6;
@@ -2027,8 +2053,8 @@ int rp_terms_upload_ex(rp_terms_t *out, int prec, int len, const uint64_t *bits,
     h->len = len;
     h->acc64 = (prec == RP_C128 || !(flags & RP_TERMS_ACC_NATIVE)) ? 1 : 0;
     h->group_acc = (prec == RP_C64 && (flags & RP_TERMS_ACC_GROUP)) ? 1 : 0;
-    choose_tiling(prec, len, count_flips(bits, nterms), nterms, h->group_acc, h->acc64,
-                  &h->tile_bits, &h->threads, &h->depth);
+    choose_tiling(prec, len, list_shape(bits, nterms), h->group_acc, h->acc64, &h->tile_bits,
+                  &h->threads, &h->depth);
     h->raw_bits.assign(bits, bits + nterms);
     h->raw_coeff.assign(coeff, coeff + 2 * nterms);
     st = upload_any(h, bits, coeff, nterms);

@@ -90,3 +90,38 @@ def test_long_lists(gpu, orc, fp, native, L, masks, depth):
         gpu.check(gpu.hip().rp_apply_ops(t.h, out.ptr, vin.ptr, acc))
         got = out.to_array(dt, len(psi)).astype(np.complex128)
         assert np.abs(got - (ref + prior if acc else ref)).max() <= tol, acc
+
+
+@pytest.mark.parametrize("fp,native", [(32, False), (32, True), (64, False)])
+@pytest.mark.parametrize("L,masks,per,depth", [(9, 1, 33, 1), (12, 2, 100, 8), (14, 1, 300, 8),
+                                               (16, 3, 700, 32), (18, 1, 260, 8)])
+def test_masks_of_many_terms(gpu, orc, fp, native, L, masks, per, depth):
+    """Few flip masks of many terms are cut into pieces that fill the slices
+    (the last one of a single term at 33)."""
+    rng = np.random.default_rng(1000 * L + per + fp)
+    dt = np.complex64 if fp == 32 else np.complex128
+    bits, co = [], []
+    for x in rng.choice(1 << L, masks, False):
+        for q in range(per):
+            z = int(rng.integers(0, 1 << L))
+            bits.append(sum((int(x) >> s & 1) << (2 * s) | (z >> s & 1) << (2 * s + 1)
+                            for s in range(L)))
+            co.append(rng.standard_normal() * (1j if q % 3 == 1 else 1))
+    bits, co = np.array(bits, np.uint64), np.array(co, np.complex128)
+    if fp == 32:
+        co = co.astype(np.complex64).astype(np.complex128)
+    psi = random_state(rng, L, dt)
+    ref = orc.apply(L, bits, co, psi.astype(np.complex128), fp=64)
+    t = Terms(L, bits, co, prec_of(dt), gpu.RP_TERMS_ACC_NATIVE if native else 0)
+    info = t.info()
+    assert info.kernel == gpu.RP_APPLY_SMALL and info.depth == depth
+    assert info.nflips == masks
+    vin, out = DeviceBuffer.from_array(psi), DeviceBuffer(psi.nbytes)
+    eps = 1.2e-7 if native else 2.3e-16
+    tol = len(bits) * eps * np.abs(co).sum() * np.abs(psi).max() + \
+        (6e-8 if fp == 32 else 1.2e-16) * np.abs(ref).max()
+    for d in [depth] + ([1, 8, 128] if L <= 16 else []):
+        if d != info.depth:
+            gpu.check(gpu.hip().rp_terms_set_tiling(t.h, 0, 256, d))
+        gpu.check(gpu.hip().rp_apply_ops(t.h, out.ptr, vin.ptr, 0))
+        assert np.abs(out.to_array(dt, len(psi)).astype(np.complex128) - ref).max() <= tol, d
