@@ -978,13 +978,23 @@ __device__ __forceinline__ void stream_run(uint32_t &s, uint32_t end, SubC &S,
                         di[q] += flip_sign(ci, rsb);
                     }
                 }
+                // input pair ((r0 + q) ^ xr) / 2, its halves exchanged where xr is
+                // odd: 16-byte reads (8 bytes of every 16 took the LDS twice)
+                float4 v[RC / 2];
 #pragma unroll
-                for (int q = 0; q < RC; q++) {
-                    const uint32_t j = (uint32_t)(r0 + q) ^ xr;
-                    const float2 v = ((const float2 *)(row + (j >> 1) * NT))[j & 1];
-                    gr[r0 + q] = __builtin_fmaf(dr[q], v.x, __builtin_fmaf(-di[q], v.y, gr[r0 + q]));
-                    gi[r0 + q] = __builtin_fmaf(dr[q], v.y, __builtin_fmaf(di[q], v.x, gi[r0 + q]));
-                }
+                for (int a = 0; a < RC / 2; a++) v[a] = row[((r0 / 2 + a) ^ (xr >> 1)) * NT];
+                auto pairs = [&](auto X) __attribute__((always_inline)) {
+#pragma unroll
+                    for (int q = 0; q < RC; q++) {
+                        const float4 w = v[q / 2];
+                        const bool hi = (q ^ decltype(X)::value) & 1;
+                        const float x = hi ? w.z : w.x, y = hi ? w.w : w.y;
+                        gr[r0 + q] = __builtin_fmaf(dr[q], x, __builtin_fmaf(-di[q], y, gr[r0 + q]));
+                        gi[r0 + q] = __builtin_fmaf(dr[q], y, __builtin_fmaf(di[q], x, gi[r0 + q]));
+                    }
+                };
+                if (xr & 1) pairs(IC<1>{});
+                else pairs(IC<0>{});
             }
         }
         S = Sn;
