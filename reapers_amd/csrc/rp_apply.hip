@@ -113,8 +113,7 @@ constexpr int kWavePad = 16;       // flip masks read past the end of the list
 // Where the list is cut into slices, a flip mask of more terms than this is
 // cut into records of its own, each with its gather (worth about six terms),
 // so that few masks of many terms fill the slices too: one mask of 300 terms
-// at 14 sites 15.0 us in one slice, 6.1 in 8 (the
-// kernel of one record a term it replaced: 10.4).
+// at 14 sites takes 15.0 us in one slice, 6.1 in 8.
 constexpr uint32_t kWavePiece = 32;
 
 __device__ __forceinline__ float flip_bit31(float c, uint32_t b)
@@ -1373,21 +1372,47 @@ static bool tiling_instantiated(int prec, int tb, int nt, int d)
 // what the choice of a layout looks at in a term list (zero coefficients
 // included)
 struct ListShape {
-    uint64_t terms, flips;    // terms, distinct flip masks
-    uint64_t pieces;          // flip masks in pieces of kWavePiece terms
+    uint64_t terms = 0, flips = 0;    // terms, distinct flip masks
+    uint64_t pieces = 0;              // flip masks in pieces of kWavePiece terms
+    uint64_t groups = 0;              // distinct flip masks above 2^12 tiles
+    uint64_t shared = 0;              // terms of flip masks that have several
+    uint64_t by_row = 0;              // terms of flip masks with more than two that
+                                      // have a phase bit among the row bits of
+                                      // k_apply_wave
 };
 static ListShape list_shape(const uint64_t *bits, uint64_t n)
 {
-    std::vector<uint32_t> x(n);
-    for (uint64_t t = 0; t < n; t++) x[t] = pext_even(bits[t]);
-    std::sort(x.begin(), x.end());
-    ListShape L{n, 0, 0};
+    std::vector<uint64_t> xz(n);
+    for (uint64_t t = 0; t < n; t++)
+        xz[t] = (uint64_t)pext_even(bits[t]) << 32 | pext_odd(bits[t]);
+    std::sort(xz.begin(), xz.end());
+    ListShape L;
+    L.terms = n;
     for (uint64_t i = 0, j; i < n; i = j) {
-        for (j = i; j < n && x[j] == x[i];) j++;
+        uint64_t rows = 0;
+        for (j = i; j < n && xz[j] >> 32 == xz[i] >> 32; j++) rows += (xz[j] & (3u << 6)) != 0;
         L.flips++;
         L.pieces += (j - i + kWavePiece - 1) / kWavePiece;
+        if (!i || xz[i] >> 44 != xz[i - 1] >> 44) L.groups++;
+        if (j - i > 1) L.shared += j - i;
+        if (j - i > 2) L.by_row += rows;
     }
     return L;
+}
+
+// Whether a list is long enough for the 16-byte records of k_apply_wide.  The
+// 48-byte ones of a short list stay in the 16 KiB scalar cache, and reading
+// them costs less than the branch on the row flip that k_apply_wide makes for
+// every record.  us per apply, single-term masks, 48-byte / 16-byte records:
+//   complex<float> 12/1024:   20 sites, 150 masks 76 / 63; 22 sites, 150 222 / 219;
+//     24 sites, 150 895 / 936, 200 1095 / 1119, 240 1421 / 1355; 25 sites, 200
+//     2213 / 2364, 240 2804 / 2767
+//   complex<double> 12/512:   20 sites, 150 masks 94 / 80; 22 sites, 60 158 / 163;
+//     24 sites, 200 2082 / 2202, 240 3032 / 2635; 26 sites, 200 9923 / 10613,
+//     240 14464 / 12210, and 60 masks of 3 terms 6577 / 7640, 200 of 3 24734 / 22615
+static bool long_list(int len, uint64_t flips, uint64_t shared)
+{
+    return flips + shared / 4 >= (len <= 20 ? 0u : len <= 22 ? 110u : 234u);
 }
 
 // Amplitudes per lane of the kernel without tiles: four where that leaves
@@ -1538,16 +1563,20 @@ static bool compact_stream(const Tables<double> &tab, int tb, int nt, std::vecto
     return true;
 }
 
-// Where k_apply_wide takes the place of the SubRec kernel: for complex<float>
-// in every pipeline of two tiles (sparse SYK, 24 qubits: 12/512 1.96 -> 1.90
-// ms, 12/1024 1.97 -> 1.84, 13/1024 2.19 -> 1.98), for complex<double> with 2^12
-// tiles (24 qubits 4.01 -> 3.39 ms); with 2^10 tiles of 128 threads its
-// workgroups drift apart in group order and lose each other's tiles in L2
-// (24 qubits 3.79 -> 5.78 ms), and so do those of complex<float> 2^12 tiles
-// beyond the Infinity Cache (12/512 at 26 qubits 9.65 -> 10.01 ms).
-static bool wide_table(int prec, int acc64, int len, int tb, int depth)
+// Where k_apply_wide takes the place of the SubRec kernel, the list being
+// long enough: for complex<float> in every pipeline of two tiles (sparse SYK,
+// 24 qubits: 12/512 1.96 -> 1.90 ms, 12/1024 1.97 -> 1.84, 13/1024 2.19 -> 1.98),
+// for complex<double> with 2^12 tiles (24 qubits 4.01 -> 3.39 ms); with 2^10
+// tiles of 128 threads its workgroups drift apart in group order and lose
+// each other's tiles in L2 (24 qubits 3.79 -> 5.78 ms), and so do those of
+// complex<float> 2^12 tiles beyond the Infinity Cache (12/512 at 26 qubits
+// 9.65 -> 10.01 ms, at 25 320 masks 3.81 -> 4.13 ms; 12/1024 there 3.79 -> 3.82).
+static bool wide_table(int prec, int acc64, int len, int tb, int nt, int depth, uint64_t flips,
+                       uint64_t shared)
 {
-    return acc64 && depth == 2 && (prec == RP_C64 ? tb > 12 || len <= 25 : tb == 12);
+    if (!acc64 || depth != 2) return false;
+    if (prec == RP_C64 ? tb <= 12 && len > (nt == 1024 ? 25 : 24) : tb != 12) return false;
+    return long_list(len, flips, shared);
 }
 template <typename R, typename A, int TB, int D> constexpr bool wide_tiling()
 {
@@ -1752,7 +1781,9 @@ static int upload_impl(rp_terms *h, const uint64_t *bits, const double *coeff, u
     if constexpr (sizeof(A) == 8) {
         std::vector<GroupC> cg;
         std::vector<SubD> cs;
-        if (tb && !h->group_acc && wide_table(h->prec, h->acc64, h->len, tb, h->depth) &&
+        if (tb && !h->group_acc &&
+            wide_table(h->prec, h->acc64, h->len, tb, h->threads, h->depth, nflips,
+                       terms.size()) &&
             compact_wide(tab, cg, cs)) {
             if ((st = up(&h->d_cgroups, cg.data(), cg.size() * sizeof(GroupC)))) return st;
             if ((st = up(&h->d_csubs, cs.data(), cs.size() * sizeof(SubD)))) return st;

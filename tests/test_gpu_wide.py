@@ -65,6 +65,33 @@ def test_two_tile_tilings(gpu, orc, fp, group, groups):
         t.free()
 
 
+@pytest.mark.parametrize("fp", [32, 64])
+@pytest.mark.parametrize("masks,per", [(109, 1), (110, 1), (60, 3), (75, 2)])
+def test_record_formats(gpu, orc, fp, masks, per):
+    """Both sides of the list length at which the FP64 sums change from 48-byte
+    to 16-byte records (21 sites: 110 masks, or fewer that share terms)."""
+    L = 21
+    dt = np.complex64 if fp == 32 else np.complex128
+    rng = np.random.default_rng(masks + per)
+    x = np.repeat(rng.choice(1 << L, masks, False), per)
+    z = rng.integers(0, 1 << L, len(x))
+    bits = np.zeros(len(x), np.uint64)
+    for s in range(L):
+        bits |= ((x >> s & 1) << (2 * s) | (z >> s & 1) << (2 * s + 1)).astype(np.uint64)
+    co = rng.standard_normal(len(x)) * 1j ** (np.arange(len(x)) % 2)
+    if fp == 32:
+        co = co.astype(np.complex64).astype(np.complex128)
+    psi = random_state(rng, L, dt)
+    ref = orc.apply(L, bits, co, psi.astype(np.complex128), fp=64)
+    t = Terms(L, bits, co, prec_of(dt))
+    gpu.check(gpu.hip().rp_terms_set_tiling(t.h, 12, 512, 2))
+    vin, out = DeviceBuffer.from_array(psi), DeviceBuffer(psi.nbytes)
+    gpu.check(gpu.hip().rp_apply_ops(t.h, out.ptr, vin.ptr, 0))
+    tol = len(bits) * 2.3e-16 * np.abs(co).sum() * np.abs(psi).max() + \
+        (6e-8 if fp == 32 else 1.2e-16) * np.abs(ref).max()
+    assert np.abs(out.to_array(dt, len(psi)).astype(np.complex128) - ref).max() <= tol
+
+
 @pytest.mark.parametrize("fp,group,L", [(32, False, 20), (32, True, 20), (64, False, 20),
                                         (32, False, 26), (32, True, 26), (32, False, 27)])
 def test_default_tilings(gpu, fp, group, L):
