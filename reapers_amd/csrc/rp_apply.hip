@@ -1097,7 +1097,7 @@ __global__ void __launch_bounds__(NT, (apply_waves_per_eu<float, TB, NT, 2>()))
 k_apply_stream(const float2 *__restrict__ in, float2 *__restrict__ out,
                const GroupC *__restrict__ groups, int ngroups, const SubC *__restrict__ subs,
                const TermC *__restrict__ terms, int accumulate, TileMap tm,
-               const int *__restrict__ stop)
+              const int *__restrict__ stop)
 {
     if (stop && *stop) return;
     __shared__ float4 tile0[1 << (TB - 1)];
@@ -1204,7 +1204,7 @@ __global__ void __launch_bounds__(NT, (apply_waves_per_eu<R, TB, NT, 2>()))
 k_apply_wide(const typename CxA<R>::T *__restrict__ in, typename CxA<R>::T *__restrict__ out,
              const GroupC *__restrict__ groups, int ngroups, const SubD *__restrict__ subs,
              const TermRec<double> *__restrict__ terms, int accumulate, TileMap tm,
-             const int *__restrict__ stop)
+              const int *__restrict__ stop)
 {
     using T = typename CxA<R>::T;
     constexpr int RP = (1 << TB) / NT;
@@ -1376,8 +1376,7 @@ struct ListShape {
     uint64_t pieces = 0;              // flip masks in pieces of kWavePiece terms
     uint64_t groups = 0;              // distinct flip masks above 2^12 tiles
     uint64_t shared = 0;              // terms of flip masks that have several
-    uint64_t by_row = 0;              // terms of flip masks with more than two that
-                                      // have a phase bit among the row bits of
+    uint64_t by_row = 0;              // those with a phase bit among the row bits of
                                       // k_apply_wave
 };
 static ListShape list_shape(const uint64_t *bits, uint64_t n)
@@ -1394,8 +1393,9 @@ static ListShape list_shape(const uint64_t *bits, uint64_t n)
         L.flips++;
         L.pieces += (j - i + kWavePiece - 1) / kWavePiece;
         if (!i || xz[i] >> 44 != xz[i - 1] >> 44) L.groups++;
-        if (j - i > 1) L.shared += j - i;
-        if (j - i > 2) L.by_row += rows;
+        if (j - i == 1) continue;
+        L.shared += j - i;
+        L.by_row += rows;
     }
     return L;
 }
@@ -1463,49 +1463,89 @@ static int wave_depth(int len, uint64_t pieces, uint64_t nterms, int acc64)
     return d;
 }
 
+// Whether the apply takes no tiles by default.  Without tiles every flip mask
+// reads the state once, with tiles every group of masks that agree above the
+// tile; a term of a shared mask costs the tiled kernel a product for every
+// row, the other only a sum, and that once for four rows unless the term has
+// a phase bit among the row bits.
+//
+// Short chains have too few tiles for the 256 CUs.  us per apply without
+// tiles / with (12, 512, 2), FP64 sums:
+//   sparse SYK, k = 8, complex<float>:  16 sites 17 / 93, 18 sites 41 / 110,
+//     19 sites 80 / 136 (group accumulation 80 / 87), 20 sites 154 / 153,
+//     21 sites 321 / 210; complex<double> 19 sites 92 / 137, 20 191 / 160
+//   random masks of single terms at 19 sites: 1000 248 / 309, 4000 964 / 1107;
+//     but group accumulation 300 76 / 79, 1000 239 / 194 (12/1024), 4000 937 /
+//     649; from 12000 masks on its tiled kernel's records overflow, 2810 / 3119
+//
+// From 20 sites on few flip masks (up to 40) that share terms:
+//   XXZ with fields (4 terms a mask), FP64 sums:  20 sites 17 / 40, 24 sites
+//     201 / 431, 26 sites 1050 / 1814, complex<double> 24 sites 385 / 728
+//   with group accumulation / its best tiling:  24 sites 195 / 310, 26 sites
+//     1052 / 1329
+//   random masks, whose terms mostly have row bits: FP64 sums, 24 sites, 20
+//     masks x 4 terms  375 / 381, 40 x 20  1911 / 2264; group accumulation
+//     375 / 313 and 1916 / 1586; FP32 sums 312 / 290 and 1531 / 1687
+// Two terms a mask is the narrow case, decided by how many groups the masks
+// make; us, masks / groups:
+//   complex<float>, FP64 sums: 26 sites 10/10 802 / 582, 40/33 1947 / 2071, 27
+//     sites 20/15 2516 / 2034, XY chain 26/15 2223 / 2454
+//   group accumulation: 22 sites 20/18 58 / 71, 40/20 116 / 106, XY chain
+//     21/11 46 / 62; 24 sites 10/9 158 / 141, XY chain 23/13 186 / 235
+//   complex<double>: 22 sites 40/28 194 / 243, 23 sites 40/28 465 / 449, 26
+//     sites 40/30 4252 / 3666, XY chain 25/15 1885 / 2640
+static bool without_tiles(int prec, int len, const ListShape &L, int group_acc, int acc64)
+{
+    const bool single = 2 * L.terms < 3 * L.flips;
+    if (len <= kWaveMaxLen)
+        return !(len == kWaveMaxLen && group_acc && single && L.flips >= 600 && L.flips <= 8192);
+    if (L.flips > kWaveMaxFlips || L.terms < 2 * L.flips) return false;
+    const bool fp32 = prec == RP_C64 && (group_acc || !acc64), rows = 4 * L.by_row > L.terms;
+    if (2 * L.terms < 5 * L.flips) {      // two terms a mask
+        if (fp32 && rows) return len < 24 && 2 * L.flips < 3 * L.groups;
+        if (fp32) return len < 24 || (len == 24 && 6 * L.flips >= 7 * L.groups);
+        if (prec == RP_C128) return len < 23 || 3 * L.flips >= 5 * L.groups;
+        return len < 26 || 6 * L.flips >= (len == 26 ? 7 : 10) * L.groups;
+    }
+    return !fp32 || !rows ||
+           (!group_acc && (L.terms >= 6 * L.flips || 2 * L.flips < 3 * L.groups));
+}
+
 // default tiling (RP_TERMS_AUTOTUNE measures the alternatives)
 static void choose_tiling(int prec, int len, const ListShape &L, int group_acc, int acc64, int *tb,
                           int *nt, int *depth)
 {
-    const uint64_t flips = L.flips, nterms = L.terms;
     *depth = 2;
-    // No tiles for short chains, nor for few flip masks with several terms
-    // each, whose sums the tiled kernel forms for every row.  us per apply
-    // without tiles / with (12, 512, 2), FP64 sums, default upload:
-    //   sparse SYK, k = 8, complex<float>:  16 sites 17 / 93, 18 sites 41 / 110,
-    //     19 sites 80 / 136 (group accumulation 80 / 87), 20 sites 154 / 153,
-    //     21 sites 321 / 210; complex<double> 19 sites 92 / 137, 20 191 / 160
-    //   XXZ with fields (4 terms a mask):   20 sites 21 / 40, 24 sites 209 / 431,
-    //     26 sites 1072 / 1814, complex<double> 24 sites 388 / 728
-    //   XY chain (2 a mask):                20 sites 16 / 28, 24 sites 196 / 297
-    //   transverse Ising (under 2):         22 sites 54 / 60, 24 sites 205 / 204
-    //   one a mask, 20 masks:               22 sites 54 / 50, 24 sites 249 / 189
-    // and with group accumulation XY 20 sites 16 / 23, 24 sites 199 / 244, but
-    // 26 sites (beyond the Infinity Cache) 1071 / 1030, XXZ there 1072 / 1461.
-    const bool several = nterms >= 2 * flips &&
-                         !(group_acc && len >= 25 && 2 * nterms < 5 * flips);
-    if (len <= kWaveMaxLen || (flips <= kWaveMaxFlips && several)) {
+    if (without_tiles(prec, len, L, group_acc, acc64)) {
         *tb = 0;
         *nt = kSmallThreads;
-        *depth = wave_depth(len, L.pieces, nterms, acc64);
+        *depth = wave_depth(len, L.pieces, L.terms, acc64);
         return;
     }
-    // Beyond, tiles of 2^12 amplitudes; for complex<double> the largest in two
-    // 64 KiB buffers.  Sparse SYK, us per apply with 12/512, 12/1024, 13/1024:
-    //   group accumulation: 20 sites 101, 89, 118; 21 sites 140, 161, 139;
-    //     25 sites 3283, 3635, 3325; 26 sites (beyond the Infinity Cache, where
-    //     the workgroups of a CU drift apart and the larger tile has fewer
-    //     passes) 10579, 8946, 7899; 28 sites 59465, 51047, 40086
-    //   FP64 sums: 20 sites 137, 116, 178; 24 sites 1896, 1842, 1984; 26 sites
-    //     9655, 9546, 10130; 27 sites 22901, 21967, 22013; 28 sites 51281,
-    //     53053, 49537
+    // Tiles of 2^12 amplitudes by 512 threads; for complex<double> the largest
+    // in two 64 KiB buffers.  us per apply with 12/512, 12/1024, 13/1024:
+    //   group accumulation, sparse SYK: 20 sites 101, 89, 118; 21 sites 140,
+    //     161, 139; 25 sites 3283, 3635, 3325; 26 sites (beyond the Infinity
+    //     Cache, where the workgroups of a CU drift apart and the larger tile has
+    //     fewer passes) 10579, 8946, 7899; 28 sites 59465, 51047, 40086
+    //   but masks that share terms, 60 x 3: 24 sites 777, 720, 884; 26 sites
+    //     2953, 2725, 3484; 28 sites 12773, 11840, 15067; and few single ones:
+    //     26 sites, 20 masks 869, 863, 983, 60 masks 1702, 1726, 1825 in one
+    //     list and 2225, 2092, 2098 in another
+    //   FP64 sums, sparse SYK: 20 sites 137, 116, 178; 24 sites 1896, 1842, 1984;
+    //     26 sites 9655, 9546, 10130; 27 sites 20634, 20351, 20351; 28 sites
+    //     44428, 49490, 44979
+    //   200 single masks: 24 sites 1133, 1119, -; 27 sites 11994, 11067, 12870;
+    //     28 sites 23980, 24228, 26742; 60 x 3: 26 sites 3853, 3517, 4777; 28
+    //     sites 14982, 13698, 18917
     *tb = 12;
     *nt = 512;
-    if (prec == RP_C64 && group_acc) {
-        if (len >= 26) *tb = 13;
-        if (len >= 26 || len == 20) *nt = 1024;
-    } else if (prec == RP_C64 && acc64) {
-        if (len >= 27) *tb = 13;
+    if (prec != RP_C64 || (!group_acc && !acc64)) return;
+    const bool single = 2 * L.terms < 3 * L.flips;
+    if (group_acc) {
+        if (single && (len >= 28 || (len >= 26 && L.flips > 64))) *tb = 13;
+        if (!single || *tb == 13 || len <= 20) *nt = 1024;
+    } else if (!single || (len < 28 && long_list(len, L.flips, L.shared))) {
         *nt = 1024;
     }
 }

@@ -92,15 +92,66 @@ def test_record_formats(gpu, orc, fp, masks, per):
     assert np.abs(out.to_array(dt, len(psi)).astype(np.complex128) - ref).max() <= tol
 
 
-@pytest.mark.parametrize("fp,group,L", [(32, False, 20), (32, True, 20), (64, False, 20),
-                                        (32, False, 26), (32, True, 26), (32, False, 27)])
-def test_default_tilings(gpu, fp, group, L):
-    """The default layout's choice at the sizes where it changes."""
-    rng = np.random.default_rng(L)
-    bits = np.array([int(rng.integers(1, 1 << (2 * L))) for _ in range(60)], np.uint64)
-    t = Terms(L, bits, np.ones(60), gpu.RP_C64 if fp == 32 else gpu.RP_C128,
-              gpu.RP_TERMS_ACC_GROUP if group else 0)
+def _random(rng, L, masks, per, row_bits=True):
+    """`masks` distinct flip masks of up to six sites, `per` Hermitian terms each."""
+    x = set()
+    while len(x) < masks:
+        x.add(sum(1 << int(s) for s in rng.choice(L, int(rng.integers(1, 7)), False)))
+    bits, co = [], []
+    for v in sorted(x):
+        for _ in range(per):
+            z = int(rng.integers(0, 1 << L)) & (~0 if row_bits else ~(3 << 6))
+            bits.append(sum((v >> s & 1) << (2 * s) | (z >> s & 1) << (2 * s + 1)
+                            for s in range(L)))
+            co.append(rng.standard_normal() * 1j ** bin(v & z).count("1"))
+    return np.array(bits, np.uint64), np.array(co, np.complex128)
+
+
+FREE, S, M, B = (0, 256), (12, 512), (12, 1024), (13, 1024)
+
+
+@pytest.mark.parametrize("mode,L,masks,per,want", [
+    # single terms: the tile by the list's length, the sums and the chain
+    ("c64", 20, 60, 1, M), ("c64", 22, 60, 1, S), ("c64", 22, 110, 1, M), ("c64", 23, 110, 1, S),
+    ("c64", 24, 240, 1, M), ("c64", 27, 240, 1, M), ("c64", 28, 240, 1, S),
+    ("group", 20, 60, 1, M), ("group", 21, 60, 1, S), ("group", 25, 60, 1, S),
+    ("group", 26, 60, 1, S), ("group", 26, 70, 1, B), ("group", 28, 60, 1, B),
+    ("c128", 20, 60, 1, S), ("native", 26, 60, 1, S),
+    # masks that share terms
+    ("c64", 26, 60, 3, M), ("c64", 28, 60, 3, M), ("group", 22, 60, 3, M), ("group", 28, 60, 3, M),
+    # few of them: without tiles, except where FP32 sums in tiles are cheaper
+    ("c64", 24, 20, 4, FREE), ("c128", 26, 40, 4, FREE), ("group", 22, 20, 4, M),
+    ("group", 22, 20, -4, FREE), ("native", 24, 20, 4, FREE), ("native", 24, 20, 20, FREE),
+    # two terms a mask and as many groups as masks
+    ("c64", 25, 10, 2, FREE), ("c64", 26, 10, 2, M), ("c128", 22, 10, 2, FREE),
+    ("c128", 23, 10, 2, S), ("group", 23, 10, 2, FREE), ("group", 23, 10, -2, FREE),
+    ("group", 25, 10, -2, M), ("group", 25, 10, 2, M),
+    ("c64", 26, 10, 1, S),
+    # 19 sites: many single-term masks with group accumulation
+    ("group", 19, 700, 1, M), ("group", 19, 300, 1, FREE), ("group", 19, 700, 2, FREE),
+    ("c64", 19, 700, 1, FREE)])
+def test_default_tilings(gpu, orc, mode, L, masks, per, want):
+    """The default layout's choice where it changes, and its apply against the
+    oracle where that is quick."""
+    rng = np.random.default_rng(7)
+    bits, co = _random(rng, L, masks, abs(per), per > 0)
+    flips = (1 << 2 * L) // 3      # the even bits
+    while per == 2 and L > 19 and len({int(b) & flips >> 24 << 24 for b in bits}) < masks:
+        bits, co = _random(rng, L, masks, 2)     # until every mask is a group of its own
+    dt = np.complex128 if mode == "c128" else np.complex64
+    if dt == np.complex64:
+        co = co.astype(np.complex64).astype(np.complex128)
+    t = Terms(L, bits, co, prec_of(dt), {"group": gpu.RP_TERMS_ACC_GROUP,
+                                         "native": gpu.RP_TERMS_ACC_NATIVE}.get(mode, 0))
     i = t.info()
-    want = {(64, False): (12, 512), (32, True): (12, 1024) if L == 20 else (13, 1024),
-            (32, False): (13, 1024) if L >= 27 else (12, 1024)}[fp, group]
-    assert (i.tile_bits, i.threads, i.depth) == want + (2,)
+    assert (i.tile_bits, i.threads) == want and (want == FREE or i.depth == 2)
+    if len(bits) << L > 1 << 29:
+        return
+    psi = random_state(rng, L, dt)
+    ref = orc.apply(L, bits, co, psi.astype(np.complex128), fp=64)
+    vin, out = DeviceBuffer.from_array(psi), DeviceBuffer(psi.nbytes)
+    gpu.check(gpu.hip().rp_apply_ops(t.h, out.ptr, vin.ptr, 0))
+    eps = 1.2e-7 if mode in ("group", "native") else 2.3e-16
+    tol = len(bits) * eps * np.abs(co).sum() * np.abs(psi).max() + \
+        (6e-8 if dt == np.complex64 else 1.2e-16) * np.abs(ref).max()
+    assert np.abs(out.to_array(dt, len(psi)).astype(np.complex128) - ref).max() <= tol
