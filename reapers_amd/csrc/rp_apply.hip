@@ -780,13 +780,26 @@ __device__ __forceinline__ uint32_t tile_index(const TileMap &tm)
     return t;
 }
 
+// The first amplitude of that tile, formed before the kernel looks at its stop
+// flag.  The tiled kernels take the flag's address before the map, so that
+// their arguments still fill three 64-byte lines: with the address behind the
+// map, and the flag looked at first, every workgroup waited for a fourth line,
+// 3 to 6 percent of an apply with few groups.
+template <int TB> __device__ __forceinline__ uint32_t first_amplitude(const TileMap &tm)
+{
+    uint32_t t0 = tile_index(tm) << TB;
+    asm volatile("" : "+s"(t0));
+    return t0;
+}
+
 template <typename R, typename A, int TB, int NT, int D, bool GA>
 __global__ void __launch_bounds__(NT, (apply_waves_per_eu<R, TB, NT, D>()))
 k_apply_tiled(const typename CxA<R>::T *__restrict__ in, typename CxA<R>::T *__restrict__ out,
-              const GroupRuns *__restrict__ groups, int ngroups, const SubRec<A> *__restrict__ subs,
-              const TermRec<A> *__restrict__ terms, int accumulate, TileMap tm,
-              const int *__restrict__ stop)
+              const GroupRuns *__restrict__ groups, int ngroups, int accumulate,
+              const SubRec<A> *__restrict__ subs, const TermRec<A> *__restrict__ terms,
+              const int *__restrict__ stop, TileMap tm)
 {
+    const uint32_t t0 = first_amplitude<TB>(tm);
     if (stop && *stop) return;
     using T = typename CxA<R>::T;
     constexpr int TILE = 1 << TB;
@@ -800,7 +813,7 @@ k_apply_tiled(const typename CxA<R>::T *__restrict__ in, typename CxA<R>::T *__r
     __shared__ T tile3[D > 3 ? TILE : 1];
     T wv[TILE / NT];
     apply_tile<R, A, TB, NT, D, GA>(in, out, groups, ngroups, subs, terms, accumulate, tile0, tile1,
-                                    tile2, tile3, tile_index(tm) << TB, wv);
+                                    tile2, tile3, t0, wv);
 }
 
 // ---------------------------------------------------------------------------
@@ -1095,15 +1108,15 @@ __device__ __forceinline__ void stream_tile(const float2 *__restrict__ in, float
 template <int TB, int NT>
 __global__ void __launch_bounds__(NT, (apply_waves_per_eu<float, TB, NT, 2>()))
 k_apply_stream(const float2 *__restrict__ in, float2 *__restrict__ out,
-               const GroupC *__restrict__ groups, int ngroups, const SubC *__restrict__ subs,
-               const TermC *__restrict__ terms, int accumulate, TileMap tm,
-              const int *__restrict__ stop)
+               const GroupC *__restrict__ groups, int ngroups, int accumulate,
+               const SubC *__restrict__ subs, const TermC *__restrict__ terms,
+               const int *__restrict__ stop, TileMap tm)
 {
+    const uint32_t t0 = first_amplitude<TB>(tm);
     if (stop && *stop) return;
     __shared__ float4 tile0[1 << (TB - 1)];
     __shared__ float4 tile1[1 << (TB - 1)];
-    stream_tile<TB, NT>(in, out, groups, ngroups, subs, terms, accumulate, tile_index(tm) << TB,
-                        tile0, tile1);
+    stream_tile<TB, NT>(in, out, groups, ngroups, subs, terms, accumulate, t0, tile0, tile1);
 }
 
 // ---------------------------------------------------------------------------
@@ -1202,16 +1215,17 @@ __device__ __forceinline__ void wide_run(uint32_t &s, uint32_t end, SubD &S,
 template <typename R, int TB, int NT>
 __global__ void __launch_bounds__(NT, (apply_waves_per_eu<R, TB, NT, 2>()))
 k_apply_wide(const typename CxA<R>::T *__restrict__ in, typename CxA<R>::T *__restrict__ out,
-             const GroupC *__restrict__ groups, int ngroups, const SubD *__restrict__ subs,
-             const TermRec<double> *__restrict__ terms, int accumulate, TileMap tm,
-              const int *__restrict__ stop)
+             const GroupC *__restrict__ groups, int ngroups, int accumulate,
+             const SubD *__restrict__ subs, const TermRec<double> *__restrict__ terms,
+             const int *__restrict__ stop, TileMap tm)
 {
     using T = typename CxA<R>::T;
     constexpr int RP = (1 << TB) / NT;
+    const uint32_t t0 = first_amplitude<TB>(tm);
     if (stop && *stop) return;
     __shared__ T tile0[1 << TB];
     __shared__ T tile1[1 << TB];
-    const uint32_t tid = threadIdx.x, t0 = tile_index(tm) << TB;
+    const uint32_t tid = threadIdx.x;
     const uint32_t lane = tid * (uint32_t)sizeof(T), lb = t0 | tid;
     double ar[RP], ai[RP];
 #pragma unroll
@@ -1870,15 +1884,15 @@ static int launch_tiled(rp_terms *h, void *res, const void *vec, int accumulate,
         if (h->group_acc && h->d_csubs) {
             RP_LAUNCH(RP_KERNEL_APPLY, (k_apply_stream<TB, NT>), dim3((unsigned)grid), dim3(NT), 0,
                       (const T *)vec, (T *)res, (const GroupC *)h->d_cgroups, (int)h->ngroups,
-                      (const SubC *)h->d_csubs, (const TermC *)h->d_cterms, accumulate, h->tmap,
-                      stop);
+                      accumulate, (const SubC *)h->d_csubs, (const TermC *)h->d_cterms, stop,
+                      h->tmap);
             return RP_OK;
         }
         if (h->group_acc) {
             RP_LAUNCH(RP_KERNEL_APPLY, (k_apply_tiled<R, A, TB, NT, D, true>), dim3((unsigned)grid),
                       dim3(NT), 0, (const T *)vec, (T *)res, (const GroupRuns *)h->d_groups,
-                      (int)h->ngroups, (const SubRec<A> *)h->d_subs,
-                      (const TermRec<A> *)h->d_terms, accumulate, h->tmap, stop);
+                      (int)h->ngroups, accumulate, (const SubRec<A> *)h->d_subs,
+                      (const TermRec<A> *)h->d_terms, stop, h->tmap);
             return RP_OK;
         }
     }
@@ -1886,15 +1900,15 @@ static int launch_tiled(rp_terms *h, void *res, const void *vec, int accumulate,
         if (h->d_csubs) {
             RP_LAUNCH(RP_KERNEL_APPLY, (k_apply_wide<R, TB, NT>), dim3((unsigned)grid), dim3(NT), 0,
                       (const T *)vec, (T *)res, (const GroupC *)h->d_cgroups, (int)h->ngroups,
-                      (const SubD *)h->d_csubs, (const TermRec<double> *)h->d_terms, accumulate,
-                      h->tmap, stop);
+                      accumulate, (const SubD *)h->d_csubs, (const TermRec<double> *)h->d_terms,
+                      stop, h->tmap);
             return RP_OK;
         }
     }
     RP_LAUNCH(RP_KERNEL_APPLY, (k_apply_tiled<R, A, TB, NT, D, false>), dim3((unsigned)grid),
               dim3(NT), 0, (const T *)vec, (T *)res, (const GroupRuns *)h->d_groups,
-              (int)h->ngroups, (const SubRec<A> *)h->d_subs, (const TermRec<A> *)h->d_terms,
-              accumulate, h->tmap, stop);
+              (int)h->ngroups, accumulate, (const SubRec<A> *)h->d_subs,
+              (const TermRec<A> *)h->d_terms, stop, h->tmap);
     return RP_OK;
 }
 
