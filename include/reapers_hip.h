@@ -169,11 +169,12 @@ int rp_terms_info(rp_terms_t h, rp_terms_info_t *info);
  * in the reference): tile bits / threads / pipeline depth must be one of the
  * instantiated combinations -- (8,128,2), (10,128,2), (12,512,2) for both
  * precisions; (12,512,3), (12,512,4), (12,1024,2), (13,1024,2) for RP_C64; (11,256,4) for
- * RP_C128 -- or, up to len 16, tile bits 0 with 256 threads: the kernel
- * without tiles, its depth the number of slices (1, 8, 32, 128) of the flip
- * masks that separate wavefronts sum.  The autotuner (RP_TERMS_AUTOTUNE)
- * chooses among the same set, the kernel without tiles up to len 18 and for
- * at most 40 flip masks. */
+ * RP_C128 -- or tile bits 0 with 256 threads: the kernel without tiles, its
+ * depth the number of slices (1, 8, 32, 128) of the flip masks that separate
+ * wavefronts sum; up to len 16 any of them, beyond only what an upload may
+ * choose itself: depth 1 and 8 up to len 19, depth 1 with at most 40 flip
+ * masks at any len.  So the tiling that rp_terms_info reports can be set
+ * again.  The autotuner (RP_TERMS_AUTOTUNE) chooses among the same set. */
 int rp_terms_set_tiling(rp_terms_t h, int tile_bits, int threads, int depth);
 
 /* GPUImpl::apply_ops + krnl_apply_ops (src/krnl.cu:220-257, 80-94):

@@ -1374,6 +1374,16 @@ constexpr TilingDesc kTilings[] = {
     {8, 128, 2, 0}, {10, 128, 2, 0}, {11, 256, 4, 16}, {12, 512, 2, 0},
     {12, 512, 3, 8}, {12, 512, 4, 8}, {12, 1024, 2, 8}, {13, 1024, 2, 8}};
 
+// Where the kernel without tiles may be set: up to kSplitMaxLen sites with any
+// slice count, and beyond in the shapes an upload chooses itself, which keep no
+// partial sums in memory (8 slices are added in LDS)
+static bool wave_allowed(int len, uint64_t flips, int depth)
+{
+    if (len <= kSplitMaxLen) return true;
+    return depth == 1 ? len <= kWaveMaxLen || flips <= (uint64_t)kWaveMaxFlips
+                      : depth == 8 && len <= kWaveMaxLen;
+}
+
 static bool tiling_instantiated(int prec, int tb, int nt, int d)
 {
     for (const TilingDesc &t : kTilings)
@@ -2086,9 +2096,8 @@ static int autotune(rp_terms *h)
     for (const TilingDesc &cd : kTilings) {
         if (st) break;
         if (cd.tb > h->len || !tiling_instantiated(h->prec, cd.tb, cd.nt, cd.depth)) continue;
-        if (cd.tb == 0 && (cd.depth == 1 ? h->len > kWaveMaxLen && h->nflips > kWaveMaxFlips
-                                         : h->len > (cd.depth == 8 ? kWaveMaxLen : kSplitMaxLen) ||
-                                               h->nterms < (uint64_t)(2 * cd.depth)))
+        if (cd.tb == 0 && (!wave_allowed(h->len, h->nflips, cd.depth) ||
+                           (cd.depth > 1 && h->nterms < (uint64_t)(2 * cd.depth))))
             continue;
         if ((st = retile(h, cd.tb, cd.nt, cd.depth))) break;
         if ((st = apply_dispatch(h, y, x, 0))) break;
@@ -2185,8 +2194,8 @@ int rp_terms_set_tiling(rp_terms_t h, int tile_bits, int threads, int depth)
     if (st) return st;
     RP_REQUIRE(h, "null term handle");
     RP_REQUIRE(tile_bits <= h->len, "tile bits exceed the chain length");
-    // the sliced kernel keeps depth / 4 * 2^len partial sums
-    RP_REQUIRE(tile_bits != 0 || h->len <= kSplitMaxLen, "tile bits 0 only up to len 16");
+    RP_REQUIRE(tile_bits != 0 || wave_allowed(h->len, h->nflips, depth),
+               "tile bits 0 only up to len 16, and where an upload may choose it");
     RP_REQUIRE(tiling_instantiated(h->prec, tile_bits, threads, depth),
                "tiling not instantiated for this precision");
     RP_CHECK_HIP(hipStreamSynchronize(ctx().stream));

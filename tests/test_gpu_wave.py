@@ -125,3 +125,31 @@ def test_masks_of_many_terms(gpu, orc, fp, native, L, masks, per, depth):
             gpu.check(gpu.hip().rp_terms_set_tiling(t.h, 0, 256, d))
         gpu.check(gpu.hip().rp_apply_ops(t.h, out.ptr, vin.ptr, 0))
         assert np.abs(out.to_array(dt, len(psi)).astype(np.complex128) - ref).max() <= tol, d
+
+
+@pytest.mark.parametrize("L,masks", [(17, 12), (18, 40), (19, 60), (20, 16), (22, 30)])
+def test_reported_tiling_can_be_set_again(gpu, L, masks):
+    """A program that tries other tilings goes back to the one it was given;
+    what no upload chooses is refused."""
+    rng = np.random.default_rng(L)
+    bits, co = _terms(rng, L, masks, 32)
+    dt = np.complex64
+    t = Terms(L, bits, co, prec_of(dt))
+    i = t.info()
+    first = (i.tile_bits, i.threads, i.depth)
+    assert first[0] == 0
+    psi = random_state(rng, L, dt)
+    vin, out = DeviceBuffer.from_array(psi), DeviceBuffer(psi.nbytes)
+    gpu.check(gpu.hip().rp_apply_ops(t.h, out.ptr, vin.ptr, 0))
+    want = out.to_array(dt, len(psi))
+    gpu.check(gpu.hip().rp_terms_set_tiling(t.h, 12, 512, 2))
+    gpu.check(gpu.hip().rp_terms_set_tiling(t.h, *first))
+    i = t.info()
+    assert (i.tile_bits, i.threads, i.depth) == first
+    gpu.check(gpu.hip().rp_apply_ops(t.h, out.ptr, vin.ptr, 0))
+    assert np.array_equal(out.to_array(dt, len(psi)), want)
+    for d in (32, 128) + ((8,) if L > 19 else ()):
+        assert gpu.hip().rp_terms_set_tiling(t.h, 0, 256, d) != 0
+    many, c = _terms(rng, L, 80, 32)
+    u = Terms(L, many, c, prec_of(dt))
+    assert (gpu.hip().rp_terms_set_tiling(u.h, 0, 256, 1) == 0) == (L <= 19)
