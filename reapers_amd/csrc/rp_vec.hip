@@ -543,16 +543,6 @@ static double *vec_scratch(int device)
     return g_scratch_ptr[device];
 }
 
-// workgroups of a sweep: one element per thread up to 2^16 elements, then
-// four, so that a row of dot partials stays short; at most kRedBlocks
-static inline int red_blocks(uint64_t n)
-{
-    const uint64_t one = (n + kRedThreads - 1) / kRedThreads;
-    if (one <= 256) return (int)(one < 1 ? 1 : one);
-    const uint64_t four = (n + 4 * kRedThreads - 1) / (4 * kRedThreads);
-    return (int)(four < 256 ? 256 : four > (uint64_t)kRedBlocks ? kRedBlocks : four);
-}
-
 // wait for the queued kernels: their results are then in pinned host memory
 static int wait_results()
 {
@@ -576,7 +566,10 @@ static int wait_results()
 
 // queue the dots of w against V[0..k) and ||w||^2 (k = 0: only that).  Each
 // workgroup takes up to 8 vectors (w is read once for all of them), 4 where
-// the vectors are so short that more workgroups matter more.
+// the vectors are so short that more workgroups matter more.  At most
+// kDotBlocks of them, of 1024 threads where 256 would each walk too many
+// elements in series: from 2^19, with one or two vectors from 2^17 (2^19
+// complex<double> elements: a dot product 19.2 -> 18.5 us with its wait).
 template <typename R>
 static int dots_launch(int cls, const VecPtrs &P, int k, const void *w, uint64_t n, double *work,
                        int real, double *host, const int *stop)
@@ -585,7 +578,7 @@ static int dots_launch(int cls, const VecPtrs &P, int k, const void *w, uint64_t
     const int most = n <= (1u << 15) ? kDotChunk / 2 : kDotChunk;
     const int rows = k > 0 ? (k + most - 1) / most : 1;
     const int kc = (k + rows - 1) / rows;
-    const int nt = n <= (1u << 19) ? 256 : 1024;
+    const int nt = n <= (kc <= 2 ? 1u << 17 : 1u << 19) ? 256 : 1024;
     const dim3 grid((unsigned)std::min<uint64_t>((n + nt - 1) / nt, kDotBlocks), rows);
     double *res = work + kPartDoubles;
 #define RP_DOTS(KC)                                                               \
@@ -617,7 +610,7 @@ static int update_launch(const VecPtrs &P, int k, void *w, uint64_t n, double *w
                          double fuse_min, int scale, double min_norm, int *stop, int step)
 {
     using T = typename Cx<R>::T;
-    const int nb = red_blocks(n), kr = (k - 1) % kUpdChunk + 1;
+    const int nb = grid_for(n, kRedThreads, kRedBlocks), kr = (k - 1) % kUpdChunk + 1;
     double *res = work + kPartDoubles;
 #define RP_UPD(KR)                                                                \
     RP_LAUNCH(RP_KERNEL_GS, (k_gs_update<R, KR, false>), dim3(nb), dim3(kRedThreads), 0, P, k,     \
@@ -745,7 +738,7 @@ template <typename R>
 static int lincomb_impl(void *y, const void *const *V, int k, const double *c, uint64_t n)
 {
     using T = typename Cx<R>::T;
-    const int nb = red_blocks(n);
+    const int nb = grid_for(n, kRedThreads, kRedBlocks);
     for (int q0 = 0; q0 < k; q0 += kMaxVecs) {
         const int kc = k - q0 < kMaxVecs ? k - q0 : kMaxVecs, kr = (kc - 1) % kUpdChunk + 1;
         VecPtrs P{};

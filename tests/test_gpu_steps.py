@@ -206,11 +206,14 @@ def test_lanczos_steps(gpu, length, m):
 
 @pytest.mark.parametrize("dtype", [np.complex64, np.complex128])
 @pytest.mark.parametrize("n,k", [(1, 1), (63, 3), (256, 4), (257, 5), (32768, 17), (32769, 9),
-                                 (65536, 8), (65537, 16), (262143, 33), (300001, 2), (4096, 64)])
+                                 (65536, 8), (65537, 16), (262143, 33), (300001, 2), (4096, 64),
+                                 (131072, 2), (131073, 1), (131073, 3), (524288, 5), (524289, 3),
+                                 (524289, 17), (1048577, 1)])
 def test_gs_pass_edges(gpu, dtype, n, k):
-    """One pass at the sizes where the launch shape changes (workgroup size
-    at 2^16 elements, vectors per workgroup at 2^15, chunks of 16 in the
-    update), twice in a row on the same workspace."""
+    """One pass at the sizes where the launch shape changes (the dots' 256 or
+    1024 threads at 2^17 elements for one or two vectors a workgroup, at 2^19
+    for more; vectors per workgroup at 2^15; chunks of 16 in the update), twice
+    in a row on the same workspace."""
     rng = np.random.default_rng(n + k)
     V = (rng.standard_normal((k, n)) + 1j * rng.standard_normal((k, n))) / np.sqrt(2 * n * k)
     V = V.astype(dtype)
