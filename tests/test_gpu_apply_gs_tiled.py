@@ -19,8 +19,9 @@ _vp = ctypes.c_void_p
 
 
 @pytest.mark.parametrize("flags", [0, 4])
-@pytest.mark.parametrize("k", [1, 8, 9, 17])
-def test_apply_gs_on_its_tiling(gpu, orc, flags, k):
+@pytest.mark.parametrize("k,fuse_min", [(1, 0.0), (8, 0.0), (9, 0.0), (17, 0.0), (1, 0.25),
+                                        (9, 0.25), (9, 1e6)])
+def test_apply_gs_on_its_tiling(gpu, orc, flags, k, fuse_min):
     L, n = 14, 1 << 14
     rng = np.random.default_rng(10 * k + flags)
     bits, coeff = orc.syk_terms(2 * L, 8.0, seed=92, fp=32)
@@ -34,7 +35,7 @@ def test_apply_gs_on_its_tiling(gpu, orc, flags, k):
     h = np.zeros(2 * k)
     norm, nz = ctypes.c_double(), ctypes.c_int()
     gpu.check(gpu.hip().rp_apply_gs(t.h, out.ptr, V[-1].ptr, (_vp * k)(*[b.ptr.value for b in V]), k,
-                                    h.ctypes.data_as(_vp), ctypes.byref(norm), 0.0,
+                                    h.ctypes.data_as(_vp), ctypes.byref(norm), fuse_min,
                                     ctypes.byref(nz)))
     h = h.view(np.complex128)
     w = out.to_array(np.complex64, n).astype(np.complex128)
@@ -46,6 +47,9 @@ def test_apply_gs_on_its_tiling(gpu, orc, flags, k):
     err = (1.2e-7 * len(bits) ** 0.5 * np.abs(coeff).sum() if flags else 0.0) \
         + 1.2e-7 * np.linalg.norm(hv)
     beta = norm.value
+    # normalized where the norm is large enough and free of cancellation
+    assert nz.value == (0 < fuse_min <= np.linalg.norm(r) and
+                        np.linalg.norm(r) ** 2 >= np.linalg.norm(hv) ** 2 / 2)
     if nz.value:
         w *= beta
     print("flags %d k %d: |dh| %.1e (bound %.1e), |dw| %.1e" % (

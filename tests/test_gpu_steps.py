@@ -31,69 +31,58 @@ def _hermitian(rng, length, nterms):
     return bits, np.array(co)
 
 
-def _dense(length, bits, coeff):
-    n = 1 << length
-    m = np.zeros((n, n), np.complex128)
-    i = np.arange(n)
-    for b, c in zip(bits, coeff):
-        x = sum(((int(b) >> (2 * s)) & 1) << s for s in range(length))
-        z = sum(((int(b) >> (2 * s + 1)) & 1) << s for s in range(length))
-        sign = np.array([(-1) ** bin(v & z).count("1") for v in range(n)])
-        m[i ^ x, i] += c * sign
-    return m
-
-
-def _arnoldi(H, v, m):
-    V, h = [v], np.zeros((m + 1, m), np.complex128)
-    for j in range(m):
-        w = H @ V[j]
-        c = np.array([np.vdot(u, w) for u in V])
-        w = w - sum(a * u for a, u in zip(c, V))
-        h[:j + 1, j] = c
-        h[j + 1, j] = np.linalg.norm(w)
-        V.append(w / h[j + 1, j])
-    return V, h
-
-
 def _ptrs(bufs):
     return (_vp * len(bufs))(*[b.ptr.value for b in bufs])
 
 
-@pytest.mark.parametrize("dtype", [np.complex64, np.complex128])
-@pytest.mark.parametrize("length,m,j0", [(2, 2, 0), (5, 9, 0), (9, 19, 0), (9, 6, 2), (10, 34, 0)])
-def test_arnoldi_steps(gpu, dtype, length, m, j0):
-    rng = np.random.default_rng(100 * length + m)
+def _case(rng, dtype, length):
+    """A Hermitian list, the bound sum |c| of its norm and a normalized vector."""
     bits, co = _hermitian(rng, length, 6 * length)
     if dtype == np.complex64:
-        co = co.real.astype(np.float32).astype(float) + 1j * co.imag.astype(np.float32).astype(float)
+        co = co.astype(np.complex64).astype(np.complex128)
+    v = rng.standard_normal(1 << length) + 1j * rng.standard_normal(1 << length)
+    return bits, co, np.abs(co).sum(), (v / np.linalg.norm(v)).astype(dtype)
+
+
+# Each step is checked from the vectors on the device, by what it leaves of
+# H V[j] = sum_i h_i V[i] + norm V[j+1]: the product is rounded once when it
+# is stored (EPS ||H||), the coefficients are FP64 sums over the stored
+# vector, and the update and the division round once more each.  The bound
+# does not grow with j.
+@pytest.mark.parametrize("dtype", [np.complex64, np.complex128])
+@pytest.mark.parametrize("length,m,j0", [(2, 2, 0), (5, 9, 0), (9, 19, 0), (9, 6, 2), (10, 34, 0),
+                                         (14, 10, 0), (17, 4, 0), (18, 9, 0), (20, 4, 1)])
+def test_arnoldi_steps(gpu, orc, dtype, length, m, j0):
+    rng = np.random.default_rng(100 * length + m)
     n = 1 << length
-    H, hnorm = _dense(length, bits, co), np.abs(co).sum()     # ||H|| <= sum |c|
-    v = rng.standard_normal(n) + 1j * rng.standard_normal(n)
-    V, h = _arnoldi(H, v / np.linalg.norm(v), m)
+    bits, co, hnorm, v = _case(rng, dtype, length)
     t = Terms(length, bits, co, prec_of(dtype))
-    bufs = [DeviceBuffer.from_array((V[j] if j <= j0 else np.zeros(n)).astype(dtype))
-            for j in range(m + 1)]
-    out, done = np.zeros((m - j0, STEP)), ctypes.c_int()
-    gpu.check(gpu.hip().rp_arnoldi_steps(t.h, _ptrs(bufs), j0, m, 1e-3,
-                                         out.ctypes.data_as(_vp), ctypes.byref(done)))
+    bufs = [DeviceBuffer.from_array(v if j == 0 else np.zeros(n, dtype)) for j in range(m + 1)]
+    out, done = np.zeros((m, STEP)), ctypes.c_int()
+    if j0:      # the first steps by a call of their own
+        gpu.check(gpu.hip().rp_arnoldi_steps(t.h, _ptrs(bufs[:j0 + 1]), 0, j0, 1e-3,
+                                             out.ctypes.data_as(_vp), ctypes.byref(done)))
+        assert done.value == j0
+    gpu.check(gpu.hip().rp_arnoldi_steps(t.h, _ptrs(bufs), j0, m, 1e-3, out[j0:].ctypes.data_as(_vp),
+                                         ctypes.byref(done)))
     assert done.value == m - j0
-    # one rounding per stored component, carried through the recurrence: each
-    # step multiplies the error of the last by about ||H|| / H(j+1, j)
-    grow = np.cumprod([max(1.0, hnorm / abs(h[j + 1, j])) for j in range(m)])
-    for j in range(j0, m):
-        o = out[j - j0]
-        tol = 8 * EPS[dtype] * grow[j]
+    V = [b.to_array(dtype, n).astype(np.complex128) for b in bufs]
+    tol = 4 * EPS[dtype] * hnorm
+    for j in range(m):
+        o = out[j]
         got = o[0:2 * j + 2:2] + 1j * o[1:2 * j + 2:2]
-        assert np.abs(got - h[:j + 1, j]).max() <= tol * hnorm
-        assert abs(o[128] - h[j + 1, j]) <= tol * hnorm
+        w = orc.apply(length, bits, co, V[j])
+        assert np.abs(got - [np.vdot(u, w) for u in V[:j + 1]]).max() <= tol, j
+        rest = w - sum(a * u for a, u in zip(got, V))
+        assert np.linalg.norm(rest - o[128] * V[j + 1]) <= tol, j
         assert o[129] in (0.0, 1.0)
-        got = bufs[j + 1].to_array(dtype, n)
-        assert np.linalg.norm(got - V[j + 1]) <= tol
         # the norm divided by: an FP64 sum of n squares, its terms' roundings
         # adding up as sqrt(n) (beta^2 = ||w||^2 - sum |h|^2 at most doubles
-        # them); then one rounding per component
-        unit = 4 * EPS[dtype] + 2.2e-16 * np.sqrt(n)
-        assert abs(np.linalg.norm(got.astype(np.complex128)) - 1) <= unit
+        # them), of a basis that is orthonormal to its own roundings; then one
+        # rounding per component
+        unit = 4 * EPS[dtype] + 2.2e-16 * np.sqrt(n) + 2 * (j + 1) * EPS[dtype] ** 2 * hnorm ** 2
+        if not o[129]:
+            assert abs(np.linalg.norm(V[j + 1]) - 1) <= unit, j
 
 
 @pytest.mark.parametrize("dtype", [np.complex64, np.complex128])
@@ -176,32 +165,28 @@ def test_arnoldi_steps_without_terms(gpu, dtype, length):
     assert not bufs[2].to_array(dtype, n).any()
 
 
-@pytest.mark.parametrize("length,m", [(3, 1), (3, 2), (8, 12), (10, 30)])
-def test_lanczos_steps(gpu, length, m):
+@pytest.mark.parametrize("dtype", [np.complex64, np.complex128])
+@pytest.mark.parametrize("length,m", [(3, 1), (3, 2), (8, 12), (10, 30), (18, 5)])
+def test_lanczos_steps(gpu, orc, dtype, length, m):
     rng = np.random.default_rng(length)
-    bits, co = _hermitian(rng, length, 4 * length)
     n = 1 << length
-    H, hnorm = _dense(length, bits, co), np.abs(co).sum()     # ||H|| <= sum |c|
-    v = rng.standard_normal(n) + 1j * rng.standard_normal(n)
-    V, al, be = [v / np.linalg.norm(v)], [], []
-    for i in range(m):
-        w = H @ V[i]
-        al.append(np.vdot(V[i], w).real)
-        if i == m - 1:
-            break
-        w = w - al[i] * V[i] - (be[i - 1] * V[i - 1] if i else 0)
-        be.append(np.linalg.norm(w))
-        V.append(w / be[i])
-    t = Terms(length, bits, co, gpu.RP_C128)
-    bufs = [DeviceBuffer.from_array(V[0] if j == 0 else np.zeros(n, np.complex128))
-            for j in range(m + 1)]
+    bits, co, hnorm, v = _case(rng, dtype, length)
+    t = Terms(length, bits, co, prec_of(dtype))
+    bufs = [DeviceBuffer.from_array(v if j == 0 else np.zeros(n, dtype)) for j in range(m + 1)]
     a, b = np.zeros(m), np.zeros(max(1, m - 1))
     gpu.check(gpu.hip().rp_lanczos_steps(t.h, _ptrs(bufs), m, a.ctypes.data_as(_vp),
                                          b.ctypes.data_as(_vp)))
-    grow = np.cumprod([max(1.0, hnorm / x) for x in be] or [1.0])[-1]
-    tol = 16 * 1.2e-16 * grow * hnorm
-    assert np.abs(a - al).max() <= tol
-    assert np.abs(b[:m - 1] - be).max() <= tol if m > 1 else True
+    V = [b.to_array(dtype, n).astype(np.complex128) for b in bufs]
+    tol = 4 * EPS[dtype] * hnorm       # as for the Arnoldi steps
+    for j in range(m):
+        w = orc.apply(length, bits, co, V[j])
+        assert abs(a[j] - np.vdot(V[j], w).real) <= tol, j
+        if j == m - 1:
+            assert np.linalg.norm(V[m] - w) <= tol
+            break
+        rest = w - a[j] * V[j] - (b[j - 1] * V[j - 1] if j else 0)
+        assert np.linalg.norm(rest - b[j] * V[j + 1]) <= tol, j
+        assert b[j] > 0 and abs(np.linalg.norm(V[j + 1]) - 1) <= 4 * EPS[dtype] + 2.2e-16 * np.sqrt(n)
 
 
 @pytest.mark.parametrize("dtype", [np.complex64, np.complex128])

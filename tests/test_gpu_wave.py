@@ -6,6 +6,8 @@ lane, the row and the remaining index bits.
 
 Tolerance: FP64 sums of the terms (n of them, each off by at most
 eps64 |c v|) and one rounding to the state's precision."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -13,6 +15,8 @@ from conftest import random_state
 from gpu_util import DeviceBuffer, Terms, prec_of
 
 pytestmark = pytest.mark.gpu
+
+_vp = ctypes.c_void_p
 
 
 def _terms(rng, L, masks, fp):
@@ -153,3 +157,48 @@ def test_reported_tiling_can_be_set_again(gpu, L, masks):
     many, c = _terms(rng, L, 80, 32)
     u = Terms(L, many, c, prec_of(dt))
     assert (gpu.hip().rp_terms_set_tiling(u.h, 0, 256, 1) == 0) == (L <= 19)
+
+
+@pytest.mark.parametrize("fp,L", [(32, 28), (32, 29), (64, 27), (64, 28)])
+def test_states_around_4_gib(gpu, fp, L):
+    """The chain with two- and many-term masks that takes no tiles at any
+    length, on both sides of the state size from which the gathers need 64-bit
+    offsets: windows of rows at the ends, the middle and at random."""
+    rng = np.random.default_rng(L + fp)
+    dt, es = (np.complex64, 8) if fp == 32 else (np.complex128, 16)
+    pair = [3 << i for i in range(L - 1)]
+    x = np.array(pair + pair + [0] * (2 * L - 1))
+    z = np.array([0] * (L - 1) + pair + pair + [1 << i for i in range(L)])
+    bits = np.zeros(len(x), np.uint64)
+    for s in range(L):
+        bits |= ((x >> s & 1) << (2 * s) | (z >> s & 1) << (2 * s + 1)).astype(np.uint64)
+    co = rng.standard_normal(len(x)) + 0j
+    if fp == 32:
+        co = co.astype(np.complex64).astype(np.complex128)
+    t = Terms(L, bits, co, prec_of(dt))
+    assert t.info().kernel == gpu.RP_APPLY_SMALL
+    hip, n = gpu.hip(), 1 << L
+    vin, out = DeviceBuffer(es << L), DeviceBuffer(es << L)
+    gpu.check(hip.rp_init_random(prec_of(dt), vin.ptr, n, 3))
+    gpu.check(hip.rp_apply_ops(t.h, out.ptr, vin.ptr, 0))
+
+    def window(buf, lo):
+        a = np.empty(64, dt)
+        gpu.check(hip.rp_memcpy(a.ctypes.data_as(_vp), _vp(buf.ptr.value + lo * es), a.nbytes,
+                                gpu.RP_D2H))
+        return a.astype(np.complex128)
+
+    for lo in [0, n // 2 - 64, n // 2, n - 64] + [int(v) * 64 for v in rng.integers(0, n // 64, 4)]:
+        m = np.arange(lo, lo + 64)
+        ref, size = np.zeros(64, np.complex128), 0.0
+        for xv in np.unique(x):
+            v = window(vin, (lo ^ int(xv)) & ~63)[(m ^ int(xv)) & 63]
+            size = max(size, np.abs(v).max())
+            for c, zv in zip(co[x == xv], z[x == xv]):
+                par = np.array([bin(int(q) & int(zv)).count("1") & 1 for q in m ^ int(xv)])
+                ref += c * (1 - 2 * par) * v
+        tol = len(co) * 2.3e-16 * np.abs(co).sum() * size + (6e-8 if fp == 32 else 1.2e-16) * \
+            np.abs(ref).max()
+        assert np.abs(window(out, lo) - ref).max() <= tol, lo
+    for b in (vin, out):
+        b.free()
