@@ -78,7 +78,7 @@ def apply_kernel_name(info):
     if info.kernel == ra.RP_APPLY_STREAM:
         return "k_apply_stream<b=%d,threads=%d>" % (info.tile_bits, info.threads)
     if info.kernel == ra.RP_APPLY_SMALL:
-        return "k_apply_small"
+        return "k_apply_wave"
     return "k_apply_tiled<%s,b=%d,threads=%d,depth=%d>" % (
         "float" if info.prec == ra.RP_C64 else "double", info.tile_bits, info.threads,
         info.depth)

@@ -159,8 +159,9 @@ typedef struct {
                                groups by flip mask) */
 } rp_terms_info_t;
 /* the apply kernel family a term handle launches: one wavefront per 64 or 256
-   amplitudes and slice of the flip masks (tile_bits 0); tiles with per-sub records; tiles with the compact sub
-   stream (complex<float>, group accumulation, two LDS tiles) */
+   amplitudes and slice of the flip masks (tile_bits 0); tiles with a record
+   per sub (48 bytes, or 16 where FP64 sums run over long lists); tiles with
+   the compact sub stream (complex<float>, group accumulation, two LDS tiles) */
 #define RP_APPLY_SMALL  0
 #define RP_APPLY_TILED  1
 #define RP_APPLY_STREAM 2
@@ -189,7 +190,8 @@ int rp_apply_ops(rp_terms_t h, void *res, const void *vec, int accumulate);
  * per basis vector, inc/algo.h:86-101 and 160): res = H vec, then the pass of
  * rp_gs_pass_fused over V[0..k) (k <= 64) on res.  Where the handle's layout
  * allows (complex<float> states with FP64 or group accumulation, 2^12-
- * amplitude tiles of 512 threads, up to 2^28 amplitudes) the coefficients
+ * amplitude tiles of 512 threads, up to 2^28 amplitudes; the default tiling
+ * only for some lists, see rp_terms_set_tiling) the coefficients
  * <V_q|res> and ||res||^2 are formed in the apply kernel from the values it
  * writes, saving the pass's separate read of res; otherwise this is
  * rp_apply_ops followed by rp_gs_pass_fused.  res must differ from vec and
@@ -249,7 +251,7 @@ int rp_arnoldi_steps(rp_terms_t h, void *const *V, int j0, int m, double min_nor
  * and, but for the last, V[j+1] -= alpha[j] V[j] + beta[j-1] V[j-1], beta[j] =
  * ||V[j+1]||, V[j+1] /= beta[j].  V[0] is normalized; beta holds m - 1. */
 int rp_lanczos_steps(rp_terms_t h, void *const *V, int m, double *alpha, double *beta);
-/* y += sum_i c[i] V[i] for k vectors (any k; one sweep per 16 of them), c
+/* y += sum_i c[i] V[i] for k vectors (any k; one sweep per 64 of them), c
    given as 2k doubles (re, im) */
 int rp_lincomb(int prec, void *y, const void *const *V, int k, const double *c, uint64_t n);
 

@@ -19,10 +19,10 @@
 // the kernel spends 2 FMAs (not 4) per term and amplitude on the first two.
 //
 // Tiled kernel: one workgroup of NT threads owns the output tile
-// [t0, t0 + 2^b); thread tid holds amplitudes t0 + r*NT + tid, r < RP.  For
-// each group it stages the input tile t0 ^ (xh << b) in LDS with coalesced
-// loads (an XOR with the high part maps an aligned tile onto an aligned
-// tile), then applies every sub of the group from LDS: the low bits of x
+// [t0, t0 + 2^b); thread tid holds amplitudes t0 + r*NT + tid, r < RP (in
+// k_apply_stream pairs of neighbours, see stream_row).  For each group it stages
+// the input tile t0 ^ (xh << b) in LDS with coalesced loads (an XOR with the
+// high part maps an aligned tile onto an aligned tile), then applies every sub of the group from LDS: the low bits of x
 // permute lanes (tid ^ (x mod NT)) and rows (r ^ (x / NT)).  The sign
 // (-1)^popcount(m & z) splits into a per-workgroup part (t0 & z), a per-lane
 // part (tid & z) computed once per sub, and a per-row part (r*NT & z) that is
@@ -1367,7 +1367,7 @@ constexpr int tiling_key(int tb, int nt, int d) { return tb * 100000 + nt * 10 +
 // pipeline depth, element bytes (0: both precisions)}
 struct TilingDesc { int tb, nt, depth, esz; };
 // Tile bits 0 is the kernel without tiles, its depth the number of term slices.
-constexpr int kSplitMaxLen = 16;       // rp_terms_set_tiling takes it up to here
+constexpr int kSplitMaxLen = 16;       // with any slice count up to here
 constexpr TilingDesc kTilings[] = {
     {0, kSmallThreads, 1, 0}, {0, kSmallThreads, 8, 0}, {0, kSmallThreads, 32, 0},
     {0, kSmallThreads, 128, 0},
@@ -2112,7 +2112,6 @@ static int autotune(rp_terms *h)
         if (ms < best) { best = ms; pick = cd; }
     }
     // the kept tiling's apply against one streaming pass of the same vector
-    // (3 scalings of x, each reading and writing it: 6 passes)
     // (3 scalings of x, each reading and writing it: 6 passes); a failure
     // here leaves the figure at 0 and the upload as it is
     if (!st && best < 1e30f) {

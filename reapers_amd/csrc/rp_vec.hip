@@ -7,7 +7,8 @@
 // All kernels are memory-bound streams with grid-stride loops.  Reductions
 // keep FP64 partial sums per thread, reduce them within a wavefront with
 // cross-lane shuffles, across the workgroup in LDS, and across workgroups in
-// a second small kernel, so every reduction is deterministic for a given n.
+// the last workgroup to arrive, in an order of its own, so every reduction is
+// deterministic for a given n.
 #include "rp_internal.h"
 
 #include <algorithm>
@@ -514,7 +515,7 @@ static inline double *ws_result() { return ws_partial() + kPartDoubles; }
 
 // The Gram-Schmidt pass's workspace in a file-scope device array, for
 // rp_gs_pass_fused_noalloc: the partials and results of the library
-// workspace layout above, 1.06 MB.  Each device holds its own copy; the
+// workspace layout above, 1.08 MB.  Each device holds its own copy; the
 // host reaches it only through the address hipGetSymbolAddress returns for
 // the current device (taken once per device at rp_init).
 static __device__ __align__(256) double scratch[kPartDoubles + kResDoubles];

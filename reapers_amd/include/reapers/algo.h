@@ -79,9 +79,10 @@ class Krylov {
         const size_t dim = s.dim();
         const auto len = s.spin_chain_length();
         // With the selective criterion nearly every step ends after one
-        // pass.  A backend that can queues all steps on that assumption and
-        // waits once; the step that needs another pass is the last of them,
-        // gets it here, and the rest go one by one.
+        // pass.  A backend that can queues all steps of this call on that
+        // assumption and waits once (a restart makes two calls: step 0, which
+        // a schedule looks at, and the others); the step that needs another
+        // pass is the last of them, gets it here, and the rest go one by one.
         int j = j0;
         if constexpr (requires(std::vector<const typename Impl::template VecType<FpType> *> &V,
                                std::vector<typename Impl::ArnoldiStep> &q) {

@@ -115,11 +115,11 @@ def test_krylov_with_fused_first_pass_vs_oracle(gpu, orc):
     psi = s.store()
     prev = gpu.set_fused_first_pass(True)
     try:
-        st = s.evolve(H, 2.0, 0.0, krydim=16, tol=1e-7)
+        st = s.evolve(H, 1.0, 0.0, krydim=12, tol=1e-7)
     finally:
         gpu.set_fused_first_pass(prev)
     got = s.store().astype(np.complex128)
-    ref, _ = orc.krylov_evolve(L, bits, coeff, psi.astype(np.complex128), 2.0, 0.0, krydim=16,
+    ref, _ = orc.krylov_evolve(L, bits, coeff, psi.astype(np.complex128), 1.0, 0.0, krydim=12,
                                tol=1e-12)
     err = np.linalg.norm(got - ref) / np.linalg.norm(ref)
     print("N=42 FP32 evolution with the fused pass: %d matvecs, rel err %.2e" % (st.matvecs, err),
