@@ -191,26 +191,28 @@ template <typename T, typename A, int ROWS>
 __device__ __forceinline__ void add_rows(const A (&d)[ROWS], const T (&v)[ROWS], bool imag,
                                          A (&ar)[ROWS], A (&ai)[ROWS])
 {
-    // the components as values first: sunk below the branch, their loads from
-    // v became one load at a chosen address, and v an array in scratch memory
-    A x[ROWS], y[ROWS];
-#pragma unroll
-    for (int r = 0; r < ROWS; r++) {
-        x[r] = v[r].x;
-        y[r] = v[r].y;
-        if constexpr (ROWS == 1 && sizeof(A) == 4) asm volatile("" : "+v"(x[r]), "+v"(y[r]));
+    if constexpr (ROWS == 1 && sizeof(A) == 4) {
+        // the components as values first: sunk below the branch, their loads
+        // from v became one load at a chosen address, and v an array in scratch
+        // memory.  (With more rows or FP64 sums it costs registers instead:
+        // 79 against 68, and the occupancy that hides the gathers.)
+        A x = v[0].x, y = v[0].y;
+        asm volatile("" : "+v"(x), "+v"(y));
+        ar[0] = fma(imag ? -d[0] : d[0], imag ? y : x, ar[0]);
+        ai[0] = fma(d[0], imag ? x : y, ai[0]);
+        return;
     }
     if (!imag) {
 #pragma unroll
         for (int r = 0; r < ROWS; r++) {
-            ar[r] = fma(d[r], x[r], ar[r]);
-            ai[r] = fma(d[r], y[r], ai[r]);
+            ar[r] = fma(d[r], (A)v[r].x, ar[r]);
+            ai[r] = fma(d[r], (A)v[r].y, ai[r]);
         }
     } else {
 #pragma unroll
         for (int r = 0; r < ROWS; r++) {
-            ar[r] = fma(-d[r], y[r], ar[r]);
-            ai[r] = fma(d[r], x[r], ai[r]);
+            ar[r] = fma(-d[r], (A)v[r].y, ar[r]);
+            ai[r] = fma(d[r], (A)v[r].x, ai[r]);
         }
     }
 }
@@ -1442,13 +1444,15 @@ static bool long_list(int len, uint64_t flips, uint64_t shared)
 // Amplitudes per lane of the kernel without tiles: four where that leaves
 // enough wavefronts.  Every term's sign and record is then shared by four
 // amplitudes, and the scalar instructions of a flip mask (about 35), which
-// bound the lists of many masks, by 256 instead of 64.
+// bound the lists of many masks, by 256 instead of 64.  At 12 sites one
+// amplitude a lane has 8192 wavefronts in 128 slices, four have 2048: 1000
+// masks 9.1 / 10.2 us, 600 masks of 4 terms 14.1 / 13.4.
 static int wave_rows(int len, int depth, uint64_t pieces, uint64_t nterms)
 {
     if (len > kSplitMaxLen || depth == 1)
         return depth <= 8 && ((uint64_t)depth << len) >= (1ull << 20) ? 4 : 1;
     return len > 8 && ((uint64_t)depth << (len - 8)) >= 2048 &&
-                   pieces + nterms >= (uint64_t)(10 * depth)
+                   pieces + nterms >= (uint64_t)((len == 12 ? 20 : 10) * depth)
                ? 4 : 1;
 }
 
@@ -1516,8 +1520,10 @@ static int wave_depth(int len, uint64_t pieces, uint64_t nterms, int acc64)
 //     sites 20/15 2516 / 2034, XY chain 26/15 2223 / 2454
 //   group accumulation: 22 sites 20/18 58 / 71, 40/20 116 / 106, XY chain
 //     21/11 46 / 62; 24 sites 10/9 158 / 141, XY chain 23/13 186 / 235
+//   FP32 sums: 20 sites 40/21 34 / 48, 23 sites 40/20 175 / 196, 24 sites 10/9
+//     154 / 132, 25 sites 40/32 972 / 840, XY chain 24/14 448 / 472
 //   complex<double>: 22 sites 40/28 194 / 243, 23 sites 40/28 465 / 449, 26
-//     sites 40/30 4252 / 3666, XY chain 25/15 1885 / 2640
+//     sites 40/30 4252 / 3666, 20/14 1518 / 1877, XY chain 25/15 1885 / 2640
 static bool without_tiles(int prec, int len, const ListShape &L, int group_acc, int acc64)
 {
     const bool single = 2 * L.terms < 3 * L.flips;
@@ -1525,14 +1531,16 @@ static bool without_tiles(int prec, int len, const ListShape &L, int group_acc, 
         return !(len == kWaveMaxLen && group_acc && single && L.flips >= 600 && L.flips <= 8192);
     if (L.flips > kWaveMaxFlips || L.terms < 2 * L.flips) return false;
     const bool fp32 = prec == RP_C64 && (group_acc || !acc64), rows = 4 * L.by_row > L.terms;
+    const double per = (double)L.flips / (double)L.groups;      // masks a group
     if (2 * L.terms < 5 * L.flips) {      // two terms a mask
-        if (fp32 && rows) return len < 24 && 2 * L.flips < 3 * L.groups;
-        if (fp32) return len < 24 || (len == 24 && 6 * L.flips >= 7 * L.groups);
-        if (prec == RP_C128) return len < 23 || 3 * L.flips >= 5 * L.groups;
-        return len < 26 || 6 * L.flips >= (len == 26 ? 7 : 10) * L.groups;
+        if (group_acc && rows) return len < 24 && per < 1.5;
+        if (fp32) return len < 24 || (len == 24 && per >= 7. / 6) ||
+                         (len == 25 && !group_acc && per >= 5. / 3);
+        if (prec == RP_C128) return len < 23 || per >= 1.4;
+        return len < 26 || per >= (len == 26 ? 7. / 6 : 1.4);
     }
     return !fp32 || !rows ||
-           (!group_acc && (L.terms >= 6 * L.flips || 2 * L.flips < 3 * L.groups));
+           (!group_acc && (len < 22 || L.terms >= 6 * L.flips || per < 1.5));
 }
 
 // default tiling (RP_TERMS_AUTOTUNE measures the alternatives)
@@ -1568,7 +1576,7 @@ static void choose_tiling(int prec, int len, const ListShape &L, int group_acc, 
     const bool single = 2 * L.terms < 3 * L.flips;
     if (group_acc) {
         if (single && (len >= 28 || (len >= 26 && L.flips > 64))) *tb = 13;
-        if (!single || *tb == 13 || len <= 20) *nt = 1024;
+        if (!single || len >= 26 || len <= 20) *nt = 1024;
     } else if (!single || (len < 28 && long_list(len, L.flips, L.shared))) {
         *nt = 1024;
     }

@@ -115,7 +115,7 @@ FREE, S, M, B = (0, 256), (12, 512), (12, 1024), (13, 1024)
     ("c64", 20, 60, 1, M), ("c64", 22, 60, 1, S), ("c64", 22, 110, 1, M), ("c64", 23, 110, 1, S),
     ("c64", 24, 240, 1, M), ("c64", 27, 240, 1, M), ("c64", 28, 240, 1, S),
     ("group", 20, 60, 1, M), ("group", 21, 60, 1, S), ("group", 25, 60, 1, S),
-    ("group", 26, 60, 1, S), ("group", 26, 70, 1, B), ("group", 28, 60, 1, B),
+    ("group", 26, 60, 1, M), ("group", 26, 70, 1, B), ("group", 28, 60, 1, B),
     ("c128", 20, 60, 1, S), ("native", 26, 60, 1, S),
     # masks that share terms
     ("c64", 26, 60, 3, M), ("c64", 28, 60, 3, M), ("group", 22, 60, 3, M), ("group", 28, 60, 3, M),
