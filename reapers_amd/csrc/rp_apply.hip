@@ -1405,20 +1405,42 @@ struct ListShape {
     uint64_t by_row = 0;              // those with a phase bit among the row bits of
                                       // k_apply_wave
 };
+// ascending order of v by bits [1, bits); long lists by a radix sort (10626
+// terms at 12 sites 0.05 ms, std::sort 0.5)
+static void sort_masks(std::vector<uint64_t> &v, int bits)
+{
+    if (v.size() < 512) {
+        std::sort(v.begin(), v.end());
+        return;
+    }
+    constexpr int kDigit = 11;
+    std::vector<uint64_t> w(v.size());
+    for (int s = 1; s < bits; s += kDigit) {
+        uint64_t at[(1 << kDigit) + 1] = {0};
+        for (uint64_t e : v) at[(e >> s & ((1 << kDigit) - 1)) + 1]++;
+        for (int d = 0; d < 1 << kDigit; d++) at[d + 1] += at[d];
+        for (uint64_t e : v) w[at[e >> s & ((1 << kDigit) - 1)]++] = e;
+        v.swap(w);
+    }
+}
 static ListShape list_shape(const uint64_t *bits, uint64_t n)
 {
-    std::vector<uint64_t> xz(n);
-    for (uint64_t t = 0; t < n; t++)
-        xz[t] = (uint64_t)pext_even(bits[t]) << 32 | pext_odd(bits[t]);
-    std::sort(xz.begin(), xz.end());
+    // flip mask, and whether the phase mask has a row bit (sites 6 and 7)
+    std::vector<uint64_t> v(n);
+    uint64_t any = 0;
+    for (uint64_t t = 0; t < n; t++) {
+        v[t] = (uint64_t)pext_even(bits[t]) << 1 | ((bits[t] >> 13 & 5) != 0);
+        any |= v[t];
+    }
+    sort_masks(v, any ? 64 - __builtin_clzll(any) : 1);
     ListShape L;
     L.terms = n;
     for (uint64_t i = 0, j; i < n; i = j) {
         uint64_t rows = 0;
-        for (j = i; j < n && xz[j] >> 32 == xz[i] >> 32; j++) rows += (xz[j] & (3u << 6)) != 0;
+        for (j = i; j < n && v[j] >> 1 == v[i] >> 1; j++) rows += v[j] & 1;
         L.flips++;
         L.pieces += (j - i + kWavePiece - 1) / kWavePiece;
-        if (!i || xz[i] >> 44 != xz[i - 1] >> 44) L.groups++;
+        if (!i || v[i] >> 13 != v[i - 1] >> 13) L.groups++;
         if (j - i == 1) continue;
         L.shared += j - i;
         L.by_row += rows;
@@ -1736,9 +1758,14 @@ static int upload_wave(rp_terms *h, const std::vector<FlatTerm<A>> &flat, UP &&u
     std::vector<TermW<A>> terms;
     std::vector<uint32_t> flips;
     std::vector<uint64_t> cost(1, 0);
+    terms.reserve(flat.size());
+    // bit l: parity of l & z, the sum of the patterns of z's bits
     auto lanes = [](uint32_t z) {
+        constexpr uint64_t bit[6] = {0xaaaaaaaaaaaaaaaaull, 0xccccccccccccccccull,
+                                     0xf0f0f0f0f0f0f0f0ull, 0xff00ff00ff00ff00ull,
+                                     0xffff0000ffff0000ull, 0xffffffff00000000ull};
         uint64_t m = 0;
-        for (uint32_t l = 0; l < 64; l++) m |= (uint64_t)(__builtin_popcount(l & z) & 1) << l;
+        for (int b = 0; b < 6; b++) m ^= bit[b] & -(uint64_t)(z >> b & 1);
         return m;
     };
     const uint32_t rowbits = 64u * (h->rows - 1);
@@ -1765,17 +1792,25 @@ static int upload_wave(rp_terms *h, const std::vector<FlatTerm<A>> &flat, UP &&u
             }
             work += j - i;
         } else {
-            uint32_t n[4] = {0, 0, 0, 0};
+            // counted, then placed: real parts without and with phase bits
+            // among the row bits, then imaginary ones
+            uint32_t n[4] = {0, 0, 0, 0}, at[4];
+            for (size_t q = i; q < j; q++) {
+                const int byrow = (flat[q].z & rowbits) != 0;
+                n[byrow] += flat[q].cr != 0;
+                n[2 + byrow] += flat[q].ci != 0;
+            }
             S.kind = kWaveMulti;
             S.term = (uint32_t)terms.size();
-            for (int k = 0; k < 4; k++)
-                for (size_t q = i; q < j; q++) {
-                    const A c = k < 2 ? flat[q].cr : flat[q].ci;
-                    const bool byrow = (flat[q].z & rowbits) != 0;
-                    if (c == 0 || byrow != (k & 1)) continue;
-                    terms.push_back({lanes(flat[q].z), c, flat[q].z, 0});
-                    n[k]++;
-                }
+            at[0] = S.term;
+            for (int k = 1; k < 4; k++) at[k] = at[k - 1] + n[k - 1];
+            terms.resize(at[3] + n[3]);
+            for (size_t q = i; q < j; q++) {
+                const int byrow = (flat[q].z & rowbits) != 0;
+                const uint64_t l = lanes(flat[q].z);
+                if (flat[q].cr != 0) terms[at[byrow]++] = {l, flat[q].cr, flat[q].z, 0};
+                if (flat[q].ci != 0) terms[at[2 + byrow]++] = {l, flat[q].ci, flat[q].z, 0};
+            }
             S.z0 = n[0];
             S.z1 = n[1];
             S.l0 = (uint64_t)n[3] << 32 | n[2];
